@@ -118,9 +118,6 @@ struct sc_dd {
   int* gate_list = nullptr;    // one entry per channel tile
   int* gate_count = nullptr;   // {tile count, flagged blocks}
   int* h_gate = nullptr;       // pinned mirror of gate_count
-  int* gather_idx = nullptr;   // 2*capacity ints
-  float* gather_out = nullptr;
-  size_t gather_capacity = 0;
   size_t device_bytes = 0;
 
   // Pinned host mirrors.
@@ -130,6 +127,8 @@ struct sc_dd {
   int* h_top_off = nullptr;
   int4* h_cand = nullptr;
   float* h_stats = nullptr;
+  int4* h_paths = nullptr;  // addIncoherentPower's path queries and results
+  size_t paths_capacity = 0;
 
   // Graph replay of the device-statistics search (keyed by input and
   // parameters), captured on a private stream and launched on the caller's.
@@ -206,8 +205,7 @@ void release(sc_dd* dd) {
   (void)hipFree(dd->gate_list);
   (void)hipFree(dd->gate_count);
   (void)hipHostFree(dd->h_gate);
-  (void)hipFree(dd->gather_idx);
-  (void)hipFree(dd->gather_out);
+  (void)hipHostFree(dd->h_paths);
   (void)hipHostFree(dd->h_colsum);
   (void)hipHostFree(dd->h_top_sum);
   (void)hipHostFree(dd->h_top_blk);
@@ -263,21 +261,26 @@ sc_status ensure_pass_scratch(sc_dd* dd, int nb) {
   return s;
 }
 
-// Path sums of one drift block into a [T_r][N] buffer; returns which buffer.
-sc_status run_tree(sc_dd* dd, const void* data, int dtype, long stride, int drift,
+// Path sums of one drift block into a [T_r][N] buffer: `out` if given, else one
+// of the handle's two (returned in *result). Up to 256 rows take one launch;
+// above, the levels from 512 on alternate between two buffers so that the
+// last one lands in `out`.
+sc_status run_tree(sc_dd* dd, const void* data, int dtype, long stride, int drift, float* out,
                    float** result, hipStream_t stream) {
-  sc_status s = ensure_tree_scratch(dd);
-  if (s != SC_OK) return s;
   const int T = dd->rounded, N = dd->num_channels;
-  SC_HIP(sc::launch_tree_blocks(data, dtype, stride, T, N, drift, dd->tree_a, stream),
-         "tree blocks");
-  float* src = dd->tree_a;
-  float* dst = dd->tree_b;
-  for (int L = 32; L <= T; L *= 2) {
-    SC_HIP(sc::launch_one_step(src, dst, T, N, L, drift, stream), "one step");
-    std::swap(src, dst);
+  if (!out || T > 256) {
+    sc_status s = ensure_tree_scratch(dd);
+    if (s != SC_OK) return s;
   }
-  *result = src;
+  float* dst = out ? out : dd->tree_a;
+  float* src = dd->tree_b;
+  for (int L = 512; L <= T; L *= 2) std::swap(src, dst);
+  SC_HIP(sc::launch_tree_blocks(data, dtype, stride, T, N, drift, dst, stream), "tree blocks");
+  for (int L = 512; L <= T; L *= 2) {
+    std::swap(src, dst);
+    SC_HIP(sc::launch_one_step(src, dst, T, N, L, drift, stream), "one step");
+  }
+  *result = dst;
   return SC_OK;
 }
 
@@ -593,7 +596,7 @@ sc_status enqueue_path_sums(sc_dd* dd, const void* data, int dtype, long row_str
              "column sums");
     for (int b = r.bmin; b <= r.bmax; ++b) {
       float* sums = nullptr;
-      sc_status s = run_tree(dd, data, dtype, row_stride, b, &sums, stream);
+      sc_status s = run_tree(dd, data, dtype, row_stride, b, nullptr, &sums, stream);
       if (s != SC_OK) return s;
       SC_HIP(sc::launch_top_update(sums, T, N, b, r.bmin, dd->top_key, stream), "top update");
     }
@@ -1039,11 +1042,17 @@ sc_status sc_dd_taylor_tree(sc_dd* dd, const void* data, int dtype, int rounded_
   if (!out) return fail(SC_ERR_INVALID_ARGUMENT, "null output");
   hipStream_t stream = (hipStream_t)stream_ptr;
   float* sums = nullptr;
-  s = run_tree(dd, data, dtype, row_stride, drift_block, &sums, stream);
+  // An output that overlaps the input is formed in the handle's buffer first.
+  const size_t count = (size_t)dd->rounded * dd->num_channels;
+  const uintptr_t d0 = (uintptr_t)data, o0 = (uintptr_t)out;
+  const size_t in_bytes =
+      ((size_t)(dd->rounded - 1) * row_stride + dd->num_channels) * (dtype == SC_F32 ? 4 : 2);
+  const bool apart = o0 + sizeof(float) * count <= d0 || d0 + in_bytes <= o0;
+  s = run_tree(dd, data, dtype, row_stride, drift_block, apart ? out : nullptr, &sums, stream);
   if (s != SC_OK) return s;
-  SC_HIP(hipMemcpyAsync(out, sums, sizeof(float) * (size_t)dd->rounded * dd->num_channels,
-                        hipMemcpyDeviceToDevice, stream),
-         "copy tree");
+  if (!apart)
+    SC_HIP(hipMemcpyAsync(out, sums, sizeof(float) * count, hipMemcpyDeviceToDevice, stream),
+           "copy tree");
   SC_HIP(hipStreamSynchronize(stream), "tree");
   return SC_OK;
 }
@@ -1059,48 +1068,34 @@ sc_status sc_dd_add_incoherent_power(sc_dd* dd, const void* data, int dtype,
   std::sort(hits, hits + num_hits, [](const sc_hit& a, const sc_hit& b) {
     return a.drift_steps < b.drift_steps;
   });
-  if (num_hits > dd->gather_capacity) {
-    (void)hipFree(dd->gather_idx);
-    (void)hipFree(dd->gather_out);
-    dd->gather_idx = nullptr;
-    dd->gather_out = nullptr;
-    s = dev_alloc(dd, (void**)&dd->gather_idx, 2 * num_hits * sizeof(int), "gather");
-    if (s == SC_OK) s = dev_alloc(dd, (void**)&dd->gather_out, num_hits * sizeof(float), "gather");
+  if (num_hits > dd->paths_capacity) {
+    (void)hipHostFree(dd->h_paths);
+    dd->h_paths = nullptr;
+    dd->paths_capacity = 0;
+    s = host_alloc((void**)&dd->h_paths, num_hits * sizeof(int4), "path queries");
     if (s != SC_OK) return s;
-    dd->gather_capacity = num_hits;
+    dd->paths_capacity = num_hits;
   }
+  // Every hit's own path is summed in the tree's order, all hits in one launch
+  // (the reference runs the whole tree of each drift block that has a hit and
+  // gathers from it). 300 hits over 118 drift blocks of 16 x 2^19:
+  // 0.12 ms against 5.8 ms for a tree, a gather and two copies per block.
   const int drift_shift = dd->rounded - 1;
-  size_t i = 0;
-  while (i < num_hits) {
+  for (size_t i = 0; i < num_hits; ++i) {
     // dedoppler.cu:156-157: block by float floor division.
-    int block = (int)std::floor((float)hits[i].drift_steps / drift_shift);
-    size_t j = i;
-    std::vector<int> idx;
-    while (j < num_hits &&
-           (int)std::floor((float)hits[j].drift_steps / drift_shift) == block) {
-      int offset = hits[j].drift_steps - block * drift_shift;
-      if (offset < 0 || offset >= drift_shift || hits[j].index < 0 ||
-          hits[j].index >= dd->num_channels)
-        return fail(SC_ERR_INVALID_ARGUMENT, "hit outside the searched range");
-      idx.push_back(offset);
-      ++j;
-    }
-    const int n = (int)(j - i);
-    for (int k = 0; k < n; ++k) idx.push_back(hits[i + k].index);
-    float* sums = nullptr;
-    s = run_tree(dd, data, dtype, row_stride, block, &sums, stream);
-    if (s != SC_OK) return s;
-    SC_HIP(hipMemcpyAsync(dd->gather_idx, idx.data(), 2 * n * sizeof(int),
-                          hipMemcpyHostToDevice, stream), "copy indices");
-    SC_HIP(sc::launch_gather(sums, dd->num_channels, dd->gather_idx, dd->gather_idx + n, n,
-                             dd->gather_out, stream), "gather");
-    std::vector<float> vals(n);
-    SC_HIP(hipMemcpyAsync(vals.data(), dd->gather_out, n * sizeof(float), hipMemcpyDeviceToHost,
-                          stream), "copy values");
-    SC_HIP(hipStreamSynchronize(stream), "incoherent power");
-    for (int k = 0; k < n; ++k) hits[i + k].incoherent_power = vals[k];
-    i = j;
+    const int block = (int)std::floor((float)hits[i].drift_steps / drift_shift);
+    const int offset = hits[i].drift_steps - block * drift_shift;
+    if (offset < 0 || offset >= drift_shift || hits[i].index < 0 ||
+        hits[i].index >= dd->num_channels)
+      return fail(SC_ERR_INVALID_ARGUMENT, "hit outside the searched range");
+    dd->h_paths[i] = make_int4(hits[i].index, block, offset, 0);
   }
+  SC_HIP(sc::launch_path_sums(data, dtype, row_stride, dd->rounded, dd->num_channels, dd->h_paths,
+                              (int)num_hits, stream),
+         "path sums");
+  SC_HIP(hipStreamSynchronize(stream), "incoherent power");
+  for (size_t i = 0; i < num_hits; ++i)
+    std::memcpy(&hits[i].incoherent_power, &dd->h_paths[i].w, sizeof(float));
   return SC_OK;
 }
 

@@ -147,8 +147,8 @@ hipError_t launch_two_pass(const void* x, int dtype, long stride, int T, int N, 
                            int b_first, int nb, int G, float* scratch, long row_pitch,
                            top_key_t* top_key, hipStream_t stream);
 
-// Level-min(T,16) sums for every time block of one drift block:
-// out[(tb*Tb + p)*N + c], Tb = min(T, 16), tb < T/Tb.
+// Level-min(T,256) sums for every time block of one drift block:
+// out[(tb*Tb + p)*N + c], Tb = min(T, 256), tb < T/Tb.
 hipError_t launch_tree_blocks(const void* x, int dtype, long stride, int T, int N,
                               int drift, float* out, hipStream_t stream);
 
@@ -197,9 +197,11 @@ hipError_t launch_window_merge(const top_key_t* key, int N, int T, int bmin, int
 hipError_t launch_candidate_offsets(const void* x, int dtype, long stride, int T, int N,
                                     int nwin, int4* cand, int* top_off, hipStream_t stream);
 
-// Gathers path sums for (offset, channel) pairs from a [T][N] buffer.
-hipError_t launch_gather(const float* sums, int N, const int* offsets, const int* chans,
-                         int n, float* out, hipStream_t stream);
+// queries[i] = {channel, drift block, path offset, -}: the path sum's float bits
+// into .w (host-visible memory; T up to 4096 rows, samples outside the coarse
+// channel count as 0).
+hipError_t launch_path_sums(const void* x, int dtype, long stride, int T, int N, int4* queries,
+                            int n, hipStream_t stream);
 
 // ---- normalisation and synthetic data -------------------------------------
 hipError_t launch_normalize(const float* x, int T, int N, long stride, int out_dtype,

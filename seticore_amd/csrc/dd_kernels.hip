@@ -153,10 +153,22 @@ __global__ void __launch_bounds__(kWave) candidate_offsets_set_kernel(TailSet ts
   candidate_offsets_body<T, In>((const In*)ts.x[c], stride, N, nwin, ts.cand[c], ts.top_off[c]);
 }
 
-// Tree of one drift block for each T-row time block (T <= 16), written out in
-// the reference's [time_block][offset][chan] layout. The shear is relative to
-// each time block's first row, as in the reference's tiled kernel
-// (taylor.cu:225-231).
+// Four consecutive channels of one output row (one 16-byte store at any 4-byte
+// alignment), cut at the last channel.
+__device__ __forceinline__ void store_row4(float* __restrict__ row, int c, int N,
+                                           const float (&v)[4]) {
+  typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+  if (c + 4 <= N) {
+    *(f4u*)(row + c) = f4u{v[0], v[1], v[2], v[3]};
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (c + j < N) row[c + j] = v[j];
+  }
+}
+
+// Tree of one drift block (T <= 16), written out as [offset][chan]. Bound by
+// the memory it reads and writes once.
 template <int T, int C, typename In>
 __global__ void __launch_bounds__(kWave)
     tree_blocks_kernel(const In* __restrict__ x, long stride, int N, int drift,
@@ -166,8 +178,7 @@ __global__ void __launch_bounds__(kWave)
   __shared__ float win_storage[Wn::kFloats];
   lds_float* win = (lds_float*)win_storage;
   const int c_w = blockIdx.x * Sh::kOut;
-  const int tb = blockIdx.y;
-  load_window<T, C, C, In>(win, x, stride, N, c_w, drift, tb * T);
+  load_window<T, C, C, In>(win, x, stride, N, c_w, drift, 0);
   __syncthreads();
   lds_float* rp[T];
   row_bases<T, C, C>(win, rp);
@@ -177,12 +188,7 @@ __global__ void __launch_bounds__(kWave)
   const int lane = threadIdx.x;
   if (lane < Sh::kValidLanes) {
 #pragma unroll
-    for (int p = 0; p < T; ++p)
-#pragma unroll
-      for (int j = 0; j < C; ++j) {
-        const int c = c_w + lane * C + j;
-        if (c < N) out[(long)(tb * T + p) * N + c] = v[p][j];
-      }
+    for (int p = 0; p < T; ++p) store_row4(out + (long)p * N, c_w + lane * C, N, v[p]);
   }
 }
 
@@ -901,6 +907,104 @@ __global__ void __launch_bounds__(kWave * Staged<M>::kWaves, Staged<M>::kMinWave
   }
 }
 
+// One offset group of one drift block with its path sums written out: phase 1
+// as above, then each wave's offsets as rows q*M .. q*M + M-1 of out.
+template <int M, int G_IDX, typename In>
+__device__ __forceinline__ void staged_write_group(int grp, const In* __restrict__ x, long stride,
+                                                   int N, int b, int c_w, lds_float* R,
+                                                   float* __restrict__ out) {
+  using St = Staged<M>;
+  constexpr int C = St::C;
+  if constexpr (G_IDX + 1 < St::kGroups) {
+    if (grp != G_IDX) {
+      staged_write_group<M, G_IDX + 1, In>(grp, x, stride, N, b, c_w, R, out);
+      return;
+    }
+  }
+  constexpr int Q0 = G_IDX * St::QG;
+  const int wave = threadIdx.x / kWave;
+  const int lane = threadIdx.x % kWave;
+  for (int k = wave; k < M; k += St::kWaves) {
+    float v[16][C];
+    staged_load<M, In>(x, stride, N, k, b, (long)c_w + (long)k * (16 * b + Q0), v);
+    staged_phase1<M, G_IDX>(v, k, R);
+  }
+  __syncthreads();
+  for (int qq = wave; qq < St::QG; qq += St::kWaves) {
+    float v[M][C];
+    const lds_float* src = R + qq * M * St::kRow + lane;
+#pragma unroll
+    for (int k = 0; k < M; ++k)
+#pragma unroll
+      for (int j = 0; j < C; ++j) v[k][j] = src[k * St::kRow + j * St::kSub];
+    tree_regs<M, C>(v);
+    if (lane * C < St::kOut) {
+#pragma unroll
+      for (int r = 0; r < M; ++r)
+        store_row4(out + (long)((Q0 + qq) * M + r) * N, c_w + lane * C, N, v[r]);
+    }
+  }
+}
+
+// The whole tree of one drift block for each T-row time block (T = 16*M =
+// 32..256), written out in the reference's [time_block][offset][chan] layout;
+// the shear is relative to each time block's first row, as in the reference's
+// tiled kernel (taylor.cu:225-231). One pass over the input and one over the
+// output, with the level-16 sums staged in LDS as in staged_tree_kernel,
+// instead of one pass over memory per level above 16: bound by the output's
+// writes. grid.x = (tile, offset group) dealt over the XCDs so that a tile's
+// groups, which read the same rows, share an L2; grid.y = time block.
+// Measured at 256 x 2^20: 0.76 ms (2.8 TB/s of input and output) against
+// 2.99 ms for level-16 trees, four one-level passes and a copy.
+template <int M, typename In>
+__global__ void __launch_bounds__(kWave * Staged<M>::kWaves, Staged<M>::kMinWaves)
+    staged_write_kernel(const In* __restrict__ x, long stride, int N, int drift, int total_items,
+                        float* __restrict__ out) {
+  using St = Staged<M>;
+  __shared__ __attribute__((aligned(16))) float r_storage[St::kFloats];
+  const int per_xcd = gridDim.x / 8;
+  const int item = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (item >= total_items) return;
+  const long tb = blockIdx.y;
+  staged_write_group<M, 0, In>(item % St::kGroups, x + tb * St::T * stride, stride, N, drift,
+                               item / St::kGroups * St::kOut, (lds_float*)r_storage,
+                               out + tb * St::T * N);
+}
+
+// One path sum per wave, in the tree's order: the pairwise recursion over the
+// rows of path (block, offset) from channel index, i.e. neighbouring rows
+// first (taylor.h:53-54). Row t of the path lies t*block plus, for every level
+// L whose upper half holds t, (offset of that level + 1)/2 channels on. T up
+// to 4096 rows: lane i owns rows i*T/64 .. of a shared array, then the lanes
+// combine by butterflies (float addition commutes, so both sides hold the
+// same sum). q[i] = {index, block, offset, result}; the array is in host
+// memory. Latency bound: T loads per hit in flight at once.
+constexpr int kMaxPathRows = 4096;
+template <typename In>
+__global__ void __launch_bounds__(kWave)
+    path_sums_kernel(const In* __restrict__ x, long stride, int T, int N, int4* __restrict__ q) {
+  __shared__ float leaf[kMaxPathRows];
+  const int lane = threadIdx.x;
+  const int4 h = q[blockIdx.x];
+  for (int t = lane; t < T; t += kWave) {
+    long c = (long)h.x + (long)t * h.y;
+    int p = h.z;
+    for (int half = T / 2; half > 0; half /= 2) {
+      if (t & half) c += (p + 1) >> 1;
+      p >>= 1;
+    }
+    leaf[t] = (c >= 0 && c < N) ? to_f32<In>(x[(long)t * stride + c]) : 0.0f;
+  }
+  __syncthreads();
+  const int per = T > kWave ? T / kWave : 1;
+  float* own = leaf + lane * per;
+  for (int w = 1; w < per; w *= 2)
+    for (int i = 0; i < per; i += 2 * w) own[i] += own[i + w];
+  float s = lane < T ? own[0] : 0.0f;
+  for (int o = 1; o < min(T, kWave); o *= 2) s += __shfl_xor(s, o);
+  if (lane == 0) q[blockIdx.x].w = __float_as_int(s);
+}
+
 // taylor.cu:97-109 + taylor.h:30-86: one stage in global memory.
 __global__ void one_step_kernel(const float* __restrict__ src, float* __restrict__ dst, int T,
                                 int N, int L, int drift) {
@@ -1510,12 +1614,6 @@ __global__ void __launch_bounds__(256)
                     ts.top_blk[c], ts.top_off[c], ts.cand[c], flags);
 }
 
-__global__ void gather_kernel(const float* __restrict__ sums, int N, const int* __restrict__ offs,
-                              const int* __restrict__ chans, int n, float* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = sums[(long)offs[i] * N + chans[i]];
-}
-
 // ---------------------------------------------------------------------------
 // Normalisation for half-width storage: FP64 mean and deviation over the
 // T*N samples, two passes with fixed-order partial reduction.
@@ -1796,13 +1894,23 @@ hipError_t staged_dispatch(const In* x, long stride, int T, int N, int bmin, int
 }
 
 template <int T, typename In>
-hipError_t tree_blocks_typed(const In* x, long stride, int Tall, int N, int drift, float* out,
+hipError_t tree_blocks_typed(const In* x, long stride, int N, int drift, float* out,
                              hipStream_t stream) {
   constexpr int C = 4;
   using Sh = TileShape<T, C>;
   const int ntiles = (N + Sh::kOut - 1) / Sh::kOut;
-  hipLaunchKernelGGL((tree_blocks_kernel<T, C, In>), dim3(ntiles, Tall / T), dim3(kWave), 0,
-                     stream, x, stride, N, drift, out);
+  hipLaunchKernelGGL((tree_blocks_kernel<T, C, In>), dim3(ntiles), dim3(kWave), 0, stream, x,
+                     stride, N, drift, out);
+  return hipGetLastError();
+}
+
+template <int M, typename In>
+hipError_t staged_write_typed(const In* x, long stride, int T, int N, int drift, float* out,
+                              hipStream_t stream) {
+  using St = Staged<M>;
+  const int items = (N + St::kOut - 1) / St::kOut * St::kGroups;
+  hipLaunchKernelGGL((staged_write_kernel<M, In>), dim3((items + 7) / 8 * 8, T / St::T),
+                     dim3(kWave * St::kWaves), 0, stream, x, stride, N, drift, items, out);
   return hipGetLastError();
 }
 
@@ -1810,12 +1918,16 @@ template <typename In>
 hipError_t tree_blocks_dispatch(const In* x, long stride, int T, int N, int drift, float* out,
                                 hipStream_t stream) {
   switch (T) {
-    case 2: return tree_blocks_typed<2, In>(x, stride, T, N, drift, out, stream);
-    case 4: return tree_blocks_typed<4, In>(x, stride, T, N, drift, out, stream);
-    case 8: return tree_blocks_typed<8, In>(x, stride, T, N, drift, out, stream);
+    case 2: return tree_blocks_typed<2, In>(x, stride, N, drift, out, stream);
+    case 4: return tree_blocks_typed<4, In>(x, stride, N, drift, out, stream);
+    case 8: return tree_blocks_typed<8, In>(x, stride, N, drift, out, stream);
+    case 16: return tree_blocks_typed<16, In>(x, stride, N, drift, out, stream);
+    case 32: return staged_write_typed<2, In>(x, stride, T, N, drift, out, stream);
+    case 64: return staged_write_typed<4, In>(x, stride, T, N, drift, out, stream);
+    case 128: return staged_write_typed<8, In>(x, stride, T, N, drift, out, stream);
     default:
-      if (T >= 16 && (T % 16) == 0)
-        return tree_blocks_typed<16, In>(x, stride, T, N, drift, out, stream);
+      if (T >= 256 && (T % 256) == 0)
+        return staged_write_typed<16, In>(x, stride, T, N, drift, out, stream);
       return hipErrorInvalidValue;
   }
 }
@@ -2131,11 +2243,25 @@ hipError_t launch_window_merge(const top_key_t* key, int N, int T, int bmin, int
   return hipGetLastError();
 }
 
-hipError_t launch_gather(const float* sums, int N, const int* offsets, const int* chans, int n,
-                         float* out, hipStream_t stream) {
+hipError_t launch_path_sums(const void* x, int dtype, long stride, int T, int N, int4* queries,
+                            int n, hipStream_t stream) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(gather_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, sums, N, offsets,
-                     chans, n, out);
+  if (T > kMaxPathRows) return hipErrorInvalidValue;
+  switch (dtype) {
+    case 0:
+      hipLaunchKernelGGL(path_sums_kernel<float>, dim3(n), dim3(kWave), 0, stream,
+                         (const float*)x, stride, T, N, queries);
+      break;
+    case 1:
+      hipLaunchKernelGGL(path_sums_kernel<__half>, dim3(n), dim3(kWave), 0, stream,
+                         (const __half*)x, stride, T, N, queries);
+      break;
+    case 2:
+      hipLaunchKernelGGL(path_sums_kernel<__hip_bfloat16>, dim3(n), dim3(kWave), 0, stream,
+                         (const __hip_bfloat16*)x, stride, T, N, queries);
+      break;
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 

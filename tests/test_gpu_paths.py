@@ -1,0 +1,74 @@
+"""Path sums written out (taylor_tree) and looked up (addIncoherentPower) at the shapes where their
+kernels change: tile edges, odd widths, one or several 256-row time blocks, each sample type. Float
+additions are in the reference's order, so the bar is equality with the oracle."""
+
+import numpy as np
+import pytest
+
+import seticore_amd as sc
+
+pytestmark = pytest.mark.gpu
+
+
+def _data(T, N, dtype, seed):
+    import torch
+    x = torch.from_numpy(np.random.default_rng(seed).exponential(size=(T, N)).astype(np.float32))
+    code, kind = {"f32": (sc.SC_F32, torch.float32), "f16": (sc.SC_F16, torch.float16),
+                  "bf16": (sc.SC_BF16, torch.bfloat16)}[dtype]
+    x = x.to(kind)
+    return x.float().numpy(), x.cuda(), code
+
+
+def _valid(T, N, b):
+    last = np.arange(N)[None, :] + (T - 1) * b + np.arange(T)[:, None]
+    return (last >= 0) & (last < N)
+
+
+# Tile widths: 240 channels at 16 rows, 224 / 192 / 184 / 180 at 32 / 64 / 128 / 256.
+@pytest.mark.parametrize("T,N,dtype", [
+    (2, 4097, "f32"), (16, 239, "f16"), (16, 1201, "bf16"), (32, 225, "f32"), (64, 192, "bf16"),
+    (64, 1155, "f32"), (128, 183, "f32"), (128, 1471, "f16"), (256, 181, "f32"),
+    (256, 1441, "bf16"), (512, 2003, "f32"), (1024, 4001, "f16")])
+def test_tree_at_tile_edges(gpu, oracle, T, N, dtype):
+    host, x, code = _data(T, N, dtype, T + N)
+    dd = sc.Dedopplerer(T, N, 1.0, 1.0)
+    for b in (-1, 0, 1):
+        print("tree", T, N, dtype, b, flush=True)
+        got = dd.taylor_tree(sc.FilterbankBuffer(T, N, data=x, dtype=code), b).cpu().numpy()
+        ok = _valid(T, N, b)
+        np.testing.assert_array_equal(got[ok], oracle.basic_taylor_tree(host, b)[ok])
+
+
+def test_tree_output_may_be_the_input(gpu, oracle):
+    import ctypes
+    T, N = 64, 777
+    host, x, code = _data(T, N, "f32", 3)
+    dd = sc.Dedopplerer(T, N, 1.0, 1.0)
+    sc.check(sc.lib().sc_dd_taylor_tree(dd._h, ctypes.c_void_p(x.data_ptr()), code, T, N, N, 1,
+                                        ctypes.c_void_p(x.data_ptr()), None))
+    ok = _valid(T, N, 1)
+    np.testing.assert_array_equal(x.cpu().numpy()[ok], oracle.basic_taylor_tree(host, 1)[ok])
+
+
+@pytest.mark.parametrize("T,N,dtype,n", [(2, 500, "f32", 1), (16, 9001, "bf16", 257),
+                                         (50, 3000, "f16", 40), (64, 3000, "f32", 33),
+                                         (128, 4000, "f32", 20), (512, 6000, "f32", 12)])
+def test_incoherent_power_of_any_path(gpu, oracle, T, N, dtype, n):
+    T_r = sc.round_up_to_power_of_two(T)
+    host, x, code = _data(T_r, N, dtype, T)
+    dd = sc.Dedopplerer(T, N, 1.0, 1.0)
+    rng = np.random.default_rng(n)
+    span = T_r - 1
+    hits = []
+    for d in rng.choice(np.arange(-3 * span, 3 * span + 1), size=min(n, 6 * span + 1), replace=False):
+        c = int(rng.integers(max(0, -d), N - max(0, d)))
+        hits.append(sc.DedopplerHit(index=c, drift_steps=int(d)))
+    print("incoherent", T, N, dtype, len(hits), flush=True)
+    dd.addIncoherentPower(sc.FilterbankBuffer(T_r, N, data=x, dtype=code), hits)
+    trees = {}
+    for h in hits:
+        b, p = divmod(h.drift_steps, span)
+        if b not in trees:
+            trees[b] = oracle.basic_taylor_tree(host, b)
+        assert h.incoherent_power == trees[b][p, h.index]
+    assert [h.drift_steps for h in hits] == sorted(h.drift_steps for h in hits)
