@@ -1110,11 +1110,11 @@ __global__ void unpack_top_kernel(const top_key_t* __restrict__ key, int N, int 
 // the exact order statistics at ranks mid = N/2, first = ceil(.05N) and
 // last = floor(.95N), and the trimmed mean/deviation over the sorted ranks
 // [first, last] in FP64, by a three-level radix select over the column sums'
-// order keys (11 + 11 + 10 bits):
-//   pass 1: histogram of the top 11 bits;
+// order keys (13 + 10 + 9 bits):
+//   pass 1: histogram of the top 13 bits;
 //   pass 2: every workgroup finds the level-1 bin of each rank from that
-//           histogram, then histograms the next 11 bits inside those bins;
-//   pass 3: likewise for the last 10 bits;
+//           histogram, then histograms the next 10 bits inside those bins;
+//   pass 3: likewise for the last 9 bits;
 //   pass 4: every workgroup resolves the three exact values, then sums
 //           (x - K) and (x - K)^2 in FP64 over the values strictly between
 //           the first and last ranks' values (K = the median);
@@ -1123,16 +1123,25 @@ __global__ void unpack_top_kernel(const top_key_t* __restrict__ key, int N, int 
 //           forms its mean, and std = sqrt(sum (x - m)^2 / count) in FP64.
 // Histograms are counted in LDS and flushed with one atomic per non-zero bin;
 // partial sums are reduced in a fixed order, so results are deterministic.
+// What passes 2 and 3 cost is the flush, so the first level is the widest:
+// column sums fill few of its bins, and the second level then counts a quarter
+// of the values it would after 11 bits. The first workgroup of a pass leaves
+// the selection it made to the next pass. Passes 1-4 and final at 2^20, alone:
+// 72 us with 11 + 11 + 10 bits, one value per load and scans through shared
+// memory in every pass; 44 us now (12 + 18 + 5 + 6 + 4).
 
 constexpr int kStatsBlocks = 256;
 constexpr int kStatsThreads = 256;
-constexpr int kL1Bits = 11, kL2Bits = 11, kL3Bits = 10;
+constexpr int kL1Bits = 13, kL2Bits = 10, kL3Bits = 9;
 constexpr int kL1 = 1 << kL1Bits, kL2 = 1 << kL2Bits, kL3 = 1 << kL3Bits;
 // Histogram words: level 1, then level 2 and level 3 for each of the 3 ranks,
 // then one word counting column sums that are not finite (NaN or infinite
 // samples; the search rejects such input).
 constexpr int kHistWords = kL1 + 3 * kL2 + 3 * kL3;
 constexpr int kNonFiniteWord = kHistWords;
+// Then the selections after levels 1 and 2 (prefix, rank inside it, values
+// below it, for each rank), written by passes 2 and 3.
+constexpr int kSelection1 = kHistWords + 1, kSelection2 = kSelection1 + 9;
 
 struct StatsState {
   unsigned key[3];    // exact order keys of ranks mid, first, last
@@ -1142,61 +1151,67 @@ struct StatsState {
   unsigned part_n[kStatsBlocks];
 };
 
-size_t stats_hist_words() { return (size_t)kHistWords + 1; }
+size_t stats_hist_words() { return (size_t)kSelection2 + 9; }
 
 __device__ __forceinline__ int rank_first(int N) { return (int)ceil(0.05 * N); }
 __device__ __forceinline__ int rank_last(int N) { return (int)floor(0.95 * N); }
 
 // For each rank r (want[r] counted among the values matching the previous
 // levels), finds the bin of `hist[r]` holding it: bin[r], the number of values
-// in lower bins (added to below[r]) and the bin count. 256 threads; nbins a
-// multiple of 256.
+// in lower bins (added to below[r]) and the bin count. 256 threads, one wave
+// per rank: each lane sums NBINS/64 consecutive bins, a wave scan places the
+// lanes, and the lane whose range holds the rank walks its bins. (A scan over
+// the whole workgroup's shared memory, rank after rank, took 48 barriers per
+// level and was most of passes 2-4.) N and the histogram agree, so exactly one
+// lane finds a rank below the count; a rank at or above it reads bin 0.
 template <int NBINS>
 __device__ void select_level(const unsigned* __restrict__ hist, int hist_stride,
                              const unsigned (&want)[3], unsigned (&bin)[3],
                              unsigned (&below)[3], unsigned (&count)[3]) {
-  constexpr int kPer = NBINS / kStatsThreads;
-  __shared__ unsigned scan[kStatsThreads];
+  constexpr int kPer = NBINS / kWave;
+  static_assert(kPer % 4 == 0, "lanes read their bins four at a time");
   __shared__ unsigned found[3][3];
-  const int tid = threadIdx.x;
-  if (tid < 9) found[tid / 3][tid % 3] = 0;
-  for (int r = 0; r < 3; ++r) {
-    const unsigned* h = hist + r * hist_stride;
+  const int lane = threadIdx.x % kWave, r = threadIdx.x / kWave;
+  if (r < 3) {
+    const uint4* h = (const uint4*)(hist + r * hist_stride) + lane * (kPer / 4);
     unsigned v[kPer];
     unsigned local = 0;
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      v[i] = h[tid * kPer + i];
-      local += v[i];
+    for (int i = 0; i < kPer / 4; ++i) {
+      const uint4 q = h[i];
+      v[4 * i] = q.x;
+      v[4 * i + 1] = q.y;
+      v[4 * i + 2] = q.z;
+      v[4 * i + 3] = q.w;
+      local += (q.x + q.y) + (q.z + q.w);
     }
-    scan[tid] = local;
-    __syncthreads();
-    for (int off = 1; off < kStatsThreads; off <<= 1) {
-      const unsigned x = tid >= off ? scan[tid - off] : 0u;
-      __syncthreads();
-      scan[tid] += x;
-      __syncthreads();
+    unsigned upto = local;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const unsigned o = __shfl_up(upto, off);
+      if (lane >= off) upto += o;
     }
-    const unsigned before = tid ? scan[tid - 1] : 0u;
-    const unsigned w = want[r];
-    if (w >= before && w < scan[tid]) {
-      unsigned cum = before;
+    unsigned cum = upto - local;
+    const unsigned w = r == 0 ? want[0] : r == 1 ? want[1] : want[2];
+    const bool mine = w >= cum && w < upto;
+    if (mine) {
 #pragma unroll
       for (int i = 0; i < kPer; ++i) {
         if (w >= cum && w < cum + v[i]) {
-          found[r][0] = (unsigned)(tid * kPer + i);
+          found[r][0] = (unsigned)(lane * kPer + i);
           found[r][1] = cum;
           found[r][2] = v[i];
         }
         cum += v[i];
       }
     }
-    __syncthreads();
+    if (__ballot(mine) == 0 && lane < 3) found[r][lane] = 0;
   }
-  for (int r = 0; r < 3; ++r) {
-    bin[r] = found[r][0];
-    below[r] = found[r][1];
-    count[r] = found[r][2];
+  __syncthreads();
+  for (int i = 0; i < 3; ++i) {
+    bin[i] = found[i][0];
+    below[i] = found[i][1];
+    count[i] = found[i][2];
   }
   __syncthreads();
 }
@@ -1207,49 +1222,81 @@ __device__ __forceinline__ void stats_ranks(int N, unsigned (&want)[3]) {
   want[2] = (unsigned)rank_last(N);
 }
 
+// Calls f(value) for every value, four consecutive values per load (v is
+// 16-byte aligned) and kStatsLoads loads in flight per thread, so that a pass
+// over a coarse channel's column sums costs about one memory latency: with one
+// value per load in flight, a thread's 16 values at 2^20 were 16 latencies.
+// Every thread of the workgroup runs the same number of rounds and calls
+// `round()` after each.
+constexpr int kStatsLoads = 4;
+template <typename F, typename R>
+__device__ __forceinline__ void for_each_value(const float* __restrict__ v, int N, F f, R round) {
+  const long quads = N / 4;
+  const long step = (long)gridDim.x * blockDim.x;
+  for (long base = (long)blockIdx.x * blockDim.x; base < quads; base += kStatsLoads * step) {
+    float4 q[kStatsLoads];
+#pragma unroll
+    for (int l = 0; l < kStatsLoads; ++l) {
+      const long i = base + l * step + threadIdx.x;
+      if (i < quads) q[l] = ((const float4*)v)[i];
+    }
+#pragma unroll
+    for (int l = 0; l < kStatsLoads; ++l) {
+      if (base + l * step + threadIdx.x < quads) {
+        f(q[l].x);
+        f(q[l].y);
+        f(q[l].z);
+        f(q[l].w);
+      }
+    }
+    round();
+  }
+  if (blockIdx.x == 0 && (int)threadIdx.x < N % 4) f(v[4 * quads + threadIdx.x]);
+}
+
 // Counts `digit(key)` into an LDS histogram for every value passing `match`,
 // then flushes the non-zero bins into global memory. Two 16-bit counters per
-// LDS word (3 * NBINS / 2 words: 12 KB at 2048 bins), so the workgroup fits
-// beside the tree kernels' 20 KB windows when one of them retires; the counts
-// are flushed every 255 strides (at most 256 * 255 increments of one counter
-// in between), which only happens above 16.7 M values.
-template <int NBINS, typename Match, typename Digit>
+// LDS word (16 KB at level 1, 6 KB at level 2), so the workgroup fits
+// beside the tree kernels' 20 KB windows when one of them retires; a round
+// adds at most 256 * 16 to a counter, so the counts are flushed every 15
+// rounds, which only happens above 15.7 M values.
+template <int NBINS, int RANKS, typename Match, typename Digit>
 __device__ void block_histogram(const float* __restrict__ v, int N, unsigned* lds,
                                 unsigned* __restrict__ out, Match match, Digit digit) {
-  constexpr int kWords = 3 * NBINS / 2;
+  constexpr int kWords = RANKS * NBINS / 2;
+  static_assert(15 * 4 * kStatsLoads * kStatsThreads + 3 < 65536, "16-bit counters");
   for (int i = threadIdx.x; i < kWords; i += blockDim.x) lds[i] = 0;
   __syncthreads();
-  const long stride = (long)gridDim.x * blockDim.x;
-  int strides = 0;
-  for (long base = (long)blockIdx.x * blockDim.x; base < N; base += stride) {
-    const long i = base + threadIdx.x;
-    if (i < N) {
-      const unsigned k = ord_key(v[i]);
+  int rounds = 0;
+  auto flush = [&](bool clear) {
+    for (int w = threadIdx.x; w < kWords; w += blockDim.x) {
+      const unsigned x = lds[w];
+      if (x & 0xFFFFu) atomicAdd(&out[2 * w], x & 0xFFFFu);
+      if (x >> 16) atomicAdd(&out[2 * w + 1], x >> 16);
+      if (clear) lds[w] = 0;
+    }
+  };
+  for_each_value(
+      v, N,
+      [&](float x) {
+        const unsigned k = ord_key(x);
 #pragma unroll
-      for (int r = 0; r < 3; ++r)
-        if (match(r, k)) {
-          const unsigned b = (unsigned)(r * NBINS) + digit(k);
-          atomicAdd(&lds[b >> 1], 1u << (16 * (b & 1)));
+        for (int r = 0; r < RANKS; ++r)
+          if (match(r, k)) {
+            const unsigned b = (unsigned)(r * NBINS) + digit(k);
+            atomicAdd(&lds[b >> 1], 1u << (16 * (b & 1)));
+          }
+      },
+      [&]() {
+        if (++rounds == 15) {  // uniform over the workgroup
+          __syncthreads();
+          flush(true);
+          __syncthreads();
+          rounds = 0;
         }
-    }
-    if (++strides == 255 && base + stride < N) {  // uniform over the workgroup
-      __syncthreads();
-      for (int w = threadIdx.x; w < kWords; w += blockDim.x) {
-        const unsigned x = lds[w];
-        if (x & 0xFFFFu) atomicAdd(&out[2 * w], x & 0xFFFFu);
-        if (x >> 16) atomicAdd(&out[2 * w + 1], x >> 16);
-        lds[w] = 0;
-      }
-      __syncthreads();
-      strides = 0;
-    }
-  }
+      });
   __syncthreads();
-  for (int w = threadIdx.x; w < kWords; w += blockDim.x) {
-    const unsigned x = lds[w];
-    if (x & 0xFFFFu) atomicAdd(&out[2 * w], x & 0xFFFFu);
-    if (x >> 16) atomicAdd(&out[2 * w + 1], x >> 16);
-  }
+  flush(false);
 }
 
 // The statistics passes below are written as device functions (LDS passed
@@ -1257,49 +1304,110 @@ __device__ void block_histogram(const float* __restrict__ v, int N, unsigned* ld
 // (grid.y = channel, a gated batch run's front) share them.
 __device__ __forceinline__ void stats_pass1_body(const float* __restrict__ v, int N,
                                                  unsigned* __restrict__ hist, unsigned* h) {
-  for (int i = threadIdx.x; i < kL1; i += blockDim.x) h[i] = 0;
-  __syncthreads();
   unsigned bad = 0;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
-    const float x = v[i];
-    // Exponent bits all ones: NaN or infinity (an integer test, which the
-    // no-NaN compile mode cannot fold away).
-    bad += (__float_as_uint(x) & 0x7F800000u) == 0x7F800000u;
-    atomicAdd(&h[ord_key(x) >> (32 - kL1Bits)], 1u);
-  }
+  block_histogram<kL1, 1>(
+      v, N, h, hist,
+      [&](int, unsigned k) {
+        // Exponent bits all ones: NaN or infinity (an integer test, which the
+        // no-NaN compile mode cannot fold away). The order key flips the sign
+        // of positive values and every bit of negative ones.
+        const unsigned e = (k & 0x80000000u) ? k : ~k;
+        bad += (e & 0x7F800000u) == 0x7F800000u;
+        return true;
+      },
+      [](unsigned k) { return k >> (32 - kL1Bits); });
   if (bad) atomicAdd(&hist[kNonFiniteWord], bad);
-  __syncthreads();
-  for (int i = threadIdx.x; i < kL1; i += blockDim.x)
-    if (h[i]) atomicAdd(&hist[i], h[i]);
 }
 
 __global__ void __launch_bounds__(kStatsThreads)
     stats_pass1_kernel(const float* __restrict__ v, int N, unsigned* __restrict__ hist) {
-  __shared__ unsigned h[kL1];
+  __shared__ unsigned h[kL1 / 2];
   stats_pass1_body(v, N, hist, h);
 }
 
 __global__ void __launch_bounds__(kStatsThreads) stats_pass1_set_kernel(FrontSet fs, int N) {
-  __shared__ unsigned h[kL1];
+  __shared__ unsigned h[kL1 / 2];
   stats_pass1_body(fs.colsum[blockIdx.y], N, fs.hist[blockIdx.y], h);
 }
 
-// Level-1 selection (replicated in every workgroup).
+// Level-1 selection (replicated in every workgroup): one scan of the histogram
+// places all three ranks.
 __device__ void select_l1(const unsigned* __restrict__ hist, int N, unsigned (&pre)[3],
                           unsigned (&want)[3], unsigned (&below)[3]) {
-  unsigned w0[3], bin[3], bl[3], cnt[3];
+  constexpr int kPer = kL1 / kStatsThreads;
+  __shared__ unsigned waves[kStatsThreads / kWave];
+  __shared__ unsigned found[3][2];
+  const int tid = threadIdx.x, lane = tid % kWave;
+  if (tid < 6) found[tid / 2][tid % 2] = 0;
+  unsigned v[kPer];
+  unsigned local = 0;
+#pragma unroll
+  for (int i = 0; i < kPer / 4; ++i) {
+    const uint4 q = ((const uint4*)hist)[tid * (kPer / 4) + i];
+    v[4 * i] = q.x;
+    v[4 * i + 1] = q.y;
+    v[4 * i + 2] = q.z;
+    v[4 * i + 3] = q.w;
+    local += (q.x + q.y) + (q.z + q.w);
+  }
+  unsigned upto = local;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const unsigned o = __shfl_up(upto, off);
+    if (lane >= off) upto += o;
+  }
+  if (lane == kWave - 1) waves[tid / kWave] = upto;
+  __syncthreads();
+  for (int w = 0; w < tid / kWave; ++w) upto += waves[w];
+  unsigned w0[3];
   stats_ranks(N, w0);
-  select_level<kL1>(hist, 0, w0, bin, bl, cnt);
   for (int r = 0; r < 3; ++r) {
-    pre[r] = bin[r];
-    want[r] = w0[r] - bl[r];
-    below[r] = bl[r];
+    unsigned cum = upto - local;
+    if (w0[r] >= cum && w0[r] < upto) {
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        if (w0[r] >= cum && w0[r] < cum + v[i]) {
+          found[r][0] = (unsigned)(tid * kPer + i);
+          found[r][1] = cum;
+        }
+        cum += v[i];
+      }
+    }
+  }
+  __syncthreads();
+  for (int r = 0; r < 3; ++r) {
+    pre[r] = found[r][0];
+    below[r] = found[r][1];
+    want[r] = w0[r] - below[r];
+  }
+  __syncthreads();
+}
+
+// A level's selection, left by the first workgroup of a pass for the next one.
+__device__ __forceinline__ void save_selection(unsigned* sel, const unsigned (&pre)[3],
+                                               const unsigned (&want)[3],
+                                               const unsigned (&below)[3]) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    for (int r = 0; r < 3; ++r) {
+      sel[r] = pre[r];
+      sel[3 + r] = want[r];
+      sel[6 + r] = below[r];
+    }
+  }
+}
+__device__ __forceinline__ void load_selection(const unsigned* sel, unsigned (&pre)[3],
+                                               unsigned (&want)[3], unsigned (&below)[3]) {
+  for (int r = 0; r < 3; ++r) {
+    pre[r] = sel[r];
+    want[r] = sel[3 + r];
+    below[r] = sel[6 + r];
   }
 }
 
 __device__ void select_l2(const unsigned* __restrict__ hist, unsigned (&pre)[3],
                           unsigned (&want)[3], unsigned (&below)[3]) {
   unsigned bin[3], bl[3], cnt[3];
+  load_selection(hist + kSelection1, pre, want, below);
   select_level<kL2>(hist + kL1, kL2, want, bin, bl, cnt);
   for (int r = 0; r < 3; ++r) {
     pre[r] = (pre[r] << kL2Bits) | bin[r];
@@ -1312,8 +1420,9 @@ __device__ __forceinline__ void stats_pass2_body(const float* __restrict__ v, in
                                                  unsigned* __restrict__ hist, unsigned* h) {
   unsigned pre[3], want[3], below[3];
   select_l1(hist, N, pre, want, below);
+  save_selection(hist + kSelection1, pre, want, below);
   const unsigned p0 = pre[0], p1 = pre[1], p2 = pre[2];
-  block_histogram<kL2>(
+  block_histogram<kL2, 3>(
       v, N, h, hist + kL1,
       [=](int r, unsigned k) {
         const unsigned top = k >> (32 - kL1Bits);
@@ -1336,10 +1445,10 @@ __global__ void __launch_bounds__(kStatsThreads) stats_pass2_set_kernel(FrontSet
 __device__ __forceinline__ void stats_pass3_body(const float* __restrict__ v, int N,
                                                  unsigned* __restrict__ hist, unsigned* h) {
   unsigned pre[3], want[3], below[3];
-  select_l1(hist, N, pre, want, below);
   select_l2(hist, pre, want, below);
+  save_selection(hist + kSelection2, pre, want, below);
   const unsigned p0 = pre[0], p1 = pre[1], p2 = pre[2];
-  block_histogram<kL3>(
+  block_histogram<kL3, 3>(
       v, N, h, hist + kL1 + 3 * kL2,
       [=](int r, unsigned k) {
         const unsigned top = k >> kL3Bits;
@@ -1359,12 +1468,11 @@ __global__ void __launch_bounds__(kStatsThreads) stats_pass3_set_kernel(FrontSet
   stats_pass3_body(fs.colsum[blockIdx.y], N, fs.hist[blockIdx.y], h);
 }
 
-// All three levels: exact keys, counts below and equal.
-__device__ void select_all(const unsigned* __restrict__ hist, int N, unsigned (&key)[3],
+// The last level: exact keys, counts below and equal.
+__device__ void select_all(const unsigned* __restrict__ hist, unsigned (&key)[3],
                            unsigned (&below)[3], unsigned (&equal)[3]) {
   unsigned pre[3], want[3];
-  select_l1(hist, N, pre, want, below);
-  select_l2(hist, pre, want, below);
+  load_selection(hist + kSelection2, pre, want, below);
   unsigned bin[3], bl[3], cnt[3];
   select_level<kL3>(hist + kL1 + 3 * kL2, kL3, want, bin, bl, cnt);
   for (int r = 0; r < 3; ++r) {
@@ -1374,15 +1482,16 @@ __device__ void select_all(const unsigned* __restrict__ hist, int N, unsigned (&
   }
 }
 
+// Sum over the workgroup in a fixed order (lanes by butterflies, then the
+// waves), returned to every thread. sh: one value per wave.
 template <typename V>
 __device__ __forceinline__ V block_sum(V x, V* sh) {
-  sh[threadIdx.x] = x;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) x += __shfl_xor(x, o);
+  if (threadIdx.x % kWave == 0) sh[threadIdx.x / kWave] = x;
   __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
-    __syncthreads();
-  }
-  const V r = sh[0];
+  V r = sh[0];
+  for (int w = 1; w < (int)blockDim.x / kWave; ++w) r += sh[w];
   __syncthreads();
   return r;
 }
@@ -1391,7 +1500,7 @@ __device__ __forceinline__ void stats_pass4_body(const float* __restrict__ v, in
                                                  const unsigned* __restrict__ hist,
                                                  StatsState* st, double* shd, unsigned* shu) {
   unsigned key[3], below[3], equal[3];
-  select_all(hist, N, key, below, equal);
+  select_all(hist, key, below, equal);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     for (int r = 0; r < 3; ++r) {
       st->key[r] = key[r];
@@ -1403,16 +1512,18 @@ __device__ __forceinline__ void stats_pass4_body(const float* __restrict__ v, in
   const double K = (double)ord_val(key[0]);
   double s1 = 0.0, s2 = 0.0;
   unsigned n = 0;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
-    const float x = v[i];
-    const unsigned k = ord_key(x);
-    if (k > k_lo && k < k_hi) {
-      const double d = __dsub_rn((double)x, K);
-      s1 = __dadd_rn(s1, d);
-      s2 = __dadd_rn(s2, __dmul_rn(d, d));
-      ++n;
-    }
-  }
+  for_each_value(
+      v, N,
+      [&](float x) {
+        const unsigned k = ord_key(x);
+        if (k > k_lo && k < k_hi) {
+          const double d = __dsub_rn((double)x, K);
+          s1 = __dadd_rn(s1, d);
+          s2 = __dadd_rn(s2, __dmul_rn(d, d));
+          ++n;
+        }
+      },
+      []() {});
   s1 = block_sum<double>(s1, shd);
   s2 = block_sum<double>(s2, shd);
   n = block_sum<unsigned>(n, shu);
@@ -1426,14 +1537,14 @@ __device__ __forceinline__ void stats_pass4_body(const float* __restrict__ v, in
 __global__ void __launch_bounds__(kStatsThreads)
     stats_pass4_kernel(const float* __restrict__ v, int N, const unsigned* __restrict__ hist,
                        StatsState* st) {
-  __shared__ double shd[kStatsThreads];
-  __shared__ unsigned shu[kStatsThreads];
+  __shared__ double shd[kStatsThreads / kWave];
+  __shared__ unsigned shu[kStatsThreads / kWave];
   stats_pass4_body(v, N, hist, st, shd, shu);
 }
 
 __global__ void __launch_bounds__(kStatsThreads) stats_pass4_set_kernel(FrontSet fs, int N) {
-  __shared__ double shd[kStatsThreads];
-  __shared__ unsigned shu[kStatsThreads];
+  __shared__ double shd[kStatsThreads / kWave];
+  __shared__ unsigned shu[kStatsThreads / kWave];
   stats_pass4_body(fs.colsum[blockIdx.y], N, fs.hist[blockIdx.y],
                    (StatsState*)fs.stats_scratch[blockIdx.y], shd, shu);
 }
@@ -1483,12 +1594,12 @@ __device__ __forceinline__ void stats_final_body(const StatsState* st, int N,
 __global__ void __launch_bounds__(kStatsThreads)
     stats_final_kernel(const StatsState* st, int N, const unsigned* __restrict__ hist,
                        float* __restrict__ stats_out) {
-  __shared__ double shd[kStatsThreads];
+  __shared__ double shd[kStatsThreads / kWave];
   stats_final_body(st, N, hist, stats_out, shd);
 }
 
 __global__ void __launch_bounds__(kStatsThreads) stats_final_set_kernel(FrontSet fs, int N) {
-  __shared__ double shd[kStatsThreads];
+  __shared__ double shd[kStatsThreads / kWave];
   stats_final_body((const StatsState*)fs.stats_scratch[blockIdx.y], N, fs.hist[blockIdx.y],
                    fs.stats_out[blockIdx.y], shd);
 }
@@ -1621,7 +1732,7 @@ constexpr int kNormBlocks = 512;
 
 __global__ void __launch_bounds__(256)
     norm_sum_kernel(const float* __restrict__ x, int T, int N, long stride, double* part) {
-  __shared__ double sh[256];
+  __shared__ double sh[256 / kWave];
   double s = 0.0;
   const long total = (long)T * N;
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < total;
@@ -1636,7 +1747,7 @@ __global__ void __launch_bounds__(256)
 __global__ void __launch_bounds__(256)
     norm_var_kernel(const float* __restrict__ x, int T, int N, long stride, const double* moments,
                     double* part) {
-  __shared__ double sh[256];
+  __shared__ double sh[256 / kWave];
   const double m = moments[0];
   double s = 0.0;
   const long total = (long)T * N;
@@ -2182,7 +2293,8 @@ hipError_t launch_unpack_top(const top_key_t* key, int N, int T, int bmin, float
   return hipGetLastError();
 }
 
-size_t device_stats_scratch_bytes(int /*N*/) { return sizeof(StatsState); }
+// (Whole 256-byte lines: the histograms may follow, read 16 bytes at a time.)
+size_t device_stats_scratch_bytes(int /*N*/) { return (sizeof(StatsState) + 255) / 256 * 256; }
 size_t device_stats_hist_bytes() { return sizeof(unsigned) * stats_hist_words(); }
 
 hipError_t launch_device_stats(const float* colsum, int N, void* scratch, unsigned* hist,
