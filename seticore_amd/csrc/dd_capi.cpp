@@ -1108,23 +1108,31 @@ sc_status sc_normalize(const float* data, int rounded_timesteps, int num_channel
   if (out_dtype != SC_F32 && out_dtype != SC_F16 && out_dtype != SC_BF16)
     return fail(SC_ERR_INVALID_ARGUMENT, "unknown dtype");
   hipStream_t stream = (hipStream_t)stream_ptr;
-  void* scratch = nullptr;
-  double* moments = nullptr;
-  SC_HIP(hipMalloc(&scratch, sc::normalize_scratch_bytes(rounded_timesteps, num_channels)),
-         "normalize scratch");
-  hipError_t e = hipMalloc((void**)&moments, 3 * sizeof(double));
-  if (e != hipSuccess) {
-    (void)hipFree(scratch);
-    return hip_fail(e, "normalize moments");
+  // The intermediates (column sums, partial moments, histograms) are done with
+  // before the first normalised sample is written, so they live in the output
+  // where it is large enough and lies apart from the input; else in memory
+  // allocated for the call.
+  const int T = rounded_timesteps, N = num_channels;
+  const size_t need = sc::norm_scratch_bytes(N);
+  const uintptr_t o0 = (uintptr_t)out, d0 = (uintptr_t)data;
+  const size_t out_bytes = (size_t)T * N * (out_dtype == SC_F32 ? 4 : 2);
+  const size_t in_bytes = ((size_t)(T - 1) * row_stride + N) * sizeof(float);
+  const uintptr_t base = (o0 + 255) / 256 * 256;
+  const bool apart = o0 + out_bytes <= d0 || d0 + in_bytes <= o0;
+  void* own = nullptr;
+  void* scratch = (void*)base;
+  if (!apart || base + need > o0 + out_bytes) {
+    SC_HIP(hipMalloc(&own, need), "normalize scratch");
+    scratch = own;
   }
-  e = sc::launch_normalize(data, rounded_timesteps, num_channels, row_stride, out_dtype, clamp,
-                           out, moments, scratch, stream);
   double h[3] = {0, 0, 0};
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(h, moments, sizeof(h), hipMemcpyDeviceToHost, stream);
+  hipError_t e = sc::launch_norm_moments(data, T, N, row_stride, scratch, stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(h, scratch, sizeof(h), hipMemcpyDeviceToHost, stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
-  (void)hipFree(scratch);
-  (void)hipFree(moments);
+  if (e == hipSuccess)
+    e = sc::launch_norm_apply(data, T, N, row_stride, out_dtype, h[2], h[1], clamp, out, stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(stream);
+  (void)hipFree(own);
   if (e != hipSuccess) return hip_fail(e, "normalize");
   if (loc_out) *loc_out = h[2];
   if (std_out) *std_out = h[1];

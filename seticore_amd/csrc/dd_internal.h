@@ -204,10 +204,14 @@ hipError_t launch_path_sums(const void* x, int dtype, long stride, int T, int N,
                             int n, hipStream_t stream);
 
 // ---- normalisation and synthetic data -------------------------------------
-hipError_t launch_normalize(const float* x, int T, int N, long stride, int out_dtype,
-                            float clamp, void* out, double* moments /* device: mean, std, location */,
-                            void* scratch, hipStream_t stream);
-size_t normalize_scratch_bytes(int T, int N);
+// {mean, standard deviation, location} of the samples as three doubles at the
+// start of scratch (norm_scratch_bytes, 256-byte aligned), then the pass that
+// writes (x - loc) / std_dev.
+hipError_t launch_norm_moments(const float* x, int T, int N, long stride, void* scratch,
+                               hipStream_t stream);
+hipError_t launch_norm_apply(const float* x, int T, int N, long stride, int out_dtype, double loc,
+                             double std_dev, float clamp, void* out, hipStream_t stream);
+size_t norm_scratch_bytes(int N);
 
 // Loader conditioning (zero rows T..T_r-1; optional DC fix on rows < T).
 hipError_t launch_condition(float* data, int T, int T_r, int N, long stride, int dc_spike,

@@ -1726,50 +1726,103 @@ __global__ void __launch_bounds__(256)
 }
 
 // ---------------------------------------------------------------------------
-// Normalisation for half-width storage: FP64 mean and deviation over the
-// T*N samples, two passes with fixed-order partial reduction.
-constexpr int kNormBlocks = 512;
+// Normalisation for half-width storage: the column sums and the FP64 mean and
+// deviation of the T*N samples in one pass over the input, then one pass that
+// writes. (A pass each for the column sums, the mean and the deviation, with
+// serial reductions between them, took 200 us at 16 x 2^20 where the reads
+// take 14 us each; the three in one take 25 us, a whole call 121 against
+// 400 us.)
 
-__global__ void __launch_bounds__(256)
-    norm_sum_kernel(const float* __restrict__ x, int T, int N, long stride, double* part) {
-  __shared__ double sh[256 / kWave];
-  double s = 0.0;
-  const long total = (long)T * N;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < total;
-       i += (long)gridDim.x * blockDim.x) {
-    const long t = i / N, c = i - t * N;
-    s += (double)x[t * stride + c];
-  }
-  s = block_sum<double>(s, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
+// Count, mean and sum of squared deviations of a set of samples; merged
+// pairwise, so the deviation keeps the accuracy of a second pass around the
+// mean whatever offset or outliers the samples have.
+struct Moments {
+  double n, mean, m2;
+};
+__device__ __forceinline__ Moments merge_moments(const Moments& a, const Moments& b) {
+  if (b.n == 0.0) return a;
+  if (a.n == 0.0) return b;
+  Moments r;
+  r.n = a.n + b.n;
+  const double delta = b.mean - a.mean, share = b.n / r.n;
+  r.mean = a.mean + delta * share;
+  r.m2 = a.m2 + b.m2 + delta * delta * (a.n * share);
+  return r;
 }
 
-__global__ void __launch_bounds__(256)
-    norm_var_kernel(const float* __restrict__ x, int T, int N, long stride, const double* moments,
-                    double* part) {
-  __shared__ double sh[256 / kWave];
-  const double m = moments[0];
-  double s = 0.0;
-  const long total = (long)T * N;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < total;
-       i += (long)gridDim.x * blockDim.x) {
-    const long t = i / N, c = i - t * N;
-    const double d = __dsub_rn((double)x[t * stride + c], m);
-    s = __dadd_rn(s, __dmul_rn(d, d));
+// Over the workgroup, in a fixed order; the result is in thread 0. sh: one per wave.
+__device__ __forceinline__ Moments block_moments(Moments m, Moments* sh) {
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    Moments u;
+    u.n = __shfl_down(m.n, o);
+    u.mean = __shfl_down(m.mean, o);
+    u.m2 = __shfl_down(m.m2, o);
+    if ((int)threadIdx.x % kWave + o < kWave) m = merge_moments(m, u);
   }
-  s = block_sum<double>(s, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
+  if (threadIdx.x % kWave == 0) sh[threadIdx.x / kWave] = m;
+  __syncthreads();
+  m = sh[0];
+  for (int w = 1; w < (int)blockDim.x / kWave; ++w) m = merge_moments(m, sh[w]);
+  return m;
 }
 
-__global__ void norm_final_kernel(const double* part, int n, double count, double* moments,
-                                  int which) {
+// One column per thread, 16 rows at a time: the column sum in row order
+// (dedoppler.cu:68-71) and the samples' moments; one partial per workgroup.
+// Also clears the statistics histograms.
+__global__ void __launch_bounds__(256)
+    norm_pass_kernel(const float* __restrict__ x, int T, int N, long stride,
+                     float* __restrict__ colsum, Moments* __restrict__ part,
+                     unsigned* __restrict__ hist, long nh) {
+  __shared__ Moments sh[256 / kWave];
+  const long c = blockIdx.x * 256L + threadIdx.x;
+  for (long i = c; i < nh; i += gridDim.x * 256L) hist[i] = 0;
+  Moments m = {0.0, 0.0, 0.0};
+  if (c < N) {
+    float s = 0.0f;
+    for (int t0 = 0; t0 < T; t0 += 16) {
+      const int n = min(16, T - t0);
+      float v[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (i < n) v[i] = x[(t0 + i) * stride + c];
+      double sum = 0.0, m2 = 0.0;
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (i < n) {
+          s += v[i];
+          sum += (double)v[i];
+        }
+      const double mean = sum / n;
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (i < n) {
+          const double d = (double)v[i] - mean;
+          m2 += d * d;
+        }
+      m = merge_moments(m, Moments{(double)n, mean, m2});
+    }
+    colsum[c] = s;
+  }
+  m = block_moments(m, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = m;
+}
+
+// moments = {mean, standard deviation, location}: the partials merged, and
+// the median column sum over T.
+__global__ void __launch_bounds__(1024)
+    norm_final_kernel(const Moments* __restrict__ part, int parts, int T,
+                      const unsigned* __restrict__ hist, double* __restrict__ moments) {
+  __shared__ Moments sh[1024 / kWave];
+  unsigned key[3], below[3], equal[3];
+  select_all(hist, key, below, equal);
+  Moments m = {0.0, 0.0, 0.0};
+  for (int i = threadIdx.x; i < parts; i += 1024) m = merge_moments(m, part[i]);
+  m = block_moments(m, sh);
   if (threadIdx.x != 0) return;
-  double s = 0.0;
-  for (int i = 0; i < n; ++i) s = __dadd_rn(s, part[i]);
-  if (which == 0)
-    moments[0] = s / count;
-  else
-    moments[1] = sqrt(s / count);
+  moments[0] = m.mean;
+  moments[1] = sqrt(m.m2 / m.n);
+  moments[2] = (double)ord_val(key[0]) / (double)T;
 }
 
 template <typename Out>
@@ -1783,24 +1836,30 @@ __device__ __forceinline__ __hip_bfloat16 from_f32<__hip_bfloat16>(float v) {
 template <>
 __device__ __forceinline__ float from_f32<float>(float v) { return v; }
 
-// Location of the normalisation: the median column sum over T (stats_out[0]
-// from the device statistics of the raw column sums).
-__global__ void norm_location_kernel(const float* stats_out, int T, double* moments) {
-  if (threadIdx.x == 0) moments[2] = (double)stats_out[0] / (double)T;
-}
-
+// Four consecutive samples of a row per thread (rows at any 4-byte or, written,
+// element alignment); grid.y = row, strided where there are more than 65535.
 template <typename Out>
-__global__ void norm_apply_kernel(const float* __restrict__ x, int T, int N, long stride,
-                                  const double* moments, float clamp, Out* __restrict__ out) {
-  const double m = moments[2];
-  const double sd = moments[1] > 0.0 ? moments[1] : 1.0;
-  const long total = (long)T * N;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < total;
-       i += (long)gridDim.x * blockDim.x) {
-    const long t = i / N, c = i - t * N;
-    float v = (float)((double)x[t * stride + c] - m) / (float)sd;
-    v = fminf(fmaxf(v, -clamp), clamp);
-    out[i] = from_f32<Out>(v);
+__global__ void __launch_bounds__(256)
+    norm_apply_kernel(const float* __restrict__ x, int T, int N, long stride, double loc, float sd,
+                      float clamp, Out* __restrict__ out) {
+  typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+  struct __attribute__((packed, aligned(sizeof(Out)))) Out4 {
+    Out v[4];
+  };
+  const long c = (blockIdx.x * 256L + threadIdx.x) * 4;
+  auto scaled = [=](float v) {
+    v = (float)((double)v - loc) / sd;
+    return from_f32<Out>(fminf(fmaxf(v, -clamp), clamp));
+  };
+  for (int t = blockIdx.y; t < T; t += gridDim.y) {
+    const float* row = x + t * stride;
+    Out* dst = out + (long)t * N;
+    if (c + 4 <= N) {
+      const f4u q = *(const f4u*)(row + c);
+      *(Out4*)(dst + c) = Out4{{scaled(q.x), scaled(q.y), scaled(q.z), scaled(q.w)}};
+    } else {
+      for (long i = c; i < N; ++i) dst[i] = scaled(row[i]);
+    }
   }
 }
 
@@ -2378,64 +2437,63 @@ hipError_t launch_path_sums(const void* x, int dtype, long stride, int T, int N,
 }
 
 namespace {
-// Scratch of launch_normalize: partial sums, column sums, statistics state,
-// histograms, statistics output.
+// Scratch of launch_norm_moments: moments out, partial moments, column sums,
+// statistics state (unused by the median alone), histograms.
 constexpr size_t norm_align(size_t n) { return (n + 255) / 256 * 256; }
 struct NormScratch {
-  size_t part, colsum, state, hist, stats, total;
+  int parts;
+  size_t moments, part, colsum, hist, total;
   explicit NormScratch(int N) {
-    part = 0;
-    colsum = norm_align(sizeof(double) * kNormBlocks);
-    state = colsum + norm_align(sizeof(float) * (size_t)N);
-    hist = state + norm_align(device_stats_scratch_bytes(N));
-    stats = hist + norm_align(device_stats_hist_bytes());
-    total = stats + norm_align(4 * sizeof(float));
+    parts = (int)(((long)N + 255) / 256);
+    moments = 0;
+    part = norm_align(3 * sizeof(double));
+    colsum = part + norm_align(sizeof(Moments) * (size_t)parts);
+    hist = colsum + norm_align(sizeof(float) * (size_t)N);
+    total = hist + norm_align(device_stats_hist_bytes());
   }
 };
 }  // namespace
 
-size_t normalize_scratch_bytes(int /*T*/, int N) { return NormScratch(N).total; }
+size_t norm_scratch_bytes(int N) { return NormScratch(N).total; }
 
-hipError_t launch_normalize(const float* x, int T, int N, long stride, int out_dtype, float clamp,
-                            void* out, double* moments, void* scratch, hipStream_t stream) {
+hipError_t launch_norm_moments(const float* x, int T, int N, long stride, void* scratch,
+                               hipStream_t stream) {
   const NormScratch L(N);
   char* base = (char*)scratch;
-  double* part = (double*)(base + L.part);
-  const double count = (double)T * (double)N;
   // Location: the median of the raw column sums over T, so the normalised
   // column sums have median ~0 whatever share of the power narrowband RFI
   // holds (the mean would put them far below zero): every positive SNR
   // threshold then lies above the zero the top path sums start from.
   float* colsum = (float*)(base + L.colsum);
+  Moments* part = (Moments*)(base + L.part);
   unsigned* hist = (unsigned*)(base + L.hist);
-  float* stats = (float*)(base + L.stats);
-  hipError_t e = launch_colsum(x, 0, stride, T, N, colsum, stream);
-  if (e == hipSuccess) e = launch_reset(nullptr, 0, hist, stream);
-  if (e == hipSuccess)
-    e = launch_device_stats(colsum, N, base + L.state, hist, stats, stream);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(norm_location_kernel, dim3(1), dim3(64), 0, stream, stats, T, moments);
-  hipLaunchKernelGGL(norm_sum_kernel, dim3(kNormBlocks), dim3(256), 0, stream, x, T, N, stride,
-                     part);
-  hipLaunchKernelGGL(norm_final_kernel, dim3(1), dim3(64), 0, stream, part, kNormBlocks, count,
-                     moments, 0);
-  hipLaunchKernelGGL(norm_var_kernel, dim3(kNormBlocks), dim3(256), 0, stream, x, T, N, stride,
-                     moments, part);
-  hipLaunchKernelGGL(norm_final_kernel, dim3(1), dim3(64), 0, stream, part, kNormBlocks, count,
-                     moments, 1);
-  const int nb = blocks_for((long)T * N, 256, 8192);
+  const dim3 grid(kStatsBlocks), block(kStatsThreads);
+  hipLaunchKernelGGL(norm_pass_kernel, dim3(L.parts), dim3(256), 0, stream, x, T, N, stride,
+                     colsum, part, hist, (long)stats_hist_words());
+  hipLaunchKernelGGL(stats_pass1_kernel, grid, block, 0, stream, colsum, N, hist);
+  hipLaunchKernelGGL(stats_pass2_kernel, grid, block, 0, stream, colsum, N, hist);
+  hipLaunchKernelGGL(stats_pass3_kernel, grid, block, 0, stream, colsum, N, hist);
+  hipLaunchKernelGGL(norm_final_kernel, dim3(1), dim3(1024), 0, stream, part, L.parts, T, hist,
+                     (double*)(base + L.moments));
+  return hipGetLastError();
+}
+
+hipError_t launch_norm_apply(const float* x, int T, int N, long stride, int out_dtype, double loc,
+                             double std_dev, float clamp, void* out, hipStream_t stream) {
+  const float sd = (float)(std_dev > 0.0 ? std_dev : 1.0);
+  const dim3 grid((unsigned)(((long)N + 1023) / 1024), std::min(T, 65535)), block(256);
   switch (out_dtype) {
     case 0:
-      hipLaunchKernelGGL(norm_apply_kernel<float>, dim3(nb), dim3(256), 0, stream, x, T, N,
-                         stride, moments, clamp, (float*)out);
+      hipLaunchKernelGGL(norm_apply_kernel<float>, grid, block, 0, stream, x, T, N, stride, loc,
+                         sd, clamp, (float*)out);
       break;
     case 1:
-      hipLaunchKernelGGL(norm_apply_kernel<__half>, dim3(nb), dim3(256), 0, stream, x, T, N,
-                         stride, moments, clamp, (__half*)out);
+      hipLaunchKernelGGL(norm_apply_kernel<__half>, grid, block, 0, stream, x, T, N, stride, loc,
+                         sd, clamp, (__half*)out);
       break;
     case 2:
-      hipLaunchKernelGGL(norm_apply_kernel<__hip_bfloat16>, dim3(nb), dim3(256), 0, stream, x, T,
-                         N, stride, moments, clamp, (__hip_bfloat16*)out);
+      hipLaunchKernelGGL(norm_apply_kernel<__hip_bfloat16>, grid, block, 0, stream, x, T, N,
+                         stride, loc, sd, clamp, (__hip_bfloat16*)out);
       break;
     default: return hipErrorInvalidValue;
   }

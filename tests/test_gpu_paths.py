@@ -72,3 +72,36 @@ def test_incoherent_power_of_any_path(gpu, oracle, T, N, dtype, n):
             trees[b] = oracle.basic_taylor_tree(host, b)
         assert h.incoherent_power == trees[b][p, h.index]
     assert [h.drift_steps for h in hits] == sorted(h.drift_steps for h in hits)
+
+
+# The output holds the intermediates where it is large enough (16 rows: from about 2 300 channels on in
+# 16 bits) and apart from the input; odd widths, more rows than a load group, strided rows.
+@pytest.mark.parametrize("T,N,stride,dtype", [
+    (1, 1, 1, "f32"), (16, 1000, 1000, "bf16"), (16, 2401, 2403, "f16"), (17, 5003, 5003, "bf16"),
+    (13, 70001, 70001, "f32"), (100, 4099, 4100, "bf16")])
+def test_normalize_against_float64(gpu, T, N, stride, dtype):
+    import torch
+    code, kind = {"f32": (sc.SC_F32, torch.float32), "f16": (sc.SC_F16, torch.float16),
+                  "bf16": (sc.SC_BF16, torch.bfloat16)}[dtype]
+    rng = np.random.default_rng(N)
+    x = (rng.exponential(size=(T, stride)) * 3.0 + 1000.0).astype(np.float32)
+    if N > 1000:
+        x[:, N // 3] = 1e8  # an interferer that holds nearly all of the power
+    d = torch.from_numpy(x).cuda()[:, :N]
+    print("normalize", T, N, stride, dtype, flush=True)
+    y, loc, sd = sc.normalize(d, code)
+    colsum = np.zeros(N, np.float32)
+    for t in range(T):
+        colsum += x[t, :N]
+    assert loc == float(np.partition(colsum, N // 2)[N // 2]) / T
+    v = x[:, :N].astype(np.float64)
+    # A few hundred FP64 roundings at most separate the merged moments from the two-pass ones.
+    np.testing.assert_allclose(sd, v.std(), rtol=1e-12, atol=0)
+    div = np.float32(sd if sd > 0 else 1.0)
+    want = ((v - loc).astype(np.float32) / div).clip(-65504.0, 65504.0)
+    np.testing.assert_array_equal(y.cpu().float().numpy(),
+                                  torch.from_numpy(want).to(kind).float().numpy())
+    if dtype == "f32" and stride == N:
+        z, loc2, sd2 = sc.normalize(d, code, out=d)  # in place
+        assert (loc2, sd2) == (loc, sd)
+        np.testing.assert_array_equal(z.cpu().numpy(), y.cpu().numpy())
