@@ -831,18 +831,12 @@ sc_status sc_dd_search(sc_dd* dd, const void* data, int dtype, int rounded_times
   if (host_stats) {
     s = enqueue_path_sums(dd, data, dtype, row_stride, r, stream);
     if (s != SC_OK) return s;
-    SC_HIP(sc::launch_unpack_top(dd->top_key, N, T, r.bmin, dd->top_sum, dd->top_blk,
-                                 dd->top_off, stream),
+    // The three top arrays, and with the column sums to the host
+    // (dedoppler.cu:232-240).
+    SC_HIP(sc::launch_unpack_top(dd->top_key, dd->colsum, N, T, r.bmin, dd->top_sum, dd->top_blk,
+                                 dd->top_off, dd->h_colsum, dd->h_top_sum, dd->h_top_blk,
+                                 dd->h_top_off, stream),
            "unpack top");
-    // dedoppler.cu:232-240
-    SC_HIP(hipMemcpyAsync(dd->h_colsum, dd->colsum, N * sizeof(float), hipMemcpyDeviceToHost,
-                          stream), "copy column sums");
-    SC_HIP(hipMemcpyAsync(dd->h_top_sum, dd->top_sum, N * sizeof(float), hipMemcpyDeviceToHost,
-                          stream), "copy top sums");
-    SC_HIP(hipMemcpyAsync(dd->h_top_blk, dd->top_blk, N * sizeof(int), hipMemcpyDeviceToHost,
-                          stream), "copy top blocks");
-    SC_HIP(hipMemcpyAsync(dd->h_top_off, dd->top_off, N * sizeof(int), hipMemcpyDeviceToHost,
-                          stream), "copy top offsets");
     SC_HIP(hipStreamSynchronize(stream), "search");
     // NaN or infinite samples make their column's sum non-finite (bit test:
     // exponent all ones). The key arithmetic assumes finite samples.

@@ -1089,20 +1089,36 @@ __global__ void reset_set_kernel(FrontSet fs, long n, long nh) {
   reset_body(fs.key[blockIdx.y], n, fs.hist[blockIdx.y], nh);
 }
 
-__global__ void unpack_top_kernel(const top_key_t* __restrict__ key, int N, int T, int bmin,
+// Also writes the three arrays and the column sums to their mirrors in host
+// memory (dedoppler.cu:232-240): a search of 13 x 5003 took 87 us with a copy
+// each and takes 57 us; at 16 x 2^20 the 16 MB cross at the same rate either way.
+__global__ void unpack_top_kernel(const top_key_t* __restrict__ key,
+                                  const float* __restrict__ colsum, int N, int T, int bmin,
                                   float* __restrict__ top_sum, int* __restrict__ top_blk,
-                                  int* __restrict__ top_off) {
+                                  int* __restrict__ top_off, float* __restrict__ h_colsum,
+                                  float* __restrict__ h_sum, int* __restrict__ h_blk,
+                                  int* __restrict__ h_off) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= N) return;
   const top_key_t k = key[c];
+  float sum = 0.0f;  // block/offset keep their previous values (dedoppler.cu:205)
+  int blk, off;
   if (k == 0) {
-    top_sum[c] = 0.0f;  // block/offset keep their previous values (dedoppler.cu:205)
+    blk = top_blk[c];
+    off = top_off[c];
   } else {
     const unsigned code = (unsigned)(kCodeMask - (k & kCodeMask));
-    top_sum[c] = key_sum(k);
-    top_blk[c] = (int)(code / (unsigned)T) + bmin;
-    top_off[c] = (int)(code % (unsigned)T);
+    sum = key_sum(k);
+    blk = (int)(code / (unsigned)T) + bmin;
+    off = (int)(code % (unsigned)T);
+    top_blk[c] = blk;
+    top_off[c] = off;
   }
+  top_sum[c] = sum;
+  h_colsum[c] = colsum[c];
+  h_sum[c] = sum;
+  h_blk[c] = blk;
+  h_off[c] = off;
 }
 
 // ---------------------------------------------------------------------------
@@ -2345,10 +2361,11 @@ hipError_t launch_reset(top_key_t* key, long n, unsigned* hist, hipStream_t stre
   return hipGetLastError();
 }
 
-hipError_t launch_unpack_top(const top_key_t* key, int N, int T, int bmin, float* top_sum,
-                             int* top_blk, int* top_off, hipStream_t stream) {
-  hipLaunchKernelGGL(unpack_top_kernel, dim3((N + 255) / 256), dim3(256), 0, stream, key, N, T,
-                     bmin, top_sum, top_blk, top_off);
+hipError_t launch_unpack_top(const top_key_t* key, const float* colsum, int N, int T, int bmin,
+                             float* top_sum, int* top_blk, int* top_off, float* h_colsum,
+                             float* h_sum, int* h_blk, int* h_off, hipStream_t stream) {
+  hipLaunchKernelGGL(unpack_top_kernel, dim3((N + 255) / 256), dim3(256), 0, stream, key, colsum,
+                     N, T, bmin, top_sum, top_blk, top_off, h_colsum, h_sum, h_blk, h_off);
   return hipGetLastError();
 }
 
