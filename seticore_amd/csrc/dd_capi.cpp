@@ -16,6 +16,8 @@
 #include <mutex>
 #include <numeric>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../include/seticore_amd.h"
@@ -284,6 +286,11 @@ sc_status run_tree(sc_dd* dd, const void* data, int dtype, long stride, int drif
   return SC_OK;
 }
 
+// From this many channels on, a host-exact search's statistics use a second
+// thread and run while the tree does; below, a thread or a further stream costs
+// more than it saves (a 13 x 5003 search takes 57 us in all).
+constexpr int kParallelStats = 65536;
+
 // dedoppler.cu:241-262, same calls on a copy of the column sums.
 void host_exact_stats(const float* colsums, int n, float* median_out, float* std_out) {
   std::vector<float> v(colsums, colsums + n);
@@ -293,8 +300,21 @@ void host_exact_stats(const float* colsums, int n, float* median_out, float* std
   std::nth_element(sums, sums + mid, end);
   int first = (int)std::ceil(0.05 * n);
   int last = (int)std::floor(0.95 * n);
+  // The two ranges are disjoint: from kParallelStats values on, a thread of its
+  // own selects in the upper one (17 % of a 16 x 2^20 search, whose time is
+  // mostly these three calls).
+  std::thread upper;
+  if (n >= kParallelStats) {
+    try {
+      upper = std::thread([=] { std::nth_element(sums + mid + 1, sums + last, end); });
+    } catch (const std::system_error&) {
+    }
+  }
   std::nth_element(sums, sums + first, sums + mid - 1);
-  std::nth_element(sums + mid + 1, sums + last, end);
+  if (upper.joinable())
+    upper.join();
+  else
+    std::nth_element(sums + mid + 1, sums + last, end);
   float median = sums[mid];
   float sum = std::accumulate(sums + first, sums + last + 1, 0.0);
   float m = sum / (last + 1 - first);
@@ -544,7 +564,9 @@ namespace {
 // sums (their own kernel) and the statistics run on the handle's second
 // stream while the path-sum kernels run on `stream` (the statistics need only
 // the column sums); `stream` waits for them at the end, so the tail is then
-// just the window merge.
+// just the window merge. With host_stats as well, the side stream copies the
+// column sums to the host instead (ev_join), for statistics made there
+// meanwhile.
 //
 // Searches that end in the device tail carry block keys when the one-pass
 // kernel is the T_r <= 16 or the staged one (block_key_search): the tail
@@ -556,7 +578,8 @@ bool block_key_search(const sc_dd* dd) {
 
 sc_status enqueue_path_sums(sc_dd* dd, const void* data, int dtype, long row_stride,
                             const DriftRange& r, hipStream_t stream,
-                            bool overlap_stats = false, bool device_tail = false) {
+                            bool overlap_stats = false, bool device_tail = false,
+                            bool host_stats = false) {
   const int T = dd->rounded, N = dd->num_channels;
   const int nblocks = r.bmax - r.bmin + 1;
   // dedoppler.cu:205 (the reference zeroes the float sums; the key 0 means "no
@@ -606,9 +629,14 @@ sc_status enqueue_path_sums(sc_dd* dd, const void* data, int dtype, long row_str
     SC_HIP(hipStreamWaitEvent(dd->aux_stream, dd->ev_fork, 0), "fork");
     SC_HIP(sc::launch_colsum(data, dtype, row_stride, T, N, dd->colsum, dd->aux_stream),
            "column sums");
-    SC_HIP(sc::launch_device_stats(dd->colsum, N, dd->stats_scratch, dd->stats_hist,
-                                   dd->stats_out, dd->aux_stream),
-           "device stats");
+    if (host_stats)
+      SC_HIP(hipMemcpyAsync(dd->h_colsum, dd->colsum, N * sizeof(float), hipMemcpyDeviceToHost,
+                            dd->aux_stream),
+             "copy column sums");
+    else
+      SC_HIP(sc::launch_device_stats(dd->colsum, N, dd->stats_scratch, dd->stats_hist,
+                                     dd->stats_out, dd->aux_stream),
+             "device stats");
     SC_HIP(hipEventRecord(dd->ev_join, dd->aux_stream), "join");
     SC_HIP(hipStreamWaitEvent(stream, dd->ev_join, 0), "join");
   }
@@ -829,15 +857,19 @@ sc_status sc_dd_search(sc_dd* dd, const void* data, int dtype, int rounded_times
   // calls have empty ranges below a few channels).
   const bool host_stats = dd->stats_mode == SC_STATS_HOST_EXACT || N < 4096;
   if (host_stats) {
-    s = enqueue_path_sums(dd, data, dtype, row_stride, r, stream);
+    const bool beside = N >= kParallelStats;
+    s = enqueue_path_sums(dd, data, dtype, row_stride, r, stream, beside, false, beside);
     if (s != SC_OK) return s;
     // The three top arrays, and with the column sums to the host
     // (dedoppler.cu:232-240).
     SC_HIP(sc::launch_unpack_top(dd->top_key, dd->colsum, N, T, r.bmin, dd->top_sum, dd->top_blk,
-                                 dd->top_off, dd->h_colsum, dd->h_top_sum, dd->h_top_blk,
-                                 dd->h_top_off, stream),
+                                 dd->top_off, beside ? nullptr : dd->h_colsum, dd->h_top_sum,
+                                 dd->h_top_blk, dd->h_top_off, stream),
            "unpack top");
-    SC_HIP(hipStreamSynchronize(stream), "search");
+    if (beside)
+      SC_HIP(hipEventSynchronize(dd->ev_join), "column sums");
+    else
+      SC_HIP(hipStreamSynchronize(stream), "search");
     // NaN or infinite samples make their column's sum non-finite (bit test:
     // exponent all ones). The key arithmetic assumes finite samples.
     long bad = 0;
@@ -846,11 +878,12 @@ sc_status sc_dd_search(sc_dd* dd, const void* data, int dtype, int rounded_times
       std::memcpy(&u, &dd->h_colsum[c], sizeof(u));
       bad += (u & 0x7F800000u) == 0x7F800000u;
     }
+    float median = 0.0f, std_dev = 0.0f;
+    if (!bad) host_exact_stats(dd->h_colsum, N, &median, &std_dev);
+    if (beside) SC_HIP(hipStreamSynchronize(stream), "search");
     if (bad)
       return fail(SC_ERR_INVALID_ARGUMENT, "input has NaN or infinite samples (" +
                                                std::to_string(bad) + " non-finite column sums)");
-    float median, std_dev;
-    host_exact_stats(dd->h_colsum, N, &median, &std_dev);
     dd->last_median = median;
     dd->last_std = std_dev;
     host_merge(dd, r, meta, beam, coarse_channel, min_drift, snr_threshold, median, std_dev);

@@ -169,8 +169,8 @@ hipError_t launch_reset(top_key_t* key, long n, unsigned* hist, hipStream_t stre
 
 // Unpacks keys into the reference's three top arrays; channels without a
 // positive path get top_sum 0 and keep their previous block/offset.
-// h_colsum, h_sum, h_blk, h_off: host-visible mirrors of the column sums and of
-// the three arrays, written by the same kernel.
+// h_colsum (may be null), h_sum, h_blk, h_off: host-visible mirrors of the
+// column sums and of the three arrays, written by the same kernel.
 hipError_t launch_unpack_top(const top_key_t* key, const float* colsum, int N, int T, int bmin,
                              float* top_sum, int* top_blk, int* top_off, float* h_colsum,
                              float* h_sum, int* h_blk, int* h_off, hipStream_t stream);

@@ -1115,7 +1115,7 @@ __global__ void unpack_top_kernel(const top_key_t* __restrict__ key,
     top_off[c] = off;
   }
   top_sum[c] = sum;
-  h_colsum[c] = colsum[c];
+  if (h_colsum) h_colsum[c] = colsum[c];
   h_sum[c] = sum;
   h_blk[c] = blk;
   h_off[c] = off;
