@@ -285,8 +285,16 @@ __global__ void __launch_bounds__(256)
 }
 
 // One workgroup per block: the whole parameter gradient of that block's loss
-// term into gpart[b][kNumParams] (every entry written).
-__global__ void __launch_bounds__(256)
+// term into gpart[b][kNumParams] (every entry written). Everything the block's
+// argmax position depends on - 3x5 positions of h2, 7x13 of h1, 9x29 of z and
+// conv2's weights - is first brought into LDS, zero outside the maps, so the
+// sums below are free of bounds tests and of memory latency: at 256 blocks
+// (one workgroup per CU) 127 us with global loads inside the sums on 256
+// threads, 21 us now.
+constexpr int kBackThreads = 512;
+constexpr int kR1H = 7, kR1W = 13, kR1 = kR1H * kR1W;  // receptive field in h1
+constexpr int kRZH = kR1H + 2, kRZW = 2 * kR1W + 3;    // and in z
+__global__ void __launch_bounds__(kBackThreads)
     backward_kernel(const unsigned short* __restrict__ z, const unsigned short* __restrict__ h1,
                     const unsigned short* __restrict__ h2, const unsigned short* __restrict__ h3,
                     const int* __restrict__ argmax, const float* __restrict__ dz,
@@ -296,18 +304,43 @@ __global__ void __launch_bounds__(256)
   const int tid = threadIdx.x;
   float* g = gpart + b * (long)kNumParams;
   __shared__ float dY3[kC3];
-  __shared__ float dY2[15][kC2];   // conv2 outputs at the 15 taps of conv3
-  __shared__ int p2y[15], p2x[15];  // their coordinates (-1: padding)
-  __shared__ float dY1[7 * 13][kC1];
+  __shared__ float h2s[15][kC2];
+  __shared__ __attribute__((aligned(16))) float dY2[15][kC2];  // conv2 outputs at conv3's taps
+  __shared__ float h1s[kR1][kC1];
+  __shared__ float dY1[kR1][kC1];
+  __shared__ float zs[kRZH][kRZW];
+  __shared__ unsigned short w2s[kC2 * 15 * kC1];
 
   const int pos = argmax[b];
   const int y3 = pos / kW3, x3 = pos % kW3;
   const float d = dz[b];
-  const unsigned short* h3p = h3 + ((b * kH3 + y3) * kW3 + x3) * kC3;
+
+  // Tap t of conv3 reads h2 at (2 y3 + t/5 - 1, 2 x3 + t%5 - 2); tap t2 of
+  // conv2 at conv3's tap j reads cell (2 (j/5) + t2/5, 2 (j%5) + t2%5) of the
+  // h1 field, whose corner is (4 y3 - 3, 4 x3 - 6); tap t of conv1 at an h1
+  // cell (y, x) reads cell (y + t/5, 2 x + t%5) of the z field.
+  const int y1o = 4 * y3 - 3, x1o = 4 * x3 - 6;
+  if (tid < 15 * kC2) {
+    const int t = tid / kC2, yy = 2 * y3 + t / 5 - 1, xx = 2 * x3 + t % 5 - 2;
+    const bool ok = yy >= 0 && yy < kH2 && xx >= 0 && xx < kW2;
+    h2s[t][tid % kC2] = ok ? bf2f(h2[((b * kH2 + yy) * kW2 + xx) * kC2 + tid % kC2]) : 0.0f;
+  }
+  for (int e = tid; e < kR1 * kC1; e += kBackThreads) {
+    const int cell = e / kC1, yy = y1o + cell / kR1W, xx = x1o + cell % kR1W;
+    const bool ok = yy >= 0 && yy < kH1 && xx >= 0 && xx < kW1;
+    h1s[cell][e % kC1] = ok ? bf2f(h1[((b * kH1 + yy) * kW1 + xx) * kC1 + e % kC1]) : 0.0f;
+  }
+  if (tid < kRZH * kRZW) {
+    const int zy = y1o - 1 + tid / kRZW, zx = 2 * x1o - 2 + tid % kRZW;
+    const bool ok = zy >= 0 && zy < kRows && zx >= 0 && zx < kPooled;
+    zs[tid / kRZW][tid % kRZW] = ok ? bf2f(z[(b * kRows + zy) * kPooled + zx]) : 0.0f;
+  }
+  for (int e = tid; e < kC2 * 15 * kC1 / 2; e += kBackThreads)
+    ((unsigned*)w2s)[e] = ((const unsigned*)w2b)[e];
 
   // Head and conv3 bias.
   if (tid < kC3) {
-    const float a = bf2f(h3p[tid]);
+    const float a = bf2f(h3[((b * kH3 + y3) * kW3 + x3) * kC3 + tid]);
     g[kOffWH + tid] = d * a;
     const float dh = d * params[kOffWH + tid];
     const float dy = a > 0.0f ? dh : 0.0f;
@@ -315,104 +348,102 @@ __global__ void __launch_bounds__(256)
     g[kOffB3 + tid] = dy;
   }
   if (tid == 0) g[kOffBH] = d;
-  if (tid < 15) {
-    const int yy = 2 * y3 + tid / 5 - 1, xx = 2 * x3 + tid % 5 - 2;
-    const bool ok = yy >= 0 && yy < kH2 && xx >= 0 && xx < kW2;
-    p2y[tid] = ok ? yy : -1;
-    p2x[tid] = ok ? xx : -1;
-  }
   __syncthreads();
 
   // conv3 weights: dW3[co][t][ci] = dY3[co] * h2[p2(t)][ci].
-  for (int e = tid; e < kC3 * 15 * kC2; e += 256) {
-    const int ci = e % kC2, t = (e / kC2) % 15, co = e / (kC2 * 15);
-    float v = 0.0f;
-    if (p2y[t] >= 0) v = dY3[co] * bf2f(h2[((b * kH2 + p2y[t]) * kW2 + p2x[t]) * kC2 + ci]);
-    g[kOffW3 + e] = v;
-  }
+  for (int e = tid; e < kC3 * 15 * kC2; e += kBackThreads)
+    g[kOffW3 + e] = dY3[e / (kC2 * 15)] * h2s[(e / kC2) % 15][e % kC2];
   // Gradient at the 15 conv2 outputs, through the ReLU.
-  for (int e = tid; e < 15 * kC2; e += 256) {
-    const int ci = e % kC2, t = e / kC2;
-    float v = 0.0f;
-    if (p2y[t] >= 0) {
-      const float a = bf2f(h2[((b * kH2 + p2y[t]) * kW2 + p2x[t]) * kC2 + ci]);
-      if (a > 0.0f) {
-        float s = 0.0f;
-        for (int co = 0; co < kC3; ++co) s += dY3[co] * bf2f(w3b[(co * 15 + t) * kC2 + ci]);
-        v = s;
-      }
-    }
-    dY2[t][ci] = v;
+  if (tid < 15 * kC2) {
+    const int ci = tid % kC2, t = tid / kC2;
+    float s = 0.0f;
+#pragma unroll
+    for (int co = 0; co < kC3; ++co) s += dY3[co] * bf2f(w3b[(co * 15 + t) * kC2 + ci]);
+    dY2[t][ci] = h2s[t][ci] > 0.0f ? s : 0.0f;
   }
   __syncthreads();
 
-  // conv2 bias and weights: dW2[co][t2][ci] = sum_j dY2[j][co] * h1[2*p2(j) + tap(t2)][ci].
+  // conv2 bias and weights: dW2[co][t2][ci] = sum_j dY2[j][co] * h1[cell(j, t2)][ci],
+  // 16 output channels per thread.
   if (tid < kC2) {
     float s = 0.0f;
     for (int j = 0; j < 15; ++j) s += dY2[j][tid];
     g[kOffB2 + tid] = s;
   }
-  for (int e = tid; e < kC2 * 15 * kC1; e += 256) {
-    const int ci = e % kC1, t2 = (e / kC1) % 15, co = e / (kC1 * 15);
+  if (tid < 2 * 15 * kC1) {
+    const int e = tid % (15 * kC1), co0 = 16 * (tid / (15 * kC1));
+    const int ci = e % kC1, t2 = e / kC1;
+    const int c0 = t2 / 5 * kR1W + t2 % 5;
+    float acc[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 15; ++j) {
+      const float h = h1s[c0 + j / 5 * 2 * kR1W + j % 5 * 2][ci];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[i] += dY2[j][co0 + i] * h;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) g[kOffW2 + (co0 + i) * 15 * kC1 + e] = acc[i];
+  }
+  // Gradient at the h1 field, through the ReLU.
+  for (int e = tid; e < kR1 * kC1; e += kBackThreads) {
+    const int ci = e % kC1, cell = e / kC1, cy = cell / kR1W, cx = cell % kR1W;
     float s = 0.0f;
     for (int j = 0; j < 15; ++j) {
-      if (p2y[j] < 0) continue;
-      const int yy = 2 * p2y[j] + t2 / 5 - 1, xx = 2 * p2x[j] + t2 % 5 - 2;
-      if (yy < 0 || yy >= kH1 || xx < 0 || xx >= kW1) continue;
-      s += dY2[j][co] * bf2f(h1[((b * kH1 + yy) * kW1 + xx) * kC1 + ci]);
+      const int ty = cy - j / 5 * 2, tx = cx - j % 5 * 2;
+      if (ty < 0 || ty >= 3 || tx < 0 || tx >= 5) continue;
+      const unsigned short* w = w2s + (ty * 5 + tx) * kC1 + ci;
+#pragma unroll
+      for (int co = 0; co < kC2; ++co) s += dY2[j][co] * bf2f(w[co * 15 * kC1]);
     }
-    g[kOffW2 + e] = s;
-  }
-  // Gradient at h1 over the 7x13 region rows 4*y3-3.., cols 4*x3-6.., through the ReLU.
-  const int y1o = 4 * y3 - 3, x1o = 4 * x3 - 6;
-  for (int e = tid; e < 7 * 13 * kC1; e += 256) {
-    const int ci = e % kC1, cell = e / kC1;
-    const int yy = y1o + cell / 13, xx = x1o + cell % 13;
-    float v = 0.0f;
-    if (yy >= 0 && yy < kH1 && xx >= 0 && xx < kW1 &&
-        bf2f(h1[((b * kH1 + yy) * kW1 + xx) * kC1 + ci]) > 0.0f) {
-      float s = 0.0f;
-      for (int j = 0; j < 15; ++j) {
-        if (p2y[j] < 0) continue;
-        const int ty = yy - 2 * p2y[j] + 1, tx = xx - 2 * p2x[j] + 2;
-        if (ty < 0 || ty >= 3 || tx < 0 || tx >= 5) continue;
-        const int t2 = ty * 5 + tx;
-        for (int co = 0; co < kC2; ++co) s += dY2[j][co] * bf2f(w2b[(co * 15 + t2) * kC1 + ci]);
-      }
-      v = s;
-    }
-    dY1[cell][ci] = v;
+    dY1[cell][ci] = h1s[cell][ci] > 0.0f ? s : 0.0f;
   }
   __syncthreads();
 
-  // conv1 bias and weights: dW1[co][t] = sum_cells dY1[cell][co] * z[y + t/5 - 1][2x + t%5 - 2].
-  if (tid < kC1) {
-    float s = 0.0f;
-    for (int cell = 0; cell < 7 * 13; ++cell) s += dY1[cell][tid];
-    g[kOffB1 + tid] = s;
-  }
+  // conv1 bias and weights: dW1[co][t] = sum_cells dY1[cell][co] * z[cell(y, x, t)].
   if (tid < kC1 * 15) {
     const int co = tid / 15, t = tid % 15;
     float s = 0.0f;
-    for (int cell = 0; cell < 7 * 13; ++cell) {
-      const int yy = y1o + cell / 13, xx = x1o + cell % 13;
-      if (yy < 0 || yy >= kH1 || xx < 0 || xx >= kW1) continue;
-      const int zy = yy + t / 5 - 1, zx = 2 * xx + t % 5 - 2;
-      if (zy < 0 || zy >= kRows || zx < 0 || zx >= kPooled) continue;
-      s += dY1[cell][co] * bf2f(z[(b * kRows + zy) * kPooled + zx]);
-    }
+    for (int cy = 0; cy < kR1H; ++cy)
+#pragma unroll
+      for (int cx = 0; cx < kR1W; ++cx)
+        s += dY1[cy * kR1W + cx][co] * zs[cy + t / 5][2 * cx + t % 5];
     g[kOffW1 + co * 15 + t] = s;
+  } else if (tid >= kBackThreads - kC1) {
+    const int co = tid - (kBackThreads - kC1);
+    float s = 0.0f;
+    for (int cell = 0; cell < kR1; ++cell) s += dY1[cell][co];
+    g[kOffB1 + co] = s;
   }
 }
 
-// grad[p] = sum over b in ascending order of gpart[b][p].
+// grad[p] = sum over b of gpart[b][p]: 64 parameters per workgroup, each of
+// its four waves sums a quarter of the blocks in ascending order with 16 loads
+// in flight, then the quarters are added in order (one thread per parameter
+// with a load at a time took 62 us at 256 blocks, 6 us now).
 __global__ void __launch_bounds__(256)
     reduce_grad_kernel(const float* __restrict__ gpart, int B, float* __restrict__ grad) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= kNumParams) return;
+  __shared__ float part[4][64];
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const int p = blockIdx.x * 64 + lane;
+  const int per = (B + 3) / 4, b1 = min(B, (wave + 1) * per);
   float s = 0.0f;
-  for (int b = 0; b < B; ++b) s += gpart[(long)b * kNumParams + p];
-  grad[p] = s;
+  if (p < kNumParams) {
+    int b = wave * per;
+    for (; b + 16 <= b1; b += 16) {
+      float v[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = gpart[(long)(b + i) * kNumParams + p];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s += v[i];
+    }
+    for (; b < b1; ++b) s += gpart[(long)b * kNumParams + p];
+  }
+  part[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && p < kNumParams)
+    grad[p] = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
 }
 
 __global__ void __launch_bounds__(256)
@@ -575,9 +606,9 @@ hipError_t launch_gradient(const Weights& w, const unsigned short* z, const floa
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(loss_kernel, dim3(1), dim3(256), 0, stream, logits, labels, B, pos_weight,
                      dz, loss);
-  hipLaunchKernelGGL(backward_kernel, dim3(B), dim3(256), 0, stream, z, a.h1, a.h2, a.h3, argmax,
+  hipLaunchKernelGGL(backward_kernel, dim3(B), dim3(kBackThreads), 0, stream, z, a.h1, a.h2, a.h3, argmax,
                      dz, w.params, w.w2b, w.w3b, gpart);
-  hipLaunchKernelGGL(reduce_grad_kernel, dim3((kNumParams + 255) / 256), dim3(256), 0, stream,
+  hipLaunchKernelGGL(reduce_grad_kernel, dim3((kNumParams + 63) / 64), dim3(256), 0, stream,
                      gpart, B, grad);
   return hipGetLastError();
 }
