@@ -419,7 +419,7 @@ sc_status sc_batch_copy_hits(const sc_batch* b, int instance, sc_hit* hits, size
  * one, the column sums, statistics, network and tile lists on another, the
  * merges on the third. Runs of up to 8 consecutive instances of one shape
  * share one launch per step (their network runs over all their blocks at
- * once, in buffers the batch allocates: 448 KiB per block of the longest
+ * once, in buffers the batch allocates: 64 KiB per block of the longest
  * run) and one tree launch; a run's front runs beside the previous run's
  * tree. pn must outlive the batch; its weights are read at every run.
  * sc_batch_info reports 0 graph nodes for it. */

@@ -1291,8 +1291,6 @@ void batch_release(sc_batch* b) {
   (void)hipHostFree(b->h_stats);
   (void)hipHostFree(b->h_gate);
   (void)hipFree(b->net_z);
-  (void)hipFree(b->net_a.h1);
-  (void)hipFree(b->net_a.h2);
   (void)hipFree(b->net_a.h3);
   (void)hipFree(b->net_logits);
   for (hipEvent_t ev : b->gate_events)
@@ -1807,8 +1805,8 @@ sc_status batch_create(const sc_instance* instances, int count, const sc_tuning*
         break;
       }
     }
-    // The network's buffers for the blocks of the longest run (448 KiB per
-    // block: tiles and three activation maps, BF16).
+    // The network's buffers for the blocks of the longest run (64 KiB per
+    // block: tiles and the last activation map, BF16; the others stay on chip).
     for (size_t a = 0, len = 0; a < b->inst.size(); a += len) {
       len = set_run(b, a);
       const long blocks =
@@ -1820,8 +1818,6 @@ sc_status batch_create(const sc_instance* instances, int count, const sc_tuning*
       void** p;
       size_t bytes;
     } bufs[] = {{(void**)&b->net_z, B * sc::pn::kRows * sc::pn::kPooled * 2},
-                {(void**)&b->net_a.h1, B * sc::pn::kActElems1 * 2},
-                {(void**)&b->net_a.h2, B * sc::pn::kActElems2 * 2},
                 {(void**)&b->net_a.h3, B * sc::pn::kActElems3 * 2},
                 {(void**)&b->net_logits, B * sizeof(float)}};
     for (auto& buf : bufs) {

@@ -37,10 +37,11 @@ constexpr long kActElems3 = (long)kH3 * kW3 * kC3;
 struct Weights {
   float* params = nullptr;          // FP32 master copy, kNumParams
   unsigned short* w1b = nullptr;    // [16][16]
-  unsigned short* w2b = nullptr;    // [32][15][16]
-  unsigned short* w3b = nullptr;    // [32][15][32]
+  unsigned short* w2b = nullptr;    // [32][15][16], as matrix-core operands
+  unsigned short* w3b = nullptr;    // [32][15][32], as matrix-core operands
 };
 
+// h1 and h2 may be null for a forward pass whose activations are not kept.
 struct Acts {
   unsigned short* h1 = nullptr;  // [B][16][512][16]
   unsigned short* h2 = nullptr;  // [B][8][256][32]

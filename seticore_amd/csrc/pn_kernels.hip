@@ -51,6 +51,29 @@ __device__ __forceinline__ float bf2f(unsigned short h) {
   return __uint_as_float((unsigned)h << 16);
 }
 
+// Where the BF16 copy of weight (co, tap t, ci) of a 3x5 convolution with CIN
+// input channels lies: in the order of the matrix-core operands, so that a
+// wave's operand is one 512-byte load (as rows of an output channel it touched
+// 16 cache lines, which bound the forward pass).
+template <int CIN>
+__device__ __forceinline__ int weight_index(int co, int t, int ci) {
+  return ((((co / 16) * 15 + t) * (CIN / 16) + ci / 16) * 64 + co % 16 + 16 * (ci % 16 / 4)) * 4 +
+         ci % 4;
+}
+
+// Four ReLU outputs to BF16 (v_cvt_pk_bf16_f32, round to nearest even as f2bf).
+__device__ __forceinline__ bf16x4 relu_bf16(const f32x4& acc, const float (&bias)[4]) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  const bf2 lo = __builtin_convertvector(
+      (f32x2{fmaxf(acc[0] + bias[0], 0.0f), fmaxf(acc[1] + bias[1], 0.0f)}), bf2);
+  const bf2 hi = __builtin_convertvector(
+      (f32x2{fmaxf(acc[2] + bias[2], 0.0f), fmaxf(acc[3] + bias[3], 0.0f)}), bf2);
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(bf16x4,
+                            (u32x2{__builtin_bit_cast(unsigned, lo), __builtin_bit_cast(unsigned, hi)}));
+}
+
 // ---------------------------------------------------------------------------
 // Pooling: z[blk][t][j] from the 4 channels 4096*blk + 4j .. +3 of row t.
 template <typename In>
@@ -98,121 +121,178 @@ __global__ void __launch_bounds__(256)
 }
 
 // ---------------------------------------------------------------------------
-// Convolution forward on the matrix cores. One wave per (64 output positions
-// along a row, output row, block). Lane layout of v_mfma_f32_16x16x16_bf16:
-// A[row][k] sits in lane row + 16*(k/4), element k%4; B[k][col] in lane
-// col + 16*(k/4), element k%4; D[row][col] in lane col + 16*(row/4), element
-// row%4. The product is formed transposed, D[channel][position] =
-// W[channel][k] * X[k][position], so each lane ends with 4 consecutive
-// channels of one position: one 8-byte store per lane and channel tile.
-// ROWS output rows per workgroup (blockIdx.y * ROWS ..), one after the other,
-// so the weights held in registers are loaded once for all of them.
-template <int CIN, int COUT, int SH, int SW, int ROWS>
-__global__ void __launch_bounds__(64)
-    conv_fwd_kernel(const unsigned short* __restrict__ in, int HI, int WI,
-                    const unsigned short* __restrict__ wb, const float* __restrict__ bias,
-                    unsigned short* __restrict__ out, int HO, int WO) {
-  constexpr int NT = COUT / 16;
-  constexpr int KS = CIN >= 16 ? CIN / 16 : 1;
-  constexpr int TAPS = CIN >= 16 ? 15 : 1;  // CIN == 1: one K step holds all 15 taps
-  constexpr int KROW = CIN >= 16 ? 15 * CIN : 16;  // weights per output channel
-  const int lane = threadIdx.x;
+// The three convolutions of a column tile in one workgroup, on the matrix
+// cores, with the activations passed through LDS.
+//
+// Lane layout of v_mfma_f32_16x16x16_bf16: A[row][k] sits in lane
+// row + 16*(k/4), element k%4; B[k][col] in lane col + 16*(k/4), element k%4;
+// D[row][col] in lane col + 16*(row/4), element row%4. The products are formed
+// transposed, D[channel][position] = W[channel][k] * X[k][position], so each
+// lane ends with 4 consecutive channels of one position: one 8-byte store.
+//
+// A workgroup takes kTile3 = 16 columns of h3 of one block: 35 columns of h2
+// and 80 of h1 (73 needed, in whole groups of 16 so that a group lies in one
+// row), halo included, 72 KB of LDS, two workgroups (16 waves) per CU. Columns
+// outside the maps and the row above them are zero in LDS, so the products
+// need no bounds tests. A stride-2 convolution reads every second column, so
+// columns are stored split by parity, and each group of four channels (a
+// lane's share of an operand) is a plane of its own: 16 lanes read 128
+// consecutive bytes, and the planes of a 32-lane half lie 32 banks apart. (With
+// a position's channels together, two thirds of the LDS cycles were bank
+// conflicts: 74 / 529 us at 256 / 2048 blocks.) conv2 takes positions 16 at a time across row ends. Each sum runs
+// over (tap, channel) in the order of the separate convolutions this replaces,
+// so logits are bit-identical to theirs.
+//
+// Separate kernels wrote and re-read every activation through memory and
+// gathered their operands from L1/L2: 108 / 868 us for 256 / 2048 blocks, with
+// the head; 60 / 479 us now, 15 instead of 46 for one. What bounds this one is
+// vector work around the products (conv1 above all: an operand's taps, bias,
+// ReLU, rounding and addresses for one product per 16 positions) and, with the
+// activations kept, writing 416 KB per block. h1, h2 may be null (not kept).
+constexpr int kTile3 = 16;
+constexpr int kCols2 = 2 * kTile3 + 3, kCols1 = (4 * kTile3 + 9 + 15) / 16 * 16;
+constexpr int kHalf2 = (kCols2 + 1) / 2, kHalf1 = kCols1 / 2;  // per column parity
+constexpr int kPitchZ = 2 * kCols1 + 4;
+constexpr int kPlane1 = (kH1 + 1) * 2 * kHalf1, kPlane2 = (kH2 + 1) * 2 * kHalf2 + 12;
+static_assert(kPlane1 * 2 % 64 == 32 && kPlane2 * 2 % 64 == 32, "planes half the banks apart");
+constexpr int kForwardThreads = 512;
+constexpr int kForwardWaves = kForwardThreads / 64;
+
+__global__ void __launch_bounds__(kForwardThreads, 4)
+    forward_kernel(const unsigned short* __restrict__ z, const unsigned short* __restrict__ w1b,
+                   const unsigned short* __restrict__ w2b, const unsigned short* __restrict__ w3b,
+                   const float* __restrict__ params, unsigned short* __restrict__ h1,
+                   unsigned short* __restrict__ h2, unsigned short* __restrict__ h3) {
+  __shared__ __attribute__((aligned(16))) bf16x4 h1s[4][kPlane1];
+  __shared__ __attribute__((aligned(16))) bf16x4 h2s[2][4][kPlane2];
+  // z is done with when h2 is first written.
+  unsigned short* zs = (unsigned short*)h2s;
+  static_assert((kRows + 2) * kPitchZ * 2 <= sizeof(h2s), "z fits");
+  static_assert(sizeof(h1s) + sizeof(h2s) <= 64 * 1024, "LDS of a workgroup");
+  constexpr int kTiles = kW3 / kTile3;
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
   const int r = lane % 16, g = lane / 16;
-  const int wo0 = blockIdx.x * 64;
-  const long b = blockIdx.z;
+  const int a3 = blockIdx.x % kTiles * kTile3;  // first column in h3
+  const int x2o = 2 * a3 - 2, x1o = 4 * a3 - 6, zo = 8 * a3 - 14;
+  const long b = blockIdx.x / kTiles;
 
-  bf16x4 bw[TAPS][KS][NT];
-#pragma unroll
-  for (int t = 0; t < TAPS; ++t)
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const unsigned short* w = wb + (long)(n * 16 + r) * KROW +
-                                  (CIN >= 16 ? t * CIN + s * 16 + 4 * g : 4 * g);
-        bw[t][s][n] = *(const bf16x4*)w;
-      }
+  // z rows -1 .. 16 (zo is even and the map 1024 wide: pairs of columns lie
+  // inside or outside together); the zero rows above h1 and h2.
+  for (int y = wave; y < kRows + 2; y += kForwardWaves) {
+    const unsigned* row = (const unsigned*)(z + (b * kRows + y - 1) * kPooled + zo);
+    for (int c = lane; c < kPitchZ / 2; c += 64) {
+      const int x = zo + 2 * c;
+      const bool ok = y >= 1 && y <= kRows && x >= 0 && x < kPooled;
+      ((unsigned*)zs)[y * (kPitchZ / 2) + c] = ok ? row[c] : 0u;
+    }
+  }
+  for (int e = tid; e < 4 * 2 * kHalf1; e += kForwardThreads)
+    h1s[e / (2 * kHalf1)][e % (2 * kHalf1)] = bf16x4{0, 0, 0, 0};
 
-  float bsv[NT][4];
+  const bf16x4 w1 = *(const bf16x4*)(w1b + r * 16 + 4 * g);
+  float bias1[4];
 #pragma unroll
-  for (int n = 0; n < NT; ++n)
+  for (int i = 0; i < 4; ++i) bias1[i] = params[kOffB1 + 4 * g + i];
+  // conv2: this wave's 16 output channels.
+  const int n = wave % 2;
+  bf16x4 w2[15];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) bsv[n][i] = bias[n * 16 + 4 * g + i];
+  for (int t = 0; t < 15; ++t)
+    w2[t] = ((const bf16x4*)w2b)[(n * 15 + t) * 64 + lane];
+  __syncthreads();
 
-  for (int ho = blockIdx.y * ROWS; ho < min(HO, (int)(blockIdx.y + 1) * ROWS); ++ho) {
-  f32x4 acc[4][NT];
+  // conv1: position (y, c) reads z rows y .. y+2, columns 2c .. 2c+4; this
+  // lane's four taps are 4g .. 4g+3 (15 does not exist). Two rows per wave.
+  int tap[4];
 #pragma unroll
-  for (int m = 0; m < 4; ++m)
+  for (int i = 0; i < 4; ++i) {
+    const int k = min(4 * g + i, 14);
+    tap[i] = k / 5 * kPitchZ + k % 5 + 2 * r;
+  }
+  static_assert(kH1 == 2 * kForwardWaves, "conv1 rows");
 #pragma unroll
-    for (int n = 0; n < NT; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  if constexpr (CIN == 1) {
+  for (int yy = 0; yy < 2; ++yy) {
+    const int y = 2 * wave + yy;
+    const unsigned short* zrow = zs + y * kPitchZ;
+    bf16x4* dst = h1s[g] + ((y + 1) * 2 + (r & 1)) * kHalf1 + (r >> 1);
+    unsigned short* keep = h1 ? h1 + ((b * kH1 + y) * kW1 + x1o) * kC1 : nullptr;
+    // All products of the row first, then the stores.
+    bf16x4 v[kCols1 / 16];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const int pos = wo0 + 16 * m + r;
+    for (int u = 0; u < kCols1 / 16; ++u) {
       bf16x4 a;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int k = 4 * g + i;
-        unsigned short v = 0;
-        if (k < 15) {
-          const int hi = ho * SH + k / 5 - 1;
-          const int wi = pos * SW + k % 5 - 2;
-          if (hi >= 0 && hi < HI && wi >= 0 && wi < WI) v = in[(b * HI + hi) * WI + wi];
-        }
-        a[i] = (short)v;
-      }
-#pragma unroll
-      for (int n = 0; n < NT; ++n)
-        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bw[0][0][n], a, acc[m][n], 0, 0, 0);
+      for (int i = 0; i < 4; ++i) a[i] = (short)zrow[tap[i] + 32 * u];
+      if (g == 3) a[3] = 0;
+      const f32x4 acc =
+          __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w1, a, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      v[u] = relu_bf16(acc, bias1);
+      const int x = x1o + 16 * u + r;
+      if (x < 0 || x >= kW1) v[u] = bf16x4{0, 0, 0, 0};
     }
-  } else {
-    // Every operand of the row first (32-bit offsets within the block's
-    // input; taps outside the input read offset 0 and are zeroed), then the
-    // products in the same (position tile, tap, K step, channel tile) order.
-    const unsigned short* blk_in = in + b * HI * WI * CIN;
-    bf16x4 a[4][15][KS];
+#pragma unroll
+    for (int u = 0; u < kCols1 / 16; ++u) dst[8 * u] = v[u];
+    if (keep) {
+#pragma unroll
+      for (int u = 0; u < kCols1 / 16; ++u) {
+        const int c = 16 * u + r;
+        if (c >= 6 && c < 6 + 4 * kTile3) *(bf16x4*)(keep + c * kC1 + 4 * g) = v[u];
+      }
+    }
+  }
+  __syncthreads();
+
+  // conv2: position (y, c) reads h1 rows 2y .. 2y+2 (row 0 is the zero row),
+  // columns 2c .. 2c+4. Waves of one channel half take every fourth group.
+  for (int e = tid; e < 8 * 2 * kHalf2; e += kForwardThreads)
+    h2s[e / (8 * kHalf2)][e / (2 * kHalf2) % 4][e % (2 * kHalf2)] = bf16x4{0, 0, 0, 0};
+  float bias2[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) bias2[i] = params[kOffB2 + n * 16 + 4 * g + i];
+  unsigned short* keep2 = h2 ? h2 + b * kH2 * kW2 * kC2 : nullptr;
+  for (int u = wave / 2; u < (kH2 * kCols2 + 15) / 16; u += kForwardWaves / 2) {
+    const int p = 16 * u + r, pc = min(p, kH2 * kCols2 - 1);
+    const int y = pc / kCols2, c = pc % kCols2, x = x2o + c;
+    const bf16x4* src = h1s[g] + 2 * y * 2 * kHalf1 + c;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < 15; ++t) {
-      const int hi = ho * SH + t / 5 - 1;
-      const bool row_ok = hi >= 0 && hi < HI;
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const int wi = (wo0 + 16 * m + r) * SW + t % 5 - 2;
-        const bool ok = row_ok && wi >= 0 && wi < WI;
-        const int off = ok ? (hi * WI + wi) * CIN + 4 * g : 0;
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-          const bf16x4 v = *(const bf16x4*)(blk_in + off + s * 16);
-          a[m][t][s] = ok ? v : bf16x4{0, 0, 0, 0};
-        }
-      }
+      const int ty = t / 5, tx = t % 5;
+      const bf16x4 a = src[(ty * 2 + (tx & 1)) * kHalf1 + (tx >> 1)];
+      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w2[t], a, acc, 0, 0, 0);
     }
-#pragma unroll
-    for (int m = 0; m < 4; ++m)
-#pragma unroll
-      for (int t = 0; t < 15; ++t)
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-#pragma unroll
-          for (int n = 0; n < NT; ++n)
-            acc[m][n] =
-                __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bw[t][s][n], a[m][t][s], acc[m][n], 0, 0, 0);
-  }
-
-#pragma unroll
-  for (int n = 0; n < NT; ++n) {
-    const int ch0 = n * 16 + 4 * g;
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const int pos = wo0 + 16 * m + r;
-      bf16x4 v;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = (short)f2bf(fmaxf(acc[m][n][i] + bsv[n][i], 0.0f));
-      *(bf16x4*)(out + ((b * HO + ho) * WO + pos) * COUT + ch0) = v;
+    bf16x4 v = relu_bf16(acc, bias2);
+    if (x < 0 || x >= kW2) v = bf16x4{0, 0, 0, 0};
+    if (p < kH2 * kCols2) {
+      h2s[n][g][((y + 1) * 2 + (c & 1)) * kHalf2 + (c >> 1)] = v;
+      if (keep2 && c >= 2 && c < 2 + 2 * kTile3)
+        *(bf16x4*)(keep2 + (y * kW2 + x) * kC2 + n * 16 + 4 * g) = v;
     }
   }
+  // conv3: one (row, channel half) per wave.
+  static_assert(kForwardWaves == 2 * kH3, "conv3 units");
+  const int y3 = wave / 2;
+  bf16x4 w3[15][2];
+#pragma unroll
+  for (int t = 0; t < 15; ++t)
+#pragma unroll
+    for (int s = 0; s < 2; ++s) w3[t][s] = ((const bf16x4*)w3b)[((n * 15 + t) * 2 + s) * 64 + lane];
+  float bias3[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) bias3[i] = params[kOffB3 + n * 16 + 4 * g + i];
+  __syncthreads();
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < 15; ++t) {
+    const int ty = t / 5, tx = t % 5;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const bf16x4 a =
+          h2s[s][g][((2 * y3 + ty) * 2 + (tx & 1)) * kHalf2 + r + (tx >> 1)];
+      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w3[t][s], a, acc, 0, 0, 0);
+    }
   }
+  *(bf16x4*)(h3 + ((b * kH3 + y3) * kW3 + a3 + r) * kC3 + n * 16 + 4 * g) = relu_bf16(acc, bias3);
 }
 
 // Head: logit[b] = max over positions of (bh + sum_c h3[pos][c] * wh[c]);
@@ -290,7 +370,7 @@ __global__ void __launch_bounds__(256)
 // conv2's weights - is first brought into LDS, zero outside the maps, so the
 // sums below are free of bounds tests and of memory latency: at 256 blocks
 // (one workgroup per CU) 127 us with global loads inside the sums on 256
-// threads, 21 us now.
+// threads, 26 us now.
 constexpr int kBackThreads = 512;
 constexpr int kR1H = 7, kR1W = 13, kR1 = kR1H * kR1W;  // receptive field in h1
 constexpr int kRZH = kR1H + 2, kRZW = 2 * kR1W + 3;    // and in z
@@ -298,8 +378,7 @@ __global__ void __launch_bounds__(kBackThreads)
     backward_kernel(const unsigned short* __restrict__ z, const unsigned short* __restrict__ h1,
                     const unsigned short* __restrict__ h2, const unsigned short* __restrict__ h3,
                     const int* __restrict__ argmax, const float* __restrict__ dz,
-                    const float* __restrict__ params, const unsigned short* __restrict__ w2b,
-                    const unsigned short* __restrict__ w3b, float* __restrict__ gpart) {
+                    const float* __restrict__ params, float* __restrict__ gpart) {
   const long b = blockIdx.x;
   const int tid = threadIdx.x;
   float* g = gpart + b * (long)kNumParams;
@@ -335,8 +414,9 @@ __global__ void __launch_bounds__(kBackThreads)
     const bool ok = zy >= 0 && zy < kRows && zx >= 0 && zx < kPooled;
     zs[tid / kRZW][tid % kRZW] = ok ? bf2f(z[(b * kRows + zy) * kPooled + zx]) : 0.0f;
   }
-  for (int e = tid; e < kC2 * 15 * kC1 / 2; e += kBackThreads)
-    ((unsigned*)w2s)[e] = ((const unsigned*)w2b)[e];
+  // The BF16 weights the forward pass used, rounded again from the master copy
+  // (whose order suits these sums).
+  for (int e = tid; e < kC2 * 15 * kC1; e += kBackThreads) w2s[e] = f2bf(params[kOffW2 + e]);
 
   // Head and conv3 bias.
   if (tid < kC3) {
@@ -358,7 +438,7 @@ __global__ void __launch_bounds__(kBackThreads)
     const int ci = tid % kC2, t = tid / kC2;
     float s = 0.0f;
 #pragma unroll
-    for (int co = 0; co < kC3; ++co) s += dY3[co] * bf2f(w3b[(co * 15 + t) * kC2 + ci]);
+    for (int co = 0; co < kC3; ++co) s += dY3[co] * bf2f(f2bf(params[kOffW3 + (co * 15 + t) * kC2 + ci]));
     dY2[t][ci] = h2s[t][ci] > 0.0f ? s : 0.0f;
   }
   __syncthreads();
@@ -461,7 +541,7 @@ __global__ void __launch_bounds__(256)
 }
 
 // BF16 copies of the convolution weights in the matrix-core layouts:
-// w1b[co][16] (tap 15 = 0), w2b[co][t][ci], w3b[co][t][ci].
+// w1b[co][16] (tap 15 = 0), w2b and w3b by weight_index.
 __global__ void __launch_bounds__(256)
     pack_kernel(const float* __restrict__ params, unsigned short* __restrict__ w1b,
                 unsigned short* __restrict__ w2b, unsigned short* __restrict__ w3b) {
@@ -470,8 +550,10 @@ __global__ void __launch_bounds__(256)
     const int co = i / 16, k = i % 16;
     w1b[i] = k < 15 ? f2bf(params[kOffW1 + co * 15 + k]) : 0;
   }
-  if (i < kC2 * 15 * kC1) w2b[i] = f2bf(params[kOffW2 + i]);
-  if (i < kC3 * 15 * kC2) w3b[i] = f2bf(params[kOffW3 + i]);
+  if (i < kC2 * 15 * kC1)
+    w2b[weight_index<kC1>(i / (15 * kC1), i / kC1 % 15, i % kC1)] = f2bf(params[kOffW2 + i]);
+  if (i < kC3 * 15 * kC2)
+    w3b[weight_index<kC2>(i / (15 * kC2), i / kC2 % 15, i % kC2)] = f2bf(params[kOffW3 + i]);
 }
 
 // ---------------------------------------------------------------------------
@@ -584,17 +666,8 @@ hipError_t launch_pool_set(const FrontSet& fs, int n, int dtype, long stride, in
 
 hipError_t launch_forward(const Weights& w, const unsigned short* z, int B, Acts& a,
                           float* logits, int* argmax, hipStream_t stream) {
-  // Rows per workgroup: 4 / 4 / 2 (grid.y 4 / 2 / 2). Measured forward at
-  // 256 / 2048 blocks: all rows of conv2 and conv3 in one workgroup and a row
-  // per workgroup for conv1, 125 / 866 us; these, 108 / 865 us (the
-  // workgroups load their weights a few times more, the blocks' rows spread
-  // over more workgroups).
-  hipLaunchKernelGGL((conv_fwd_kernel<1, kC1, 1, 2, 4>), dim3(kW1 / 64, kH1 / 4, B), dim3(64), 0,
-                     stream, z, kRows, kPooled, w.w1b, w.params + kOffB1, a.h1, kH1, kW1);
-  hipLaunchKernelGGL((conv_fwd_kernel<kC1, kC2, 2, 2, 4>), dim3(kW2 / 64, kH2 / 4, B), dim3(64),
-                     0, stream, a.h1, kH1, kW1, w.w2b, w.params + kOffB2, a.h2, kH2, kW2);
-  hipLaunchKernelGGL((conv_fwd_kernel<kC2, kC3, 2, 2, 2>), dim3(kW3 / 64, kH3 / 2, B), dim3(64),
-                     0, stream, a.h2, kH2, kW2, w.w3b, w.params + kOffB3, a.h3, kH3, kW3);
+  hipLaunchKernelGGL(forward_kernel, dim3(kW3 / kTile3 * B), dim3(kForwardThreads), 0, stream, z,
+                     w.w1b, w.w2b, w.w3b, w.params, a.h1, a.h2, a.h3);
   hipLaunchKernelGGL(head_kernel, dim3(B), dim3(256), 0, stream, a.h3, w.params, logits, argmax);
   return hipGetLastError();
 }
@@ -607,7 +680,7 @@ hipError_t launch_gradient(const Weights& w, const unsigned short* z, const floa
   hipLaunchKernelGGL(loss_kernel, dim3(1), dim3(256), 0, stream, logits, labels, B, pos_weight,
                      dz, loss);
   hipLaunchKernelGGL(backward_kernel, dim3(B), dim3(kBackThreads), 0, stream, z, a.h1, a.h2, a.h3, argmax,
-                     dz, w.params, w.w2b, w.w3b, gpart);
+                     dz, w.params, gpart);
   hipLaunchKernelGGL(reduce_grad_kernel, dim3((kNumParams + 63) / 64), dim3(256), 0, stream,
                      gpart, B, grad);
   return hipGetLastError();
