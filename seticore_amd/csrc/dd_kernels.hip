@@ -648,20 +648,20 @@ __device__ __forceinline__ void staged_load(const In* __restrict__ x, long strid
   const long g_lo = b >= 0 ? base : base + 15L * b;
   const long g_hi = b >= 0 ? base + 15L * b : base;
   if (g_lo >= 0 && g_hi + kWave * C <= N) {
-    const In* src = x + (long)(16 * k) * stride + base + lane * C;
+    const In* src = x + (long)(16 * k) * stride + base;  // uniform
     const long step = stride + b;
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
       if constexpr (sizeof(In) == 4) {
         typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-        const f4u w = *(const f4u*)src;
+        const f4u w = *(const f4u*)(src + lane * C);
         v[t][0] = w.x;
         v[t][1] = w.y;
         v[t][2] = w.z;
         v[t][3] = w.w;
       } else {
 #pragma unroll
-        for (int j = 0; j < C; ++j) v[t][j] = to_f32<In>(src[j]);
+        for (int j = 0; j < C; ++j) v[t][j] = to_f32<In>(src[lane * C + j]);
       }
       src += step;
     }
@@ -805,9 +805,13 @@ __device__ __forceinline__ void staged_group(const In* __restrict__ x, long stri
                                              Best<Staged<M>::C, BK>& best) {
   using St = Staged<M>;
   constexpr int Q0 = G_IDX * St::QG;
-  const int wave = threadIdx.x / kWave;
-  // (Double-buffering the rows of the next time block measured slower: the
-  // extra registers halve the waves per SIMD.)
+  // The wave index as a scalar: the rows' addresses are then scalar too, and a
+  // row costs one load with a per-lane offset (two 64-bit vector additions and
+  // 55 more registers at M = 4 otherwise): 50 -> 64 x 300001 in FP16, 66 drift
+  // blocks, 0.86 -> 0.70 ms; 256 x 2^20 18.4 -> 17.9 ms. (Loading the next time
+  // block's rows during the upper levels measured slower, 19.5 ms: what is left
+  // there is L2 bandwidth, 22 of the 27 TB/s that loads alone reach.)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   for (int k = wave; k < M; k += St::kWaves) {
     float v[16][St::C];
     staged_load<M, In>(x, stride, N, k, b, (long)c_w + (long)k * (16 * b + Q0), v);
@@ -922,7 +926,7 @@ __device__ __forceinline__ void staged_write_group(int grp, const In* __restrict
     }
   }
   constexpr int Q0 = G_IDX * St::QG;
-  const int wave = threadIdx.x / kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // as in staged_group
   const int lane = threadIdx.x % kWave;
   for (int k = wave; k < M; k += St::kWaves) {
     float v[16][C];
