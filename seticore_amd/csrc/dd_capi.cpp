@@ -61,22 +61,35 @@ int round_up_pow2(int n) {
 }  // namespace
 
 namespace sc {
-// Default fused-kernel shape per T_r: channels per lane and drift blocks per
-// LDS window.
-void default_tuning(int T, int* lanes, int* group, int* prefetch) {
-  // Measured on MI355X: at 16 x 2^20 (132 drift blocks) C=4, G=4 with chunked
-  // windows (mode 2) is the fastest T=16 shape; at 32..256 x 2^20 (66 blocks)
-  // the LDS-staged one-pass kernel with 8, 16, 8, 32 drift blocks per
-  // workgroup (1.29, 2.83, 5.46, 20.1 ms against 2.25 ms for fused32_kernel at
-  // 32 and 4.25, 7.83, 16.5, 33.7 ms for the two-pass search); at 256 with one
-  // workgroup per offset group (20.1 ms against 21.9 for one workgroup over
-  // all four groups at 8 blocks; at 128 the split is slower, 5.58 vs 5.46)
-  // and all drift blocks (up to 256) in one chunk: 18.1 vs 18.8 ms at 32.
-  // Below 16 time steps: 8 channels per lane, 16 drift blocks per window.
+// Default one-pass kernel shape: channels per lane, drift blocks per LDS window
+// (T <= 16) or per workgroup (staged), window mode or kernel selector.
+//
+// Measured on MI355X: at 16 x 2^20 (132 drift blocks) C=4, G=4 with chunked
+// windows (mode 2) is the fastest T=16 shape. At 32..256 the LDS-staged
+// one-pass kernel (1.01, 1.83, 4.7, 17.8 ms at 2^20 channels and 66 blocks); at
+// 256 with one workgroup per offset group (17.8 ms against 21.3 for one
+// workgroup over all four; at 128 the split is slower). Below 16 time steps:
+// 8 channels per lane, 16 drift blocks per window.
+void default_tuning(int T, int N, bool half_width, int* lanes, int* group, int* prefetch) {
   const bool staged = T >= 32 && T <= 256;
   *lanes = (T == 16 || staged) ? 4 : 8;
-  *group = T == 16 ? 4 : T == 64 ? 16 : T == 256 ? 256 : staged ? 8 : 16;
+  *group = T == 16 ? 4 : 16;
   *prefetch = T == 16 ? 2 : T == 32 ? sc::kStaged32 : T == 256 ? 1 : 0;
+  // Drift blocks per workgroup of the staged kernel. Long chunks save atomic
+  // merges and, at 256 time steps, let neighbouring tiles share rows in L2;
+  // they also leave fewer workgroups, so a narrow coarse channel ends with a
+  // nearly empty round of them. ms at 66 blocks for 4 / 8 / 16 (and 32 / 256)
+  // per workgroup:
+  //   32 x 2^16  .101 .115        32 x 2^20  1.09 1.02 1.01
+  //   64 x 2^16  .159 .168 .200   64 x 300001 .574 .561 .593  x 2^20 2.09 1.91 1.83
+  //   128 x 2^16 .403 .455        128 x 2^19 2.44 2.44        x 2^20 5.17 4.73 4.88
+  //   256 x 2^14 .49 .52 .60 .75 .97    256 x 2^16 1.55 1.51 1.50 1.66 1.65
+  //   256 x 2^18 5.28 5.10 4.92 5.00 4.72;  in 16 bits (half the L2 traffic to
+  //   save) 4.43 4.42 4.44 4.64 4.68, at 2^20 -- 17.0 -- 16.6 16.4.
+  if (T == 32) *group = N < (1 << 18) ? 4 : 8;
+  if (T == 64) *group = N < (1 << 18) ? 4 : N < 3 << 18 ? 8 : 16;
+  if (T == 128) *group = N < (1 << 19) ? 4 : 8;
+  if (T == 256) *group = N < (1 << 15) ? 4 : N < (half_width ? 3 << 18 : 1 << 17) ? 16 : 256;
 }
 
 }  // namespace sc
@@ -93,6 +106,7 @@ struct sc_dd {
   int lanes = 4;     // fused kernel: channels per lane
   int group = 8;     // fused kernel: drift blocks per LDS window
   int prefetch = 0;  // fused kernel: register prefetch of the next window
+  bool tuned = false;  // the shape is the caller's (sc_dd_set_tuning), not the default
   int device = 0;
 
   // Device state.
@@ -437,7 +451,7 @@ sc_status sc_dd_create(int num_timesteps, int num_channels, double foff_mhz, dou
   dd->drift_timesteps = rounded - 1;
   // dedoppler.cu:87
   dd->resolution = 1e6 * foff_mhz / (dd->drift_timesteps * tsamp_s);
-  sc::default_tuning(rounded, &dd->lanes, &dd->group, &dd->prefetch);
+  sc::default_tuning(rounded, num_channels, false, &dd->lanes, &dd->group, &dd->prefetch);
   if (rounded <= 256 && !sc::fused_supported(rounded, dd->lanes, dd->group, dd->prefetch)) {
     // Every T_r up to 256 has a compiled one-pass default; never fall back
     // to the staged global-memory path silently.
@@ -529,6 +543,7 @@ sc_status sc_dd_set_tuning(sc_dd* dd, int channels_per_lane, int drift_group, in
   dd->lanes = channels_per_lane;
   dd->group = drift_group;
   dd->prefetch = prefetch;
+  dd->tuned = true;
   dd->use_two_pass = false;
   return SC_OK;
 }
@@ -587,6 +602,9 @@ sc_status enqueue_path_sums(sc_dd* dd, const void* data, int dtype, long row_str
   SC_HIP(sc::launch_reset(dd->top_key, N, dd->stats_hist, stream), "reset");
   const bool one_pass = (T <= 16 || !dd->use_two_pass) &&
                         sc::fused_supported(T, dd->lanes, dd->group, dd->prefetch);
+  // The default shape follows the sample type too.
+  int lanes = dd->lanes, group = dd->group, prefetch = dd->prefetch;
+  if (!dd->tuned) sc::default_tuning(T, N, dtype != SC_F32, &lanes, &group, &prefetch);
   // The fork point is right after the reset, but the side stream's launches
   // are issued after the path sums': a captured graph submits its nodes in
   // the order they were captured, and with the statistics first the tree
@@ -595,8 +613,8 @@ sc_status enqueue_path_sums(sc_dd* dd, const void* data, int dtype, long row_str
   if (overlap_stats) SC_HIP(hipEventRecord(dd->ev_fork, stream), "fork");
   if (dd->timing) SC_HIP(hipEventRecord(dd->ev_start, stream), "timing event");
   if (one_pass) {
-    SC_HIP(sc::launch_fused_tree_top(data, dtype, row_stride, T, N, r.bmin, nblocks, dd->lanes,
-                                     dd->group, dd->prefetch, dd->top_key,
+    SC_HIP(sc::launch_fused_tree_top(data, dtype, row_stride, T, N, r.bmin, nblocks, lanes,
+                                     group, prefetch, dd->top_key,
                                      overlap_stats ? nullptr : dd->colsum, stream, nullptr,
                                      nullptr, device_tail && block_key_search(dd)),
            "fused tree");

@@ -33,9 +33,10 @@ inline DriftRange drift_range_of(double resolution, int drift_timesteps, double 
 sc_hit make_hit(const sc_meta* meta, int index, int drift_steps, double drift_rate, float snr,
                 int beam, int coarse_channel, int num_timesteps, float power);
 
-// Default one-pass kernel shape for T_r (channels per lane, drift blocks per
-// LDS window or workgroup, window mode / kernel selector), as measured best.
-void default_tuning(int T, int* lanes, int* group, int* prefetch);
+// Default one-pass kernel shape for T_r time steps, N channels and the sample
+// width (channels per lane, drift blocks per LDS window or workgroup, window
+// mode / kernel selector), as measured best.
+void default_tuning(int T, int N, bool half_width, int* lanes, int* group, int* prefetch);
 
 // Per-channel search state: the bits of an FP64 key whose value orders
 // (top path sum, -code) lexicographically - the float sum widened to double

@@ -136,7 +136,7 @@ extern "C" sc_status sc_dd_search_static(int num_timesteps, int rounded_timestep
   const int nblocks = r.bmax - r.bmin + 1;
   if ((long)nblocks * T > 0x1FFFFFFFL) return fail(SC_ERR_UNSUPPORTED, "drift range too large");
   int lanes = 0, group = 0, prefetch = 0;
-  sc::default_tuning(T, &lanes, &group, &prefetch);
+  sc::default_tuning(T, N, dtype != SC_F32, &lanes, &group, &prefetch);
   if (!sc::fused_supported(T, lanes, group, prefetch))
     return fail(SC_ERR_UNSUPPORTED, "no compiled default kernel shape for this T_r");
   const bool block_keys = T <= 16 || sc::staged_shape(T, lanes, group, prefetch);
