@@ -118,8 +118,6 @@ struct sc_dd {
   void* stats_scratch = nullptr;
   unsigned* stats_hist = nullptr;  // level-1 and level-2 histograms
   float* stats_out = nullptr;  // {median, std, mean, count}
-  int4* cand = nullptr;        // per-window candidates (+ one slot: the statistics)
-  size_t cand_capacity = 0;
   float* tree_a = nullptr;     // T_r*N scratch for the staged path and tree API
   float* tree_b = nullptr;
   // Two-pass search (T_r = 32..256): scratch of pass_blocks * T_r * pass_pitch
@@ -214,7 +212,6 @@ void release(sc_dd* dd) {
   (void)hipFree(dd->stats_scratch);
   (void)hipFree(dd->stats_hist);
   (void)hipFree(dd->stats_out);
-  (void)hipFree(dd->cand);
   (void)hipFree(dd->tree_a);
   (void)hipFree(dd->tree_b);
   (void)hipFree(dd->pass_scratch);
@@ -474,15 +471,13 @@ sc_status sc_dd_create(int num_timesteps, int num_channels, double foff_mhz, dou
     s = dev_alloc(dd, (void**)&dd->stats_hist, sc::device_stats_hist_bytes(), "stats hist");
   if (s == SC_OK) s = dev_alloc(dd, (void**)&dd->stats_out, 4 * sizeof(float), "stats");
   // At most one candidate per window and window >= 2 (max_drift > 0).
-  dd->cand_capacity = (N + 1) / 2 + 1;
-  if (s == SC_OK)
-    s = dev_alloc(dd, (void**)&dd->cand, dd->cand_capacity * sizeof(int4), "candidates");
+  const size_t cand_capacity = (N + 1) / 2 + 1;
   if (s == SC_OK) s = host_alloc((void**)&dd->h_colsum, N * sizeof(float), "column sums");
   if (s == SC_OK) s = host_alloc((void**)&dd->h_top_sum, N * sizeof(float), "top sums");
   if (s == SC_OK) s = host_alloc((void**)&dd->h_top_blk, N * sizeof(int), "top blocks");
   if (s == SC_OK) s = host_alloc((void**)&dd->h_top_off, N * sizeof(int), "top offsets");
   if (s == SC_OK)
-    s = host_alloc((void**)&dd->h_cand, dd->cand_capacity * sizeof(int4), "candidates");
+    s = host_alloc((void**)&dd->h_cand, cand_capacity * sizeof(int4), "candidates");
   if (s == SC_OK) s = host_alloc((void**)&dd->h_stats, 4 * sizeof(float), "stats");
   if (sc::two_pass_supported(rounded, dd->pass_group)) {
     // The one-pass kernels (default up to 256 time steps) need no scratch;
@@ -661,38 +656,40 @@ sc_status enqueue_path_sums(sc_dd* dd, const void* data, int dtype, long row_str
   return SC_OK;
 }
 
-// Device statistics, window merge (with the candidates' offsets after a
-// block-key search of `data`) and the copies of the per-window candidates.
+// One channel's part of a tail launch on handle dd: candidates and statistics
+// go straight to host memory.
+void tail_entry(sc::TailSet* ts, int i, const sc_dd* dd, const void* data, const DriftRange& r,
+                double snr_threshold, int4* h_cand, float* h_stats) {
+  ts->x[i] = data;
+  ts->key[i] = dd->top_key;
+  ts->stats[i] = dd->stats_out;
+  ts->top_sum[i] = dd->top_sum;
+  ts->top_blk[i] = dd->top_blk;
+  ts->top_off[i] = dd->top_off;
+  ts->cand[i] = h_cand;
+  ts->stats_copy[i] = h_stats;
+  ts->window[i] = r.window;
+  ts->snr[i] = snr_threshold;
+}
+
+// Device statistics, then the window merge with the candidates' offsets after
+// a block-key search of `data`.
 sc_status enqueue_device_tail(sc_dd* dd, const DriftRange& r, double snr_threshold,
                               const void* data, int dtype, long row_stride, hipStream_t stream,
-                              int4* h_cand = nullptr, float* h_stats = nullptr,
-                              bool stats_done = false, bool gated = false) {
-  // The handle's own buffers (a single search): the statistics ride in the
-  // candidates' copy, at h_cand[nwin] (one copy instead of two).
-  const bool own = !h_cand && !h_stats;
-  if (!h_cand) h_cand = dd->h_cand;
-  if (!h_stats) h_stats = dd->h_stats;
+                              int4* h_cand, float* h_stats, bool stats_done = false,
+                              bool gated = false, int* h_gate = nullptr) {
   const int T = dd->rounded, N = dd->num_channels;
   if (!stats_done)
     SC_HIP(sc::launch_device_stats(dd->colsum, N, dd->stats_scratch, dd->stats_hist,
                                    dd->stats_out, stream),
            "device stats");
-  const bool bk = block_key_search(dd);
-  SC_HIP(sc::launch_window_merge(dd->top_key, N, T, r.bmin, r.window, snr_threshold,
-                                 dd->stats_out, dd->top_sum, dd->top_blk, dd->top_off, dd->cand,
-                                 bk, stream, gated, own),
+  sc::TailSet ts = {};
+  tail_entry(&ts, 0, dd, data, r, snr_threshold, h_cand, h_stats);
+  ts.gate[0] = dd->gate_count;
+  ts.gate_copy[0] = h_gate;
+  SC_HIP(sc::launch_window_merge_set(ts, 1, dtype, row_stride, N, T, r.bmin, block_key_search(dd),
+                                     stream, gated),
          "window merge");
-  const int nwin = (int)(((long)N + r.window - 1) / r.window);
-  if (bk)
-    SC_HIP(sc::launch_candidate_offsets(data, dtype, row_stride, T, N, nwin, dd->cand,
-                                        dd->top_off, stream),
-           "candidate offsets");
-  SC_HIP(hipMemcpyAsync(h_cand, dd->cand, (nwin + (own ? 1 : 0)) * sizeof(int4),
-                        hipMemcpyDeviceToHost, stream),
-         "copy candidates");
-  if (!own)
-    SC_HIP(hipMemcpyAsync(h_stats, dd->stats_out, 4 * sizeof(float), hipMemcpyDeviceToHost,
-                          stream), "copy stats");
   return SC_OK;
 }
 
@@ -718,7 +715,7 @@ sc_status search_graph(sc_dd* dd, const void* data, int dtype, long row_stride,
       enqueue_path_sums(dd, data, dtype, row_stride, r, dd->capture_stream, true, true);
   if (s == SC_OK)
     s = enqueue_device_tail(dd, r, snr_threshold, data, dtype, row_stride, dd->capture_stream,
-                            nullptr, nullptr, true);
+                            dd->h_cand, dd->h_stats, true);
   hipGraph_t graph = nullptr;
   hipError_t e = hipStreamEndCapture(dd->capture_stream, &graph);
   if (s != SC_OK) {
@@ -939,15 +936,12 @@ sc_status sc_dd_search(sc_dd* dd, const void* data, int dtype, int rounded_times
     } else {
       s = enqueue_path_sums(dd, data, dtype, row_stride, r, stream, true, true);
       if (s == SC_OK)
-        s = enqueue_device_tail(dd, r, snr_threshold, data, dtype, row_stride, stream, nullptr,
-                                nullptr, true);
+        s = enqueue_device_tail(dd, r, snr_threshold, data, dtype, row_stride, stream,
+                                dd->h_cand, dd->h_stats, true);
       if (s != SC_OK) return s;
     }
     SC_HIP(hipStreamSynchronize(stream), "search");
-    // The statistics came with the candidates (enqueue_device_tail).
-    const int nwin = (int)(((long)N + r.window - 1) / r.window);
-    s = device_hits(dd, r, meta, beam, coarse_channel, min_drift, nullptr,
-                    (const float*)(dd->h_cand + nwin));
+    s = device_hits(dd, r, meta, beam, coarse_channel, min_drift);
     if (s != SC_OK) return s;
   }
   if (dd->timing) {
@@ -993,21 +987,10 @@ sc_status sc_dd_search_proposed(sc_dd* dd, sc_pn* pn, const void* data, int dtyp
   s = enqueue_gate_front(dd, pn, data, dtype, row_stride, logit_threshold, stream);
   if (s == SC_OK) s = enqueue_gated_tree(dd, data, dtype, row_stride, r, stream);
   if (s != SC_OK) return s;
-  SC_HIP(sc::launch_window_merge(dd->top_key, N, T, r.bmin, r.window, snr_threshold,
-                                 dd->stats_out, dd->top_sum, dd->top_blk, dd->top_off, dd->cand,
-                                 true, stream, true),
-         "window merge");
-  const int nwin = (int)(((long)N + r.window - 1) / r.window);
-  SC_HIP(sc::launch_candidate_offsets(data, dtype, row_stride, T, N, nwin, dd->cand, dd->top_off,
-                                      stream),
-         "candidate offsets");
+  s = enqueue_device_tail(dd, r, snr_threshold, data, dtype, row_stride, stream, dd->h_cand,
+                          dd->h_stats, true, true, dd->h_gate);
+  if (s != SC_OK) return s;
   if (dd->timing) SC_HIP(hipEventRecord(dd->ev_stop, stream), "timing event");
-  SC_HIP(hipMemcpyAsync(dd->h_cand, dd->cand, nwin * sizeof(int4), hipMemcpyDeviceToHost,
-                        stream), "copy candidates");
-  SC_HIP(hipMemcpyAsync(dd->h_stats, dd->stats_out, 4 * sizeof(float), hipMemcpyDeviceToHost,
-                        stream), "copy stats");
-  SC_HIP(hipMemcpyAsync(dd->h_gate, dd->gate_count, 2 * sizeof(int), hipMemcpyDeviceToHost,
-                        stream), "copy tile count");
   SC_HIP(hipStreamSynchronize(stream), "gated search");
   s = device_hits(dd, r, meta, beam, coarse_channel, min_drift);
   if (s != SC_OK) return s;
@@ -1449,52 +1432,20 @@ sc_status enqueue_gated(sc_batch* b, hipStream_t stream) {
     s = issue_front(r + 1, (long)a);
     if (s != SC_OK) break;
     SC_HIP(hipStreamWaitEvent(Q, sums_ev(a), 0), "wait tree");
-    if (e - a > 1) {
-      // The run's window merges (channels without a key skipped) and
-      // candidate offsets, one launch each.
-      sc::TailSet ts = {};
-      for (size_t j = a; j < e; ++j) {
-        const sc_batch::Instance& bj = b->inst[j];
-        sc_dd* dj = b->shapes[bj.shape];
-        ts.x[j - a] = bj.in.data;
-        ts.key[j - a] = dj->top_key;
-        ts.stats[j - a] = dj->stats_out;
-        ts.top_sum[j - a] = dj->top_sum;
-        ts.top_blk[j - a] = dj->top_blk;
-        ts.top_off[j - a] = dj->top_off;
-        ts.cand[j - a] = dj->cand;
-        ts.window[j - a] = bj.r.window;
-        ts.snr[j - a] = bj.in.snr_threshold;
-      }
-      SC_HIP(sc::launch_window_merge_set(ts, (int)(e - a), d0->num_channels, 16, b0.r.bmin, Q,
-                                         true),
-             "window merges");
-      SC_HIP(sc::launch_candidate_offsets_set(ts, (int)(e - a), b0.in.dtype, b0.in.row_stride,
-                                              d0->num_channels, Q),
-             "candidate offsets");
+    // The run's window merges (channels without a key skipped), one launch.
+    sc::TailSet ts = {};
+    for (size_t j = a; j < e; ++j) {
+      const sc_batch::Instance& bj = b->inst[j];
+      const sc_dd* dj = b->shapes[bj.shape];
+      tail_entry(&ts, (int)(j - a), dj, bj.in.data, bj.r, bj.in.snr_threshold,
+                 b->h_cand + bj.cand_offset, b->h_stats + 4 * j);
+      ts.gate[j - a] = dj->gate_count;
+      ts.gate_copy[j - a] = b->h_gate + 2 * j;
     }
-    for (size_t i = a; i < e; ++i) {
-      sc_batch::Instance& bi = b->inst[i];
-      sc_dd* dd = b->shapes[bi.shape];
-      if (e - a > 1) {
-        const int nwin = (int)(((long)dd->num_channels + bi.r.window - 1) / bi.r.window);
-        SC_HIP(hipMemcpyAsync(b->h_cand + bi.cand_offset, dd->cand, nwin * sizeof(int4),
-                              hipMemcpyDeviceToHost, Q),
-               "copy candidates");
-        SC_HIP(hipMemcpyAsync(b->h_stats + 4 * i, dd->stats_out, 4 * sizeof(float),
-                              hipMemcpyDeviceToHost, Q),
-               "copy stats");
-      } else {
-        s = enqueue_device_tail(dd, bi.r, bi.in.snr_threshold, bi.in.data, bi.in.dtype,
-                                bi.in.row_stride, Q, b->h_cand + bi.cand_offset,
-                                b->h_stats + 4 * i, true, true);
-      }
-      if (s != SC_OK) break;
-      SC_HIP(hipMemcpyAsync(b->h_gate + 2 * i, dd->gate_count, 2 * sizeof(int),
-                            hipMemcpyDeviceToHost, Q),
-             "copy tile count");
-      SC_HIP(hipEventRecord(tail_ev(i), Q), "tail done");
-    }
+    SC_HIP(sc::launch_window_merge_set(ts, (int)(e - a), b0.in.dtype, b0.in.row_stride,
+                                       d0->num_channels, 16, b0.r.bmin, true, Q, true),
+           "window merges");
+    for (size_t i = a; i < e; ++i) SC_HIP(hipEventRecord(tail_ev(i), Q), "tail done");
   }
   if (s != SC_OK) return s;
   // Each run's tails follow its tree, and its front precedes it: the tails'
@@ -1543,42 +1494,23 @@ sc_status enqueue_plain(sc_batch* b, hipStream_t M, hipStream_t Q, NewEvent&& ne
       const sc_batch::Instance& b0 = b->inst[i];
       const int N = b->shapes[b0.shape]->num_channels;
       e = sc::launch_device_stats_set(fs, (int)n, N, Q);
-      // Window merges and candidate offsets (block keys), one launch each.
+      // Window merges (block keys), one launch.
       sc::TailSet ts = {};
       for (size_t j = 0; j < n; ++j) {
         const sc_batch::Instance& bj = b->inst[i + j];
-        sc_dd* dj = b->shapes[bj.shape];
-        ts.x[j] = bj.in.data;
-        ts.key[j] = dj->top_key;
-        ts.stats[j] = dj->stats_out;
-        ts.top_sum[j] = dj->top_sum;
-        ts.top_blk[j] = dj->top_blk;
-        ts.top_off[j] = dj->top_off;
-        ts.cand[j] = dj->cand;
-        ts.window[j] = bj.r.window;
-        ts.snr[j] = bj.in.snr_threshold;
+        tail_entry(&ts, (int)j, b->shapes[bj.shape], bj.in.data, bj.r, bj.in.snr_threshold,
+                   b->h_cand + bj.cand_offset, b->h_stats + 4 * (i + j));
       }
-      if (e == hipSuccess) e = sc::launch_window_merge_set(ts, (int)n, N, 16, b0.r.bmin, Q);
       if (e == hipSuccess)
-        e = sc::launch_candidate_offsets_set(ts, (int)n, b0.in.dtype, b0.in.row_stride, N, Q);
+        e = sc::launch_window_merge_set(ts, (int)n, b0.in.dtype, b0.in.row_stride, N, 16,
+                                        b0.r.bmin, true, Q);
     }
     for (size_t j = i; j < i + n && s == SC_OK && e == hipSuccess; ++j) {
       sc_batch::Instance& bj = b->inst[j];
-      sc_dd* dj = b->shapes[bj.shape];
-      if (n > 1) {
-        // The candidates and statistics to the host (merged above).
-        const int nwin = (int)(((long)dj->num_channels + bj.r.window - 1) / bj.r.window);
-        e = hipMemcpyAsync(b->h_cand + bj.cand_offset, dj->cand, nwin * sizeof(int4),
-                           hipMemcpyDeviceToHost, Q);
-        if (e == hipSuccess)
-          e = hipMemcpyAsync(b->h_stats + 4 * j, dj->stats_out, 4 * sizeof(float),
-                             hipMemcpyDeviceToHost, Q);
-        if (e != hipSuccess) break;
-      } else {
-        s = enqueue_device_tail(dj, bj.r, bj.in.snr_threshold, bj.in.data, bj.in.dtype,
-                                bj.in.row_stride, Q, b->h_cand + bj.cand_offset,
+      if (n == 1)
+        s = enqueue_device_tail(b->shapes[bj.shape], bj.r, bj.in.snr_threshold, bj.in.data,
+                                bj.in.dtype, bj.in.row_stride, Q, b->h_cand + bj.cand_offset,
                                 b->h_stats + 4 * j);
-      }
       if (s != SC_OK) break;
       hipEvent_t tail = nullptr;
       e = new_event(&tail);

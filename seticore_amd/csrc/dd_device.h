@@ -73,8 +73,7 @@ __device__ __forceinline__ float key_sum(unsigned long long k) {
 // (sum bits, ~block) with block = drift_block - min_drift_block, for sums > 0
 // only. Their unsigned order is (sum, -block), so a 64-bit atomic max keeps
 // the largest sum and, among equal sums, the lowest block; the window merge
-// reads the sums, and candidate_offsets_kernel finds the offset of each
-// window's candidate.
+// reads the sums and finds the offset of each window's candidate.
 __device__ __forceinline__ unsigned long long block_key(float s, int block) {
   return ((unsigned long long)__float_as_uint(s) << 32) | (unsigned)~(unsigned)block;
 }
@@ -270,7 +269,7 @@ __device__ __forceinline__ bool block_interior(int c_w, int b, int N) {
 // only - a block replaces the best when its largest sum is strictly larger
 // (blocks come in ascending order), which is the reference's rule
 // (dedoppler.cu:40,49,214) up to the offset within the block; the offset of a
-// hit is recovered afterwards (candidate_offsets_kernel). About a third less
+// hit is recovered afterwards (window_merge_kernel). About a third less
 // VALU work per path sum.
 template <int C, bool BK>
 struct Best;

@@ -54,7 +54,7 @@ typedef unsigned long long top_key_t;
 // tiles tile_list[0 .. *tile_count) are searched (tiles of
 // fused_tile_width(T, C) channels). With block_keys (T_r <= 16 and the staged
 // kernel; fused32_kernel ignores it) the keys are block keys: (sum bits << 32) | ~(drift block -
-// bmin), the offset left to launch_candidate_offsets after the window merge.
+// bmin), the offset left to the window merge.
 hipError_t launch_fused_tree_top(const void* x, int dtype, long stride, int T, int N,
                                  int bmin, int nblocks, int C, int G, int P,
                                  top_key_t* top_key, float* colsum, hipStream_t stream,
@@ -94,10 +94,9 @@ hipError_t launch_front_set_stats(const FrontSet& fs, int n, int dtype, long str
 // stats_out), each pass one launch for all of them.
 hipError_t launch_device_stats_set(const FrontSet& fs, int n, int N, hipStream_t stream);
 
-// Per-channel buffers and parameters of a batch run's tail (16 time steps,
-// block keys): launch_window_merge and launch_candidate_offsets for n
-// channels of one width and drift-block range, one launch each (grid.y =
-// channel).
+// Per-channel buffers and parameters of a search's tail, for one channel or a
+// batch run's of one width and drift-block range. cand and the copies may be
+// host-visible memory.
 struct TailSet {
   const void* x[kMaxFusedSet];
   const top_key_t* key[kMaxFusedSet];
@@ -106,13 +105,21 @@ struct TailSet {
   int* top_blk[kMaxFusedSet];
   int* top_off[kMaxFusedSet];
   int4* cand[kMaxFusedSet];
+  float* stats_copy[kMaxFusedSet];  // may be null: receives the four statistics
+  const int* gate[kMaxFusedSet];    // {tiles, blocks flagged} of a gated search,
+  int* gate_copy[kMaxFusedSet];     // copied here unless null
   int window[kMaxFusedSet];
   double snr[kMaxFusedSet];
 };
-hipError_t launch_window_merge_set(const TailSet& ts, int n, int N, int T, int bmin,
-                                   hipStream_t stream, bool skip_empty = false);
-hipError_t launch_candidate_offsets_set(const TailSet& ts, int n, int dtype, long stride, int N,
-                                        hipStream_t stream);
+// Per-window merge (dedoppler.cu:273-303) for n channels (grid.y = channel),
+// fused with unpacking the keys into the three top arrays.
+// cand[c][i] = {index or -1, sum bits, drift block, path offset} for window i.
+// With block keys the offsets of the candidates are found from the input
+// (T <= 256 rows); other channels' unpacked offsets are -1. skip_empty:
+// channels without a key neither form nor suppress a candidate.
+hipError_t launch_window_merge_set(const TailSet& ts, int n, int dtype, long stride, int N, int T,
+                                   int bmin, bool block_keys, hipStream_t stream,
+                                   bool skip_empty = false);
 
 // Whether launch_fused16_set has a kernel for (T, C, G, P) (the default
 // 16-time-step shape).
@@ -184,22 +191,6 @@ size_t device_stats_hist_bytes();
 // stats_out = {median, std, mean}.
 hipError_t launch_device_stats(const float* colsum, int N, void* scratch, unsigned* hist,
                                float* stats_out, hipStream_t stream);
-
-// Per-window merge (dedoppler.cu:273-303) fused with unpacking the keys into
-// the three top arrays. cand_out[i] = {index or -1, sum bits, drift block,
-// path offset} for window i. With block keys the offsets (unpacked and in
-// the candidates) are -1 until launch_candidate_offsets fills the candidates'.
-// With stats_slot, cand_out[number of windows] also receives the four
-// statistics (float bits), for one copy to the host.
-hipError_t launch_window_merge(const top_key_t* key, int N, int T, int bmin, int window,
-                               double snr_threshold, const float* stats, float* top_sum,
-                               int* top_blk, int* top_off, int4* cand_out, bool block_keys,
-                               hipStream_t stream, bool skip_empty = false,
-                               bool stats_slot = false);
-// After a block-key merge (T_r <= 16): each candidate's path offset, from the
-// input of the search.
-hipError_t launch_candidate_offsets(const void* x, int dtype, long stride, int T, int N,
-                                    int nwin, int4* cand, int* top_off, hipStream_t stream);
 
 // queries[i] = {channel, drift block, path offset, -}: the path sum's float bits
 // into .w (host-visible memory; T up to 4096 rows, samples outside the coarse

@@ -89,68 +89,23 @@ __device__ float path_sum_exact(const In* __restrict__ x, long stride, int N, in
   }
 }
 
-// Offset of each window's candidate after a block-key search: the candidate
-// record holds its channel, sum and drift block; the offset is the first
-// (lowest) one whose path sum in that block equals the sum (the reference
-// keeps the first of equal sums, dedoppler.cu:49). Also completes the
-// unpacked offset of that channel. min(T, 64) lanes per window, one offset
-// each per round.
+// Offset of a window's candidate after a block-key search, by the whole
+// workgroup (one offset per thread, T <= 256 of them): the first (lowest) one
+// whose path sum in the recorded block equals the recorded sum (the reference
+// keeps the first of equal sums, dedoppler.cu:49). -1: none does (the tree
+// kernels and this re-addition disagree on an addition order); the host
+// reports an error.
 template <int T, typename In>
-__device__ __forceinline__ void candidate_offsets_body(const In* __restrict__ x, long stride,
-                                                       int N, int nwin, int4* __restrict__ cand,
-                                                       int* __restrict__ top_off) {
-  constexpr int kLanes = T < kWave ? T : kWave;
-  constexpr int kPerWave = kWave / kLanes;
-  const int slot = threadIdx.x / kLanes;
-  const int lane = threadIdx.x % kLanes;
-  const int w = blockIdx.x * kPerWave + slot;
-  const unsigned long long group_mask = kLanes == kWave ? ~0ull : ((1ull << kLanes) - 1);
-  int4 r = make_int4(-1, 0, 0, 0);
-  int pmax = 0;
-  // A candidate whose top sum is the zero the search starts from (no positive
-  // path; only when the threshold is below zero) keeps the block and offset
-  // the merge read from the top arrays, as the reference reports them
-  // (dedoppler.cu:305-306).
-  bool empty = false;
-  if (w < nwin) {
-    r = cand[w];
-    empty = r.x >= 0 && r.y == 0;
-    if (r.x >= 0 && !empty) {
-      const int last0 = r.x + (T - 1) * r.z;
-      pmax = last0 < 0 ? 0 : min(T, N - last0);
-    }
-  }
-  int p_best = -1;
-  for (int p0 = 0; p0 < T; p0 += kLanes) {  // uniform trip count: every lane takes the ballot
-    const int p = p0 + lane;
-    const bool match =
-        p < pmax && path_sum_exact<T, In>(x, stride, N, r.z, p, r.x) == __int_as_float(r.y);
-    const unsigned long long mine = (__ballot(match) >> (slot * kLanes)) & group_mask;
-    if (p_best < 0 && mine) p_best = p0 + __ffsll((long long)mine) - 1;
-  }
-  if (lane == 0 && w < nwin && r.x >= 0 && !empty) {
-    // -1: no offset reproduces the recorded sum (the tree kernels and this
-    // re-addition disagree on an addition order); the host reports an error.
-    r.w = p_best;
-    cand[w] = r;
-    top_off[r.x] = r.w;
-  }
-}
-
-template <int T, typename In>
-__global__ void __launch_bounds__(kWave)
-    candidate_offsets_kernel(const In* __restrict__ x, long stride, int N, int nwin,
-                             int4* __restrict__ cand, int* __restrict__ top_off) {
-  candidate_offsets_body<T, In>(x, stride, N, nwin, cand, top_off);
-}
-
-// Several channels (grid.y = channel; each checks its own window count).
-template <int T, typename In>
-__global__ void __launch_bounds__(kWave) candidate_offsets_set_kernel(TailSet ts, long stride,
-                                                                      int N) {
-  const int c = blockIdx.y;
-  const int nwin = (int)(((long)N + ts.window[c] - 1) / ts.window[c]);
-  candidate_offsets_body<T, In>((const In*)ts.x[c], stride, N, nwin, ts.cand[c], ts.top_off[c]);
+__device__ __forceinline__ int candidate_offset(const In* __restrict__ x, long stride, int N,
+                                                int c, int b, float sum, int* shared_best) {
+  const int p = threadIdx.x;
+  const int last0 = c + (T - 1) * b;
+  const int pmax = last0 < 0 ? 0 : min(T, N - last0);
+  if (p == 0) *shared_best = T;
+  __syncthreads();
+  if (p < pmax && path_sum_exact<T, In>(x, stride, N, b, p, c) == sum) atomicMin(shared_best, p);
+  __syncthreads();
+  return *shared_best < T ? *shared_best : -1;
 }
 
 // Four consecutive channels of one output row (one 16-byte store at any 4-byte
@@ -1625,36 +1580,45 @@ __global__ void __launch_bounds__(kStatsThreads) stats_final_set_kernel(FrontSet
 }
 
 // ---------------------------------------------------------------------------
-// Window merge (dedoppler.cu:273-303), one workgroup per window, fused with the
-// unpacking of the keys into the reference's three top arrays (each
-// workgroup unpacks its own window; channels without a positive path keep
-// their previous block and offset, dedoppler.cu:205).
-__device__ __forceinline__ void window_merge_body(const top_key_t* __restrict__ key, int N, int T,
-                                                  int bmin, int window, double snr_threshold,
-                                                  const float* __restrict__ stats,
-                                                  float* __restrict__ top_sum,
-                                                  int* __restrict__ top_blk,
-                                                  int* __restrict__ top_off,
-                                                  int4* __restrict__ out, int flags) {
-  const bool block_keys = flags & 1;
+// Window merge (dedoppler.cu:273-303), one workgroup per window and channel
+// (grid.y), fused with the unpacking of the keys into the reference's three top
+// arrays (each workgroup unpacks its own window; channels without a positive
+// path keep their previous block and offset, dedoppler.cu:205), with the
+// candidate's path offset after a block-key search (T > 0), and with bringing
+// candidates, statistics and tile counts to the host: `cand` and the copies
+// may be host memory, so a search's tail is one launch (merge, offsets and
+// one or two copies were a launch each: 24 us of a 16 x 2^20 search). What it
+// takes is latency: the window's keys are read twice by up to 1024 threads.
+// The tail of a 16 x 2^20 search takes 10 us for 18 (and two launches less);
+// at 256 x 2^20, with 32 windows of 33396 channels, 44 for 145.
+template <int T, typename In>
+__global__ void __launch_bounds__(1024)
+    window_merge_kernel(TailSet ts, long stride, int N, int rows, int bmin, int flags) {
+  const int ch = blockIdx.y;
+  const int window = ts.window[ch];
+  const int wid = blockIdx.x;
+  if (wid >= (int)(((long)N + window - 1) / window)) return;
+  const top_key_t* __restrict__ key = ts.key[ch];
+  const float* __restrict__ stats = ts.stats[ch];
+  float* __restrict__ top_sum = ts.top_sum[ch];
+  int* __restrict__ top_blk = ts.top_blk[ch];
+  int* __restrict__ top_off = ts.top_off[ch];
+  int4* __restrict__ out = ts.cand[ch];
+  constexpr bool block_keys = T > 0;
   // Gated search: a channel without a key (not searched, or no positive
   // path) neither forms nor suppresses a candidate.
   const float empty = (flags & 2) ? -INFINITY : 0.0f;
-  __shared__ float sv[4];
-  __shared__ int si[4];
-  __shared__ int any_larger;
-  const int wid = blockIdx.x;
+  __shared__ float sv[1024 / kWave];
+  __shared__ int si[1024 / kWave];
+  __shared__ int any_larger, best_offset;
   const int tid = threadIdx.x;
-  // flags & 4: the statistics also go to out[number of windows], so that one
-  // copy brings both to the host.
-  if ((flags & 4) && wid == 0 && tid == 0)
-    out[gridDim.x] = make_int4(__float_as_int(stats[0]), __float_as_int(stats[1]),
-                               __float_as_int(stats[2]), __float_as_int(stats[3]));
+  if (wid == 0 && tid < 4 && ts.stats_copy[ch]) ts.stats_copy[ch][tid] = stats[tid];
+  if (wid == 0 && tid < 2 && ts.gate_copy[ch]) ts.gate_copy[ch][tid] = ts.gate[ch][tid];
   const int lane = tid % kWave, wave = tid / kWave;
   const float median = stats[0];
   const float sd = stats[1];
   // float path_sum_threshold = snr_threshold * std_dev + median; (double math, no FMA)
-  const float thr = (float)__dadd_rn(__dmul_rn(snr_threshold, (double)sd), (double)median);
+  const float thr = (float)__dadd_rn(__dmul_rn(ts.snr[ch], (double)sd), (double)median);
   const long lo = (long)wid * window;
   const long hi = min(lo + (long)window, (long)N);
   float bv = thr;
@@ -1665,11 +1629,11 @@ __device__ __forceinline__ void window_merge_body(const top_key_t* __restrict__ 
     const float cv = k ? v : empty;
     if (k && block_keys) {
       top_blk[f] = (int)~(unsigned)k + bmin;
-      top_off[f] = -1;  // completed for candidates by candidate_offsets_kernel
+      top_off[f] = -1;  // completed for the candidate below
     } else if (k) {
       const unsigned code = (unsigned)(kCodeMask - (k & kCodeMask));
-      top_blk[f] = (int)(code / (unsigned)T) + bmin;
-      top_off[f] = (int)(code % (unsigned)T);
+      top_blk[f] = (int)(code / (unsigned)rows) + bmin;
+      top_off[f] = (int)(code % (unsigned)rows);
     }
     top_sum[f] = v;
     if (cv > bv) {
@@ -1694,7 +1658,7 @@ __device__ __forceinline__ void window_merge_body(const top_key_t* __restrict__ 
   __syncthreads();
   bv = sv[0];
   bi = si[0];
-  for (int w = 1; w < 4; ++w) {
+  for (int w = 1; w < (int)blockDim.x / kWave; ++w) {
     const float ov = sv[w];
     const int oi = si[w];
     if (oi >= 0 && (bi < 0 || ov > bv || (ov == bv && oi < bi))) {
@@ -1715,34 +1679,27 @@ __device__ __forceinline__ void window_merge_body(const top_key_t* __restrict__ 
   }
   if (larger) any_larger = 1;
   __syncthreads();
-  if (tid == 0) {
-    if (any_larger) {
-      out[wid] = make_int4(-1, 0, 0, 0);
-    } else {
-      // The candidate lies in this window, so this workgroup unpacked it.
-      out[wid] = make_int4(bi, __float_as_int(bv), top_blk[bi], top_off[bi]);
+  if (any_larger) {
+    if (tid == 0) out[wid] = make_int4(-1, 0, 0, 0);
+    return;
+  }
+  // The candidate lies in this window, so this workgroup unpacked it. One
+  // whose top sum is the zero the search starts from (no positive path; only
+  // when the threshold is below zero) keeps the block and offset of the top
+  // arrays, as the reference reports them (dedoppler.cu:305-306).
+  if constexpr (T > 0) {
+    const top_key_t k = key[bi];
+    if (__float_as_int(bv) != 0) {
+      const int off = candidate_offset<T, In>((const In*)ts.x[ch], stride, N, bi,
+                                              (int)~(unsigned)k + bmin, bv, &best_offset);
+      if (tid == 0) {
+        top_off[bi] = off;
+        out[wid] = make_int4(bi, __float_as_int(bv), (int)~(unsigned)k + bmin, off);
+      }
+      return;
     }
   }
-}
-
-__global__ void __launch_bounds__(256)
-    window_merge_kernel(const top_key_t* __restrict__ key, int N, int T, int bmin, int window,
-                        double snr_threshold, const float* __restrict__ stats,
-                        float* __restrict__ top_sum, int* __restrict__ top_blk,
-                        int* __restrict__ top_off, int4* __restrict__ out, int flags) {
-  window_merge_body(key, N, T, bmin, window, snr_threshold, stats, top_sum, top_blk, top_off, out,
-                    flags);
-}
-
-// Several channels' merges (grid.y = channel, grid.x = the most windows of
-// any of them).
-__global__ void __launch_bounds__(256)
-    window_merge_set_kernel(TailSet ts, int N, int T, int bmin, int flags) {
-  const int c = blockIdx.y;
-  const int nwin = (int)(((long)N + ts.window[c] - 1) / ts.window[c]);
-  if ((int)blockIdx.x >= nwin) return;
-  window_merge_body(ts.key[c], N, T, bmin, ts.window[c], ts.snr[c], ts.stats[c], ts.top_sum[c],
-                    ts.top_blk[c], ts.top_off[c], ts.cand[c], flags);
+  if (tid == 0) out[wid] = make_int4(bi, __float_as_int(bv), top_blk[bi], top_off[bi]);
 }
 
 // ---------------------------------------------------------------------------
@@ -2188,87 +2145,57 @@ hipError_t launch_fused_tree_top(const void* x, int dtype, long stride, int T, i
                         tile_list, tile_count, block_keys);
 }
 
-template <int T, typename In>
-hipError_t candidate_offsets_typed(const In* x, long stride, int N, int nwin, int4* cand,
-                                   int* top_off, hipStream_t stream) {
-  constexpr int per_wave = kWave / (T < kWave ? T : kWave);
-  hipLaunchKernelGGL((candidate_offsets_kernel<T, In>), dim3((nwin + per_wave - 1) / per_wave),
-                     dim3(kWave), 0, stream, x, stride, N, nwin, cand, top_off);
-  return hipGetLastError();
-}
-
+namespace {
 template <typename In>
-hipError_t candidate_offsets_dispatch(const In* x, long stride, int T, int N, int nwin,
-                                      int4* cand, int* top_off, hipStream_t stream) {
+hipError_t window_merge_dispatch(const TailSet& ts, dim3 grid, dim3 block, long stride, int T,
+                                 int N, int bmin, int flags, hipStream_t stream) {
   switch (T) {
-    case 2: return candidate_offsets_typed<2, In>(x, stride, N, nwin, cand, top_off, stream);
-    case 4: return candidate_offsets_typed<4, In>(x, stride, N, nwin, cand, top_off, stream);
-    case 8: return candidate_offsets_typed<8, In>(x, stride, N, nwin, cand, top_off, stream);
-    case 16: return candidate_offsets_typed<16, In>(x, stride, N, nwin, cand, top_off, stream);
-    case 32: return candidate_offsets_typed<32, In>(x, stride, N, nwin, cand, top_off, stream);
-    case 64: return candidate_offsets_typed<64, In>(x, stride, N, nwin, cand, top_off, stream);
-    case 128:
-      return candidate_offsets_typed<128, In>(x, stride, N, nwin, cand, top_off, stream);
-    case 256:
-      return candidate_offsets_typed<256, In>(x, stride, N, nwin, cand, top_off, stream);
+#define SC_MERGE_CASE(TT)                                                                       \
+  case TT:                                                                                      \
+    hipLaunchKernelGGL((window_merge_kernel<TT, In>), grid, block, 0, stream, ts, stride, N, T, \
+                       bmin, flags);                                                            \
+    return hipGetLastError();
+    SC_MERGE_CASE(2)
+    SC_MERGE_CASE(4)
+    SC_MERGE_CASE(8)
+    SC_MERGE_CASE(16)
+    SC_MERGE_CASE(32)
+    SC_MERGE_CASE(64)
+    SC_MERGE_CASE(128)
+    SC_MERGE_CASE(256)
+#undef SC_MERGE_CASE
   }
   return hipErrorInvalidValue;
 }
+}  // namespace
 
-hipError_t launch_window_merge_set(const TailSet& ts, int n, int N, int T, int bmin,
-                                   hipStream_t stream, bool skip_empty) {
+hipError_t launch_window_merge_set(const TailSet& ts, int n, int dtype, long stride, int N, int T,
+                                   int bmin, bool block_keys, hipStream_t stream,
+                                   bool skip_empty) {
   if (n < 1 || n > kMaxFusedSet) return hipErrorInvalidValue;
-  int nwin = 0;
+  int nwin = 0, widest = 0;
   for (int c = 0; c < n; ++c) {
     if (ts.window[c] <= 0) return hipErrorInvalidValue;
     nwin = std::max(nwin, (int)(((long)N + ts.window[c] - 1) / ts.window[c]));
+    widest = std::max(widest, std::min(ts.window[c], N));
   }
-  hipLaunchKernelGGL(window_merge_set_kernel, dim3(nwin, n), dim3(256), 0, stream, ts, N, T,
-                     bmin, 1 | (skip_empty ? 2 : 0));
-  return hipGetLastError();
-}
-
-hipError_t launch_candidate_offsets_set(const TailSet& ts, int n, int dtype, long stride, int N,
-                                        hipStream_t stream) {
-  if (n < 1 || n > kMaxFusedSet) return hipErrorInvalidValue;
-  int nwin = 0;
-  for (int c = 0; c < n; ++c) {
-    if (ts.window[c] <= 0) return hipErrorInvalidValue;
-    nwin = std::max(nwin, (int)(((long)N + ts.window[c] - 1) / ts.window[c]));
+  // Every thread takes one or two keys of a window up to 2048 channels wide;
+  // few, wide windows (many time steps) take more threads instead.
+  const dim3 grid(nwin, n), block(widest > 2048 ? 1024 : 256);
+  const int flags = skip_empty ? 2 : 0;
+  if (!block_keys) {
+    hipLaunchKernelGGL((window_merge_kernel<0, float>), grid, block, 0, stream, ts, stride, N, T,
+                       bmin, flags);
+    return hipGetLastError();
   }
-  constexpr int per_wave = kWave / 16;
-  const dim3 grid((nwin + per_wave - 1) / per_wave, n);
   switch (dtype) {
     case 0:
-      hipLaunchKernelGGL((candidate_offsets_set_kernel<16, float>), grid, dim3(kWave), 0, stream,
-                         ts, stride, N);
-      break;
+      return window_merge_dispatch<float>(ts, grid, block, stride, T, N, bmin, flags, stream);
     case 1:
-      hipLaunchKernelGGL((candidate_offsets_set_kernel<16, __half>), grid, dim3(kWave), 0, stream,
-                         ts, stride, N);
-      break;
+      return window_merge_dispatch<__half>(ts, grid, block, stride, T, N, bmin, flags, stream);
     case 2:
-      hipLaunchKernelGGL((candidate_offsets_set_kernel<16, __hip_bfloat16>), grid, dim3(kWave), 0,
-                         stream, ts, stride, N);
-      break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-
-hipError_t launch_candidate_offsets(const void* x, int dtype, long stride, int T, int N,
-                                    int nwin, int4* cand, int* top_off, hipStream_t stream) {
-  if (nwin <= 0) return hipSuccess;
-  switch (dtype) {
-    case 0:
-      return candidate_offsets_dispatch<float>((const float*)x, stride, T, N, nwin, cand,
-                                               top_off, stream);
-    case 1:
-      return candidate_offsets_dispatch<__half>((const __half*)x, stride, T, N, nwin, cand,
-                                                top_off, stream);
-    case 2:
-      return candidate_offsets_dispatch<__hip_bfloat16>((const __hip_bfloat16*)x, stride, T, N,
-                                                        nwin, cand, top_off, stream);
+      return window_merge_dispatch<__hip_bfloat16>(ts, grid, block, stride, T, N, bmin, flags,
+                                                   stream);
   }
   return hipErrorInvalidValue;
 }
@@ -2421,17 +2348,6 @@ hipError_t launch_device_stats_set(const FrontSet& fs, int n, int N, hipStream_t
   hipLaunchKernelGGL(stats_pass3_set_kernel, grid, block, 0, stream, fs, N);
   hipLaunchKernelGGL(stats_pass4_set_kernel, grid, block, 0, stream, fs, N);
   hipLaunchKernelGGL(stats_final_set_kernel, dim3(1, n), block, 0, stream, fs, N);
-  return hipGetLastError();
-}
-
-hipError_t launch_window_merge(const top_key_t* key, int N, int T, int bmin, int window,
-                               double snr_threshold, const float* stats, float* top_sum,
-                               int* top_blk, int* top_off, int4* cand_out, bool block_keys,
-                               hipStream_t stream, bool skip_empty, bool stats_slot) {
-  const int nwin = (int)(((long)N + window - 1) / window);
-  hipLaunchKernelGGL(window_merge_kernel, dim3(nwin), dim3(256), 0, stream, key, N, T, bmin,
-                     window, snr_threshold, stats, top_sum, top_blk, top_off, cand_out,
-                     (block_keys ? 1 : 0) | (skip_empty ? 2 : 0) | (stats_slot ? 4 : 0));
   return hipGetLastError();
 }
 

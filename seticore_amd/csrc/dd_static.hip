@@ -164,14 +164,19 @@ extern "C" sc_status sc_dd_search_static(int num_timesteps, int rounded_timestep
          "fused tree");
   SC_HIP(sc::launch_device_stats(colsum, N, stats_state, stats_hist, stats_out, stream),
          "device stats");
-  SC_HIP(sc::launch_window_merge(key, N, T, r.bmin, r.window, snr_threshold, stats_out, top_sum,
-                                 top_blk, top_off, cand, block_keys, stream),
+  sc::TailSet tail = {};
+  tail.x[0] = data;
+  tail.key[0] = key;
+  tail.stats[0] = stats_out;
+  tail.top_sum[0] = top_sum;
+  tail.top_blk[0] = top_blk;
+  tail.top_off[0] = top_off;
+  tail.cand[0] = cand;
+  tail.window[0] = r.window;
+  tail.snr[0] = snr_threshold;
+  SC_HIP(sc::launch_window_merge_set(tail, 1, dtype, row_stride, N, T, r.bmin, block_keys, stream),
          "window merge");
   const int nwin = (int)(((long)N + r.window - 1) / r.window);
-  if (block_keys)
-    SC_HIP(sc::launch_candidate_offsets(data, dtype, row_stride, T, N, nwin, cand, top_off,
-                                        stream),
-           "candidate offsets");
 
   // {median, std, mean, number of non-finite column sums}
   float stats[4];
