@@ -1556,16 +1556,19 @@ sc_status enqueue_plain(sc_batch* b, hipStream_t M, hipStream_t Q, NewEvent&& ne
       // dedoppler.cu:205 per channel, then the set launch (column sums
       // written by the workgroups that hold drift block 0).
       sc::FusedSet set = {};
-      for (size_t j = 0; j < n && e == hipSuccess; ++j) {
+      sc::FrontSet fs = {};
+      for (size_t j = 0; j < n; ++j) {
         sc_batch::Instance& bj = b->inst[i + j];
         sc_dd* dj = b->shapes[bj.shape];
-        e = sc::launch_reset(dj->top_key, dj->num_channels, dj->stats_hist, M);
+        fs.key[j] = dj->top_key;
+        fs.hist[j] = dj->stats_hist;
         set.x[j] = bj.in.data;
         set.key[j] = dj->top_key;
         set.colsum[j] = dj->colsum;
       }
       const sc_batch::Instance& b0 = b->inst[i];
       const sc_dd* d0 = b->shapes[b0.shape];
+      e = sc::launch_reset_set(fs, (int)n, d0->num_channels, M);
       if (e == hipSuccess && timers) e = hipEventRecord(timers->back().start, M);
       if (e == hipSuccess)
         e = sc::launch_fused16_set(set, (int)n, b0.in.dtype, b0.in.row_stride, 16,

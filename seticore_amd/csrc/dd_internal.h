@@ -86,6 +86,8 @@ struct FrontSet {
   int* list[kMaxFusedSet];
   int* count[kMaxFusedSet];  // {tiles listed, blocks flagged}
 };
+// launch_reset for n channels of one width (their key and hist), one launch.
+hipError_t launch_reset_set(const FrontSet& fs, int n, int N, hipStream_t stream);
 // launch_reset, launch_colsum and launch_device_stats for n channels of one
 // shape, each step one launch for all of them.
 hipError_t launch_front_set_stats(const FrontSet& fs, int n, int dtype, long stride, int T,

@@ -2316,11 +2316,16 @@ hipError_t launch_device_stats(const float* colsum, int N, void* scratch, unsign
   return hipGetLastError();
 }
 
-hipError_t launch_front_set_stats(const FrontSet& fs, int n, int dtype, long stride, int T,
-                                  int N, hipStream_t stream) {
+hipError_t launch_reset_set(const FrontSet& fs, int n, int N, hipStream_t stream) {
   if (n < 1 || n > kMaxFusedSet) return hipErrorInvalidValue;
   hipLaunchKernelGGL(reset_set_kernel, dim3(blocks_for(N, 256, 2048), n), dim3(256), 0, stream,
                      fs, (long)N, (long)stats_hist_words());
+  return hipGetLastError();
+}
+
+hipError_t launch_front_set_stats(const FrontSet& fs, int n, int dtype, long stride, int T,
+                                  int N, hipStream_t stream) {
+  if (launch_reset_set(fs, n, N, stream) != hipSuccess) return hipErrorInvalidValue;
   const dim3 cgrid((N + 255) / 256, n);
   switch (dtype) {
     case 0:
@@ -2342,11 +2347,14 @@ hipError_t launch_front_set_stats(const FrontSet& fs, int n, int dtype, long str
 
 hipError_t launch_device_stats_set(const FrontSet& fs, int n, int N, hipStream_t stream) {
   if (n < 1 || n > kMaxFusedSet) return hipErrorInvalidValue;
-  const dim3 grid(kStatsBlocks, n), block(kStatsThreads);
+  const dim3 block(kStatsThreads);
+  // The histograms' flushes are most of a counting pass over several channels:
+  // fewer workgroups per channel flush fewer bins.
+  const dim3 grid(std::max(32, kStatsBlocks / n), n);
   hipLaunchKernelGGL(stats_pass1_set_kernel, grid, block, 0, stream, fs, N);
   hipLaunchKernelGGL(stats_pass2_set_kernel, grid, block, 0, stream, fs, N);
   hipLaunchKernelGGL(stats_pass3_set_kernel, grid, block, 0, stream, fs, N);
-  hipLaunchKernelGGL(stats_pass4_set_kernel, grid, block, 0, stream, fs, N);
+  hipLaunchKernelGGL(stats_pass4_set_kernel, dim3(kStatsBlocks, n), block, 0, stream, fs, N);
   hipLaunchKernelGGL(stats_final_set_kernel, dim3(1, n), block, 0, stream, fs, N);
   return hipGetLastError();
 }
