@@ -540,6 +540,13 @@ struct Staged {
   // workgroups (12 waves) per CU. Measured: 168 VGPRs (one spilled) at M = 16
   // beat 197 at two waves; M = 4 keeps its 237 registers.
   static constexpr int kMinWaves = M <= 4 ? 2 : 3;
+  // The last lane whose row samples reach an output of time block k: R
+  // columns up to 4*kUsed for the group's last offset (k*(QG-1) columns on),
+  // and a level-16 path spans 15 channels more.
+  __device__ static constexpr int last_lane(int k) {
+    return (C * kUsed + k * (QG - 1) + 15 - 1) / C < kWave ? (C * kUsed + k * (QG - 1) + 15 - 1) / C
+                                                          : kWave - 1;
+  }
   static_assert(kOut <= TileShape<M, C>::kOut, "phase 2 tile");
   static_assert(kUsed <= kLevel16Lanes, "phase 1 writes every position read");
   static_assert(QG * M <= 64 && kGroups * QG == 16, "group shape");
@@ -605,18 +612,23 @@ __device__ __forceinline__ void staged_load(const In* __restrict__ x, long strid
   if (g_lo >= 0 && g_hi + kWave * C <= N) {
     const In* src = x + (long)(16 * k) * stride + base;  // uniform
     const long step = stride + b;
+    // Lanes past the columns this time block's outputs depend on read the
+    // last one's samples again (their own outputs are discarded): 9 % fewer
+    // bytes from L2 at M = 16, 17.6 -> 16.8 ms for 256 x 2^20 in float32 (no
+    // change where L2 does not bound: fewer time steps, 16-bit samples).
+    const int cl = min(lane, Staged<M>::last_lane(k)) * C;
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
       if constexpr (sizeof(In) == 4) {
         typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-        const f4u w = *(const f4u*)(src + lane * C);
+        const f4u w = *(const f4u*)(src + cl);
         v[t][0] = w.x;
         v[t][1] = w.y;
         v[t][2] = w.z;
         v[t][3] = w.w;
       } else {
 #pragma unroll
-        for (int j = 0; j < C; ++j) v[t][j] = to_f32<In>(src[lane * C + j]);
+        for (int j = 0; j < C; ++j) v[t][j] = to_f32<In>(src[cl + j]);
       }
       src += step;
     }
@@ -764,8 +776,8 @@ __device__ __forceinline__ void staged_group(const In* __restrict__ x, long stri
   // row costs one load with a per-lane offset (two 64-bit vector additions and
   // 55 more registers at M = 4 otherwise): 50 -> 64 x 300001 in FP16, 66 drift
   // blocks, 0.86 -> 0.70 ms; 256 x 2^20 18.4 -> 17.9 ms. (Loading the next time
-  // block's rows during the upper levels measured slower, 19.5 ms: what is left
-  // there is L2 bandwidth, 22 of the 27 TB/s that loads alone reach.)
+  // block's rows during the upper levels measured slower, 19.5 ms: what bounds
+  // it there is L2 bandwidth, 22 of the 27 TB/s that loads alone reach.)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   for (int k = wave; k < M; k += St::kWaves) {
     float v[16][St::C];
