@@ -1118,6 +1118,12 @@ __global__ void unpack_top_kernel(const top_key_t* __restrict__ key,
 // memory in every pass; 44 us now (12 + 18 + 5 + 6 + 4).
 
 constexpr int kStatsBlocks = 256;
+// Workgroups of a counting pass over one channel where it runs beside a tree or
+// over several channels at once: its cost is the flush of every workgroup's
+// non-zero bins and the slots taken from the tree. 16 x 2^20, 54 drift blocks:
+// 276 us a call with 256, 272 with 64, 267 with 32, 272 with 16. (Alone, in
+// normalize, 256 are as fast.)
+constexpr int kCountBlocks = 32;
 constexpr int kStatsThreads = 256;
 constexpr int kL1Bits = 13, kL2Bits = 10, kL3Bits = 9;
 constexpr int kL1 = 1 << kL1Bits, kL2 = 1 << kL2Bits, kL3 = 1 << kL3Bits;
@@ -2319,11 +2325,11 @@ size_t device_stats_hist_bytes() { return sizeof(unsigned) * stats_hist_words();
 hipError_t launch_device_stats(const float* colsum, int N, void* scratch, unsigned* hist,
                                float* stats_out, hipStream_t stream) {
   StatsState* st = (StatsState*)scratch;
-  const dim3 grid(kStatsBlocks), block(kStatsThreads);
+  const dim3 grid(kCountBlocks), block(kStatsThreads);
   hipLaunchKernelGGL(stats_pass1_kernel, grid, block, 0, stream, colsum, N, hist);
   hipLaunchKernelGGL(stats_pass2_kernel, grid, block, 0, stream, colsum, N, hist);
   hipLaunchKernelGGL(stats_pass3_kernel, grid, block, 0, stream, colsum, N, hist);
-  hipLaunchKernelGGL(stats_pass4_kernel, grid, block, 0, stream, colsum, N, hist, st);
+  hipLaunchKernelGGL(stats_pass4_kernel, dim3(kStatsBlocks), block, 0, stream, colsum, N, hist, st);
   hipLaunchKernelGGL(stats_final_kernel, dim3(1), block, 0, stream, st, N, hist, stats_out);
   return hipGetLastError();
 }
@@ -2360,9 +2366,7 @@ hipError_t launch_front_set_stats(const FrontSet& fs, int n, int dtype, long str
 hipError_t launch_device_stats_set(const FrontSet& fs, int n, int N, hipStream_t stream) {
   if (n < 1 || n > kMaxFusedSet) return hipErrorInvalidValue;
   const dim3 block(kStatsThreads);
-  // The histograms' flushes are most of a counting pass over several channels:
-  // fewer workgroups per channel flush fewer bins.
-  const dim3 grid(std::max(32, kStatsBlocks / n), n);
+  const dim3 grid(kCountBlocks, n);
   hipLaunchKernelGGL(stats_pass1_set_kernel, grid, block, 0, stream, fs, N);
   hipLaunchKernelGGL(stats_pass2_set_kernel, grid, block, 0, stream, fs, N);
   hipLaunchKernelGGL(stats_pass3_set_kernel, grid, block, 0, stream, fs, N);
