@@ -38,6 +38,27 @@ __device__ __forceinline__ float ord_val(unsigned k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k);
 }
 
+// Four consecutive samples at any element alignment, in one load.
+template <typename In>
+__device__ __forceinline__ void load4(const In* __restrict__ src, float (&v)[4]) {
+  if constexpr (sizeof(In) == 4) {
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+    const f4u w = *(const f4u*)src;
+    v[0] = w.x;
+    v[1] = w.y;
+    v[2] = w.z;
+    v[3] = w.w;
+  } else {
+    typedef unsigned u2u __attribute__((ext_vector_type(2), aligned(2)));
+    const u2u w = *(const u2u*)src;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const unsigned short bits = (unsigned short)((j < 2 ? w.x : w.y) >> (16 * (j & 1)));
+      v[j] = to_f32<In>(__builtin_bit_cast(In, bits));
+    }
+  }
+}
+
 // Level-L entry (tb, p) of drift block b's tree at start channel c, added in
 // the register tree's order: entry (2tb, p/2) at c plus entry (2tb+1, p/2) at
 // c + (p+1)/2 (tree_stage); level 1 is row tb at c + tb*b (the shear), 0
@@ -110,11 +131,16 @@ __device__ __forceinline__ int candidate_offset(const In* __restrict__ x, long s
 
 // Four consecutive channels of one output row (one 16-byte store at any 4-byte
 // alignment), cut at the last channel.
+template <bool STREAM = false>
 __device__ __forceinline__ void store_row4(float* __restrict__ row, int c, int N,
                                            const float (&v)[4]) {
   typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+  const f4u q = {v[0], v[1], v[2], v[3]};
   if (c + 4 <= N) {
-    *(f4u*)(row + c) = f4u{v[0], v[1], v[2], v[3]};
+    if constexpr (STREAM)
+      __builtin_nontemporal_store(q, (f4u*)(row + c));
+    else
+      *(f4u*)(row + c) = q;
   } else {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -619,13 +645,10 @@ __device__ __forceinline__ void staged_load(const In* __restrict__ x, long strid
     const int cl = min(lane, Staged<M>::last_lane(k)) * C;
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
+      // (The compiler joins the 16-bit samples into one 8-byte load; written
+      // as one, the unpacking scheduled 2 % slower at 64 time steps.)
       if constexpr (sizeof(In) == 4) {
-        typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-        const f4u w = *(const f4u*)(src + cl);
-        v[t][0] = w.x;
-        v[t][1] = w.y;
-        v[t][2] = w.z;
-        v[t][3] = w.w;
+        load4<In>(src + cl, v[t]);
       } else {
 #pragma unroll
         for (int j = 0; j < C; ++j) v[t][j] = to_f32<In>(src[cl + j]);
@@ -639,18 +662,7 @@ __device__ __forceinline__ void staged_load(const In* __restrict__ x, long strid
     const In* row = x + (long)(16 * k + t) * stride;
     const long g0 = base + (long)t * b;
     if (g0 >= 0 && g0 + kWave * C <= N) {
-      const In* src = row + g0 + lane * C;
-      if constexpr (sizeof(In) == 4) {
-        typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-        const f4u w = *(const f4u*)src;
-        v[t][0] = w.x;
-        v[t][1] = w.y;
-        v[t][2] = w.z;
-        v[t][3] = w.w;
-      } else {
-#pragma unroll
-        for (int j = 0; j < C; ++j) v[t][j] = to_f32<In>(src[j]);
-      }
+      load4<In>(row + g0 + lane * C, v[t]);
     } else {
 #pragma unroll
       for (int j = 0; j < C; ++j) {
@@ -878,17 +890,19 @@ __global__ void __launch_bounds__(kWave * Staged<M>::kWaves, Staged<M>::kMinWave
   }
 }
 
+constexpr long kLastLevelCache = 256L << 20;
+
 // One offset group of one drift block with its path sums written out: phase 1
 // as above, then each wave's offsets as rows q*M .. q*M + M-1 of out.
 template <int M, int G_IDX, typename In>
 __device__ __forceinline__ void staged_write_group(int grp, const In* __restrict__ x, long stride,
                                                    int N, int b, int c_w, lds_float* R,
-                                                   float* __restrict__ out) {
+                                                   float* __restrict__ out, bool streamed) {
   using St = Staged<M>;
   constexpr int C = St::C;
   if constexpr (G_IDX + 1 < St::kGroups) {
     if (grp != G_IDX) {
-      staged_write_group<M, G_IDX + 1, In>(grp, x, stride, N, b, c_w, R, out);
+      staged_write_group<M, G_IDX + 1, In>(grp, x, stride, N, b, c_w, R, out, streamed);
       return;
     }
   }
@@ -910,9 +924,14 @@ __device__ __forceinline__ void staged_write_group(int grp, const In* __restrict
       for (int j = 0; j < C; ++j) v[k][j] = src[k * St::kRow + j * St::kSub];
     tree_regs<M, C>(v);
     if (lane * C < St::kOut) {
+      float* rows = out + (long)(Q0 + qq) * M * N;
+      if (streamed) {
 #pragma unroll
-      for (int r = 0; r < M; ++r)
-        store_row4(out + (long)((Q0 + qq) * M + r) * N, c_w + lane * C, N, v[r]);
+        for (int r = 0; r < M; ++r) store_row4<true>(rows + (long)r * N, c_w + lane * C, N, v[r]);
+      } else {
+#pragma unroll
+        for (int r = 0; r < M; ++r) store_row4(rows + (long)r * N, c_w + lane * C, N, v[r]);
+      }
     }
   }
 }
@@ -924,13 +943,15 @@ __device__ __forceinline__ void staged_write_group(int grp, const In* __restrict
 // output, with the level-16 sums staged in LDS as in staged_tree_kernel,
 // instead of one pass over memory per level above 16: bound by the output's
 // writes. grid.x = (tile, offset group) dealt over the XCDs so that a tile's
-// groups, which read the same rows, share an L2; grid.y = time block.
-// Measured at 256 x 2^20: 0.76 ms (2.8 TB/s of input and output) against
+// groups, which read the same rows, share an L2; grid.y = time block. An output
+// larger than the last-level cache is stored past it (`streamed`), so that the
+// rows still to be read stay there (734 us otherwise).
+// Measured at 256 x 2^20: 0.695 ms (3.1 TB/s of input and output) against
 // 2.99 ms for level-16 trees, four one-level passes and a copy.
 template <int M, typename In>
 __global__ void __launch_bounds__(kWave * Staged<M>::kWaves, Staged<M>::kMinWaves)
     staged_write_kernel(const In* __restrict__ x, long stride, int N, int drift, int total_items,
-                        float* __restrict__ out) {
+                        float* __restrict__ out, bool streamed) {
   using St = Staged<M>;
   __shared__ __attribute__((aligned(16))) float r_storage[St::kFloats];
   const int per_xcd = gridDim.x / 8;
@@ -939,7 +960,7 @@ __global__ void __launch_bounds__(kWave * Staged<M>::kWaves, Staged<M>::kMinWave
   const long tb = blockIdx.y;
   staged_write_group<M, 0, In>(item % St::kGroups, x + tb * St::T * stride, stride, N, drift,
                                item / St::kGroups * St::kOut, (lds_float*)r_storage,
-                               out + tb * St::T * N);
+                               out + tb * St::T * N, streamed);
 }
 
 // One path sum per wave, in the tree's order: the pairwise recursion over the
@@ -1017,14 +1038,30 @@ __global__ void top_update_kernel(const float* __restrict__ sums, int T, int N, 
   }
 }
 
+// Column sums in row order (dedoppler.cu:68-71), four channels per thread: a
+// quarter of the load instructions and addresses of one channel per thread
+// (a gated batch's front 2 % of the batch; no change beside a single tree).
 template <typename In>
 __device__ __forceinline__ void colsum_body(const In* __restrict__ x, long stride, int T, int N,
                                             float* __restrict__ colsum) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= N) return;
-  float s = 0.0f;
-  for (int t = 0; t < T; ++t) s += to_f32<In>(x[(long)t * stride + c]);
-  colsum[c] = s;
+  const int c = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
+  if (c + 4 <= N) {
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
+    for (int t = 0; t < T; ++t) {
+      float v[4];
+      load4<In>(x + (long)t * stride + c, v);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s[j] += v[j];
+    }
+    *(float4*)(colsum + c) = make_float4(s[0], s[1], s[2], s[3]);
+  } else {
+    for (int i = c; i < N; ++i) {
+      float s = 0.0f;
+      for (int t = 0; t < T; ++t) s += to_f32<In>(x[(long)t * stride + i]);
+      colsum[i] = s;
+    }
+  }
 }
 
 template <typename In>
@@ -2075,7 +2112,8 @@ hipError_t staged_write_typed(const In* x, long stride, int T, int N, int drift,
   using St = Staged<M>;
   const int items = (N + St::kOut - 1) / St::kOut * St::kGroups;
   hipLaunchKernelGGL((staged_write_kernel<M, In>), dim3((items + 7) / 8 * 8, T / St::T),
-                     dim3(kWave * St::kWaves), 0, stream, x, stride, N, drift, items, out);
+                     dim3(kWave * St::kWaves), 0, stream, x, stride, N, drift, items, out,
+                     4L * T * N > kLastLevelCache);
   return hipGetLastError();
 }
 
@@ -2285,7 +2323,7 @@ hipError_t launch_top_update(const float* sums, int T, int N, int drift, int bmi
 
 hipError_t launch_colsum(const void* x, int dtype, long stride, int T, int N, float* colsum,
                          hipStream_t stream) {
-  const dim3 grid((N + 255) / 256), block(256);
+  const dim3 grid((N + 1023) / 1024), block(256);
   switch (dtype) {
     case 0:
       hipLaunchKernelGGL(colsum_kernel<float>, grid, block, 0, stream, (const float*)x, stride, T,
@@ -2344,7 +2382,7 @@ hipError_t launch_reset_set(const FrontSet& fs, int n, int N, hipStream_t stream
 hipError_t launch_front_set_stats(const FrontSet& fs, int n, int dtype, long stride, int T,
                                   int N, hipStream_t stream) {
   if (launch_reset_set(fs, n, N, stream) != hipSuccess) return hipErrorInvalidValue;
-  const dim3 cgrid((N + 255) / 256, n);
+  const dim3 cgrid((N + 1023) / 1024, n);
   switch (dtype) {
     case 0:
       hipLaunchKernelGGL(colsum_set_kernel<float>, cgrid, dim3(256), 0, stream, fs, stride, T, N);

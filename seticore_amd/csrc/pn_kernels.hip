@@ -97,7 +97,13 @@ __device__ __forceinline__ void pool_body(const In* __restrict__ x, long stride,
   const int t = (int)((i / kPooled) % kRows);
   const long blk = i / ((long)kPooled * kRows);
   const In* p = x + t * stride + blk * kBlockChannels + 4L * j;
-  const float s = (load_f32<In>(p) + load_f32<In>(p + 1)) + (load_f32<In>(p + 2) + load_f32<In>(p + 3));
+  // The four samples in one load, at any element alignment.
+  struct __attribute__((packed, aligned(sizeof(In)))) In4 {
+    In v[4];
+  };
+  const In4 q = *(const In4*)p;
+  const float s = (load_f32<In>(&q.v[0]) + load_f32<In>(&q.v[1])) +
+                  (load_f32<In>(&q.v[2]) + load_f32<In>(&q.v[3]));
   const float median = stats[0], sd = stats[1];
   float v = 2.0f * (s - 0.25f * median) / sd;
   v = fminf(fmaxf(v, kZMin), kZMax);
