@@ -66,10 +66,11 @@ namespace sc {
 //
 // Measured on MI355X: at 16 x 2^20 (132 drift blocks) C=4, G=4 with chunked
 // windows (mode 2) is the fastest T=16 shape. At 32..256 the LDS-staged
-// one-pass kernel (1.01, 1.83, 4.7, 17.8 ms at 2^20 channels and 66 blocks); at
+// one-pass kernel (1.01, 1.83, 4.7, 16.8 ms at 2^20 channels and 66 blocks); at
 // 256 with one workgroup per offset group (17.8 ms against 21.3 for one
-// workgroup over all four; at 128 the split is slower). Below 16 time steps:
-// 8 channels per lane, 16 drift blocks per window.
+// workgroup over all four, before the row loads were trimmed; at 128 the split
+// is slower). Below 16 time steps: 8 channels per lane, 16 drift blocks per
+// window.
 void default_tuning(int T, int N, bool half_width, int* lanes, int* group, int* prefetch) {
   const bool staged = T >= 32 && T <= 256;
   *lanes = (T == 16 || staged) ? 4 : 8;

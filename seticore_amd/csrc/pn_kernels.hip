@@ -376,7 +376,7 @@ __global__ void __launch_bounds__(256)
 // conv2's weights - is first brought into LDS, zero outside the maps, so the
 // sums below are free of bounds tests and of memory latency: at 256 blocks
 // (one workgroup per CU) 127 us with global loads inside the sums on 256
-// threads, 26 us now.
+// threads, 21 us now.
 constexpr int kBackThreads = 512;
 constexpr int kR1H = 7, kR1W = 13, kR1 = kR1H * kR1W;  // receptive field in h1
 constexpr int kRZH = kR1H + 2, kRZW = 2 * kR1W + 3;    // and in z
