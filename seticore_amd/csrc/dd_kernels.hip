@@ -997,20 +997,41 @@ __global__ void __launch_bounds__(kWave)
   if (lane == 0) q[blockIdx.x].w = __float_as_int(s);
 }
 
-// taylor.cu:97-109 + taylor.h:30-86: one stage in global memory.
-__global__ void one_step_kernel(const float* __restrict__ src, float* __restrict__ dst, int T,
-                                int N, int L, int drift) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+// taylor.cu:97-109 + taylor.h:30-86: one stage in global memory, level L from
+// the two halves of level L/2. Offsets 2h and 2h + 1 add the same lower entry h
+// to upper entry h at c + h and c + h + 1 (plus the shear), so a thread takes
+// both for four channels: every input is loaded once and the outputs are
+// 16-byte stores. Bound by memory: the whole tree of 512 x 2^17 takes 292 us (a
+// third of it this level), 4096 x 2^15 1050 with four levels here; with a
+// channel per thread looping over the rows 477 and 6577. Entries whose upper
+// half starts outside the coarse channel stay unwritten. grid.y = h, grid.z =
+// time block.
+__global__ void __launch_bounds__(256)
+    one_step_kernel(const float* __restrict__ src, float* __restrict__ dst, int N, int L,
+                    int drift) {
+  const long c = (blockIdx.x * 256L + threadIdx.x) * 4;
   if (c >= N) return;
-  const int ntb = T / L;
-  for (int tb = 0; tb < ntb; ++tb) {
-    for (int p = L - 1; p >= 0; --p) {
-      const int half = p / 2;
-      const int shift = (p + 1) / 2 + drift * L / 2;
-      if (c + shift < 0 || c + shift >= N) continue;
-      dst[(long)(tb * L + p) * N + c] = src[(long)(tb * L + half) * N + c] +
-                                        src[(long)(tb * L + half + L / 2) * N + c + shift];
-    }
+  const int h = blockIdx.y;
+  const float* lo = src + ((long)blockIdx.z * L + h) * N;
+  const float* up = lo + (long)(L / 2) * N;
+  float* even = dst + ((long)blockIdx.z * L + 2 * h) * N;
+  float* odd = even + N;
+  const long u = c + h + drift * L / 2;
+  if (c + 4 <= N && u >= 0 && u + 5 <= N) {
+    float a[4], b[4];
+    load4<float>(lo + c, a);
+    load4<float>(up + u, b);
+    const float last = up[u + 4];
+    const float s0[4] = {a[0] + b[0], a[1] + b[1], a[2] + b[2], a[3] + b[3]};
+    const float s1[4] = {a[0] + b[1], a[1] + b[2], a[2] + b[3], a[3] + last};
+    store_row4(even, (int)c, N, s0);
+    store_row4(odd, (int)c, N, s1);
+    return;
+  }
+  for (long i = c; i < min(c + 4, (long)N); ++i) {
+    const long v = u + (i - c);
+    if (v >= 0 && v < N) even[i] = lo[i] + up[v];
+    if (v + 1 >= 0 && v + 1 < N) odd[i] = lo[i] + up[v + 1];
   }
 }
 
@@ -2309,8 +2330,8 @@ hipError_t launch_tree_blocks(const void* x, int dtype, long stride, int T, int 
 
 hipError_t launch_one_step(const float* src, float* dst, int T, int N, int L, int drift,
                            hipStream_t stream) {
-  hipLaunchKernelGGL(one_step_kernel, dim3((N + 255) / 256), dim3(256), 0, stream, src, dst, T,
-                     N, L, drift);
+  hipLaunchKernelGGL(one_step_kernel, dim3((unsigned)(((long)N + 1023) / 1024), L / 2, T / L),
+                     dim3(256), 0, stream, src, dst, N, L, drift);
   return hipGetLastError();
 }
 

@@ -39,6 +39,18 @@ def test_tree_at_tile_edges(gpu, oracle, T, N, dtype):
         np.testing.assert_array_equal(got[ok], oracle.basic_taylor_tree(host, b)[ok])
 
 
+# Levels above 256 run in memory, four channels per thread and 1024 per workgroup.
+@pytest.mark.parametrize("T,N", [(512, 513), (512, 1024), (512, 1027), (1024, 2050), (2048, 4099)])
+def test_tree_levels_in_memory(gpu, oracle, T, N):
+    host, x, code = _data(T, N, "f32", T + N)
+    dd = sc.Dedopplerer(T, N, 1.0, 1.0)
+    for b in (-1, 0, 1):
+        print("levels", T, N, b, flush=True)
+        got = dd.taylor_tree(sc.FilterbankBuffer(T, N, data=x, dtype=code), b).cpu().numpy()
+        ok = _valid(T, N, b)
+        np.testing.assert_array_equal(got[ok], oracle.basic_taylor_tree(host, b)[ok])
+
+
 def test_tree_output_may_be_the_input(gpu, oracle):
     import ctypes
     T, N = 64, 777
