@@ -1035,27 +1035,55 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// dedoppler.cu:32-55 for one drift block, folded into the key (launched once
-// per drift block in ascending order, so a plain read-modify-write suffices).
-__global__ void top_update_kernel(const float* __restrict__ sums, int T, int N, int drift,
-                                  int bmin, top_key_t* __restrict__ top_key) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+// dedoppler.cu:32-55 for one drift block, folded into the key: kTopRows offsets
+// of four channels per thread (grid.y = rows), so that a narrow coarse channel
+// still fills the chip and the loads are 16 bytes wide. Keys order by (sum,
+// lowest offset) whichever chunk comes first; a key at or below the one stored
+// (which only rises) needs no atomic.
+constexpr int kTopRows = 32;
+__global__ void __launch_bounds__(256)
+    top_update_kernel(const float* __restrict__ sums, int T, int N, int drift, int bmin,
+                      top_key_t* __restrict__ top_key) {
+  const int c = (int)min((blockIdx.x * 256L + threadIdx.x) * 4, (long)N);
   if (c >= N) return;
-  float best = 0.0f;
-  int code = 0;
-  for (int p = 0; p < T; ++p) {
-    const int last = (T - 1) * drift + p + c;
-    if (last < 0 || last >= N) break;
-    const float s = sums[(long)N * p + c];
-    if (s > best) {
-      best = s;
-      code = (drift - bmin) * T + p;
+  const int p0 = blockIdx.y * kTopRows;
+  // Offsets [0, pmax) of channel c + j end inside the coarse channel.
+  int pmax[4];
+  float best[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  int at[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const long last0 = (long)(T - 1) * drift + c + j;
+    pmax[j] = (c + j >= N || last0 < 0) ? 0 : (int)max(0L, min((long)T, N - last0));
+  }
+  if (max(max(pmax[0], pmax[1]), max(pmax[2], pmax[3])) <= p0) return;
+  const bool whole = c + 4 <= N;
+#pragma unroll 8
+  for (int p = p0; p < min(T, p0 + kTopRows); ++p) {
+    const float* row = sums + (long)N * p + c;
+    float v[4];
+    if (whole) {
+      load4<float>(row, v);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = c + j < N ? row[j] : 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (p < pmax[j] && v[j] > best[j]) {
+        best[j] = v[j];
+        at[j] = p;
+      }
     }
   }
-  if (best > 0.0f) {
-    const top_key_t k = (top_key_t)__double_as_longlong(
-        make_key(best, (unsigned)kCodeMask - (unsigned)code));
-    if (k > top_key[c]) top_key[c] = k;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (best[j] > 0.0f) {
+      const unsigned code = (unsigned)((drift - bmin) * T + at[j]);
+      const top_key_t k =
+          (top_key_t)__double_as_longlong(make_key(best[j], (unsigned)kCodeMask - code));
+      if (k > top_key[c + j]) atomicMax(&top_key[c + j], k);
+    }
   }
 }
 
@@ -2337,8 +2365,9 @@ hipError_t launch_one_step(const float* src, float* dst, int T, int N, int L, in
 
 hipError_t launch_top_update(const float* sums, int T, int N, int drift, int bmin,
                              top_key_t* top_key, hipStream_t stream) {
-  hipLaunchKernelGGL(top_update_kernel, dim3((N + 255) / 256), dim3(256), 0, stream, sums, T, N,
-                     drift, bmin, top_key);
+  hipLaunchKernelGGL(top_update_kernel,
+                     dim3((unsigned)(((long)N + 1023) / 1024), (T + kTopRows - 1) / kTopRows),
+                     dim3(256), 0, stream, sums, T, N, drift, bmin, top_key);
   return hipGetLastError();
 }
 

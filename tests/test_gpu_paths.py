@@ -51,6 +51,33 @@ def test_tree_levels_in_memory(gpu, oracle, T, N):
         np.testing.assert_array_equal(got[ok], oracle.basic_taylor_tree(host, b)[ok])
 
 
+# Above 256 rows the path maxima are taken from memory, 32 offsets of four channels per thread; ties
+# between offsets and drift blocks keep the reference's first.
+@pytest.mark.parametrize("T,N,ties", [(300, 1024, False), (512, 1027, True), (600, 5001, True),
+                                      (2048, 515, False)])
+def test_search_above_256_rows(gpu, oracle, T, N, ties):
+    T_r = sc.round_up_to_power_of_two(T)
+    host = np.zeros((T_r, N), np.float32)
+    host[:T] = np.random.default_rng(T).exponential(size=(T, N))
+    if ties:
+        host = np.rint(host)
+    foff, tsamp = -2.79e-6, 18.25
+    max_drift = 2.6 * abs(1e6 * foff) / tsamp
+    import torch
+    dd = sc.Dedopplerer(T, N, foff, tsamp)
+    hits = []
+    print("search", T, N, ties, flush=True)
+    dd.search(sc.FilterbankBuffer(T_r, N, data=torch.from_numpy(host).cuda()),
+              sc.FilterbankMetadata(coarse_channel_size=N), sc.NO_BEAM, 0, max_drift, 0.0, 2.0, hits)
+    ref = oracle.search(host, T, foff, tsamp, max_drift, 0.0, 2.0)
+    st = dd.state()
+    np.testing.assert_array_equal(st["top_sums"], ref.top_sums)
+    pos = ref.top_sums > 0
+    np.testing.assert_array_equal(st["top_blocks"][pos], ref.top_blocks[pos])
+    np.testing.assert_array_equal(st["top_offsets"][pos], ref.top_offsets[pos])
+    assert [(h.index, h.drift_steps) for h in hits] == [(h["index"], h["drift_steps"]) for h in ref.hits]
+
+
 def test_tree_output_may_be_the_input(gpu, oracle):
     import ctypes
     T, N = 64, 777
