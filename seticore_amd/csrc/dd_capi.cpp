@@ -277,10 +277,11 @@ sc_status ensure_pass_scratch(sc_dd* dd, int nb) {
 
 // Path sums of one drift block into a [T_r][N] buffer: `out` if given, else one
 // of the handle's two (returned in *result). Up to 256 rows take one launch;
-// above, the levels from 512 on alternate between two buffers so that the
-// last one lands in `out`.
-sc_status run_tree(sc_dd* dd, const void* data, int dtype, long stride, int drift, float* out,
-                   float** result, hipStream_t stream) {
+// above, the levels from 512 up to `last` (T_r, or T_r/2 for a search, which
+// forms its last level in launch_top_step) alternate between two buffers so
+// that the last one lands in `out`.
+sc_status run_tree(sc_dd* dd, const void* data, int dtype, long stride, int drift, int last,
+                   float* out, float** result, hipStream_t stream) {
   const int T = dd->rounded, N = dd->num_channels;
   if (!out || T > 256) {
     sc_status s = ensure_tree_scratch(dd);
@@ -288,9 +289,9 @@ sc_status run_tree(sc_dd* dd, const void* data, int dtype, long stride, int drif
   }
   float* dst = out ? out : dd->tree_a;
   float* src = dd->tree_b;
-  for (int L = 512; L <= T; L *= 2) std::swap(src, dst);
+  for (int L = 512; L <= last; L *= 2) std::swap(src, dst);
   SC_HIP(sc::launch_tree_blocks(data, dtype, stride, T, N, drift, dst, stream), "tree blocks");
-  for (int L = 512; L <= T; L *= 2) {
+  for (int L = 512; L <= last; L *= 2) {
     std::swap(src, dst);
     SC_HIP(sc::launch_one_step(src, dst, T, N, L, drift, stream), "one step");
   }
@@ -627,16 +628,19 @@ sc_status enqueue_path_sums(sc_dd* dd, const void* data, int dtype, long row_str
                                  dd->pass_scratch, dd->pass_pitch, dd->top_key, stream),
              "two-pass tree");
     }
-  } else {
+  } else if (T > 256) {
     if (!overlap_stats)
       SC_HIP(sc::launch_colsum(data, dtype, row_stride, T, N, dd->colsum, stream),
              "column sums");
     for (int b = r.bmin; b <= r.bmax; ++b) {
-      float* sums = nullptr;
-      sc_status s = run_tree(dd, data, dtype, row_stride, b, nullptr, &sums, stream);
+      float* half = nullptr;
+      sc_status s = run_tree(dd, data, dtype, row_stride, b, T / 2, nullptr, &half, stream);
       if (s != SC_OK) return s;
-      SC_HIP(sc::launch_top_update(sums, T, N, b, r.bmin, dd->top_key, stream), "top update");
+      SC_HIP(sc::launch_top_step(half, T, N, b, r.bmin, dd->top_key, stream), "top step");
     }
+  } else {
+    // sc_dd_create and sc_dd_set_tuning admit compiled shapes only.
+    return fail(SC_ERR_UNSUPPORTED, "no compiled kernel shape for this T_r");
   }
   if (dd->timing) SC_HIP(hipEventRecord(dd->ev_stop, stream), "timing event");
   if (overlap_stats) {
@@ -1077,7 +1081,8 @@ sc_status sc_dd_taylor_tree(sc_dd* dd, const void* data, int dtype, int rounded_
   const size_t in_bytes =
       ((size_t)(dd->rounded - 1) * row_stride + dd->num_channels) * (dtype == SC_F32 ? 4 : 2);
   const bool apart = o0 + sizeof(float) * count <= d0 || d0 + in_bytes <= o0;
-  s = run_tree(dd, data, dtype, row_stride, drift_block, apart ? out : nullptr, &sums, stream);
+  s = run_tree(dd, data, dtype, row_stride, drift_block, dd->rounded, apart ? out : nullptr, &sums,
+               stream);
   if (s != SC_OK) return s;
   if (!apart)
     SC_HIP(hipMemcpyAsync(out, sums, sizeof(float) * count, hipMemcpyDeviceToDevice, stream),

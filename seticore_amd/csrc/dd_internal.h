@@ -166,9 +166,9 @@ hipError_t launch_tree_blocks(const void* x, int dtype, long stride, int T, int 
 hipError_t launch_one_step(const float* src, float* dst, int T, int N, int L, int drift,
                            hipStream_t stream);
 
-// Sequential per-drift-block top update from a [T][N] path-sum buffer.
-hipError_t launch_top_update(const float* sums, int T, int N, int drift, int bmin,
-                             top_key_t* top_key, hipStream_t stream);
+// The last stage (L = T > 256) from level T/2, its path sums folded into the keys.
+hipError_t launch_top_step(const float* src, int T, int N, int drift, int bmin,
+                           top_key_t* top_key, hipStream_t stream);
 
 // Column sums (dedoppler.cu:63-72 order) for the paths that do not fuse them.
 hipError_t launch_colsum(const void* x, int dtype, long stride, int T, int N, float* colsum,

@@ -1035,18 +1035,22 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// dedoppler.cu:32-55 for one drift block, folded into the key: kTopRows offsets
-// of four channels per thread (grid.y = rows), so that a narrow coarse channel
-// still fills the chip and the loads are 16 bytes wide. Keys order by (sum,
-// lowest offset) whichever chunk comes first; a key at or below the one stored
-// (which only rises) needs no atomic.
-constexpr int kTopRows = 32;
+// The last level of a tree above 256 rows (one_step_kernel's sums) with
+// dedoppler.cu:32-55 for its drift block folded into the key: 2 * kTopSteps
+// offsets of four channels per thread (grid.y), so that a narrow coarse channel
+// still fills the chip and the loads are 16 bytes wide. The path sums are never
+// written: bound by reading the level below. Keys order by (sum, lowest offset)
+// whichever chunk comes first; a key at or below the one stored (which only
+// rises) needs no atomic. A search of 512 x 2^17 (28 drift blocks) took 14.4 ms
+// with one thread per channel over the written sums, 9.4 in chunks of them,
+// 6.7 here; 1024 x 2^16 22.7, 11.7, 9.2.
+constexpr int kTopSteps = 16;
 __global__ void __launch_bounds__(256)
-    top_update_kernel(const float* __restrict__ sums, int T, int N, int drift, int bmin,
-                      top_key_t* __restrict__ top_key) {
+    top_step_kernel(const float* __restrict__ src, int T, int N, int drift, int bmin,
+                    top_key_t* __restrict__ top_key) {
   const int c = (int)min((blockIdx.x * 256L + threadIdx.x) * 4, (long)N);
   if (c >= N) return;
-  const int p0 = blockIdx.y * kTopRows;
+  const int h0 = blockIdx.y * kTopSteps;
   // Offsets [0, pmax) of channel c + j end inside the coarse channel.
   int pmax[4];
   float best[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -1056,23 +1060,37 @@ __global__ void __launch_bounds__(256)
     const long last0 = (long)(T - 1) * drift + c + j;
     pmax[j] = (c + j >= N || last0 < 0) ? 0 : (int)max(0L, min((long)T, N - last0));
   }
-  if (max(max(pmax[0], pmax[1]), max(pmax[2], pmax[3])) <= p0) return;
+  if (max(max(pmax[0], pmax[1]), max(pmax[2], pmax[3])) <= 2 * h0) return;
   const bool whole = c + 4 <= N;
-#pragma unroll 8
-  for (int p = p0; p < min(T, p0 + kTopRows); ++p) {
-    const float* row = sums + (long)N * p + c;
-    float v[4];
-    if (whole) {
-      load4<float>(row, v);
+#pragma unroll 4
+  for (int h = h0; h < min(T / 2, h0 + kTopSteps); ++h) {
+    const float* lo = src + (long)h * N + c;
+    const float* up = src + (long)(T / 2 + h) * N;
+    const long u = (long)drift * (T / 2) + c + h;
+    float a[4], b[5];
+    if (whole && u >= 0 && u + 5 <= N) {
+      float b4[4];
+      load4<float>(lo, a);
+      load4<float>(up + u, b4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b[j] = b4[j];
+      b[4] = up[u + 4];
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = c + j < N ? row[j] : 0.0f;
+      for (int j = 0; j < 4; ++j) a[j] = c + j < N ? lo[j] : 0.0f;
+#pragma unroll
+      for (int j = 0; j < 5; ++j) b[j] = u + j >= 0 && u + j < N ? up[u + j] : 0.0f;
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if (p < pmax[j] && v[j] > best[j]) {
-        best[j] = v[j];
-        at[j] = p;
+      const float even = a[j] + b[j], odd = a[j] + b[j + 1];
+      if (2 * h < pmax[j] && even > best[j]) {
+        best[j] = even;
+        at[j] = 2 * h;
+      }
+      if (2 * h + 1 < pmax[j] && odd > best[j]) {
+        best[j] = odd;
+        at[j] = 2 * h + 1;
       }
     }
   }
@@ -2363,11 +2381,11 @@ hipError_t launch_one_step(const float* src, float* dst, int T, int N, int L, in
   return hipGetLastError();
 }
 
-hipError_t launch_top_update(const float* sums, int T, int N, int drift, int bmin,
-                             top_key_t* top_key, hipStream_t stream) {
-  hipLaunchKernelGGL(top_update_kernel,
-                     dim3((unsigned)(((long)N + 1023) / 1024), (T + kTopRows - 1) / kTopRows),
-                     dim3(256), 0, stream, sums, T, N, drift, bmin, top_key);
+hipError_t launch_top_step(const float* src, int T, int N, int drift, int bmin,
+                           top_key_t* top_key, hipStream_t stream) {
+  hipLaunchKernelGGL(top_step_kernel,
+                     dim3((unsigned)(((long)N + 1023) / 1024), (T / 2 + kTopSteps - 1) / kTopSteps),
+                     dim3(256), 0, stream, src, T, N, drift, bmin, top_key);
   return hipGetLastError();
 }
 
