@@ -201,13 +201,17 @@ hipError_t launch_path_sums(const void* x, int dtype, long stride, int T, int N,
                             int n, hipStream_t stream);
 
 // ---- normalisation and synthetic data -------------------------------------
-// {mean, standard deviation, location} of the samples as three doubles at the
-// start of scratch (norm_scratch_bytes, 256-byte aligned), then the pass that
-// writes (x - loc) / std_dev.
+// {mean, standard deviation, location} of the samples as three doubles in device
+// memory (scratch: norm_scratch_bytes, 256-byte aligned), then the pass that
+// writes (x - loc) / deviation, clamped.
 hipError_t launch_norm_moments(const float* x, int T, int N, long stride, void* scratch,
-                               hipStream_t stream);
-hipError_t launch_norm_apply(const float* x, int T, int N, long stride, int out_dtype, double loc,
-                             double std_dev, float clamp, void* out, hipStream_t stream);
+                               double* moments, hipStream_t stream);
+hipError_t launch_norm_apply(const float* x, int T, int N, long stride, int out_dtype,
+                             const double* moments, float clamp, void* out, hipStream_t stream);
+// One of kNormSlots places for the moments in the current device's memory; the
+// caller sees to it that a slot has one user at a time.
+constexpr int kNormSlots = 64;
+hipError_t norm_slot_address(int slot, double** out);
 size_t norm_scratch_bytes(int N);
 
 // Loader conditioning (zero rows T..T_r-1; optional DC fix on rows < T).

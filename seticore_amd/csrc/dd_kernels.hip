@@ -1829,7 +1829,7 @@ __global__ void __launch_bounds__(1024)
 // deviation of the T*N samples in one pass over the input, then one pass that
 // writes. (A pass each for the column sums, the mean and the deviation, with
 // serial reductions between them, took 200 us at 16 x 2^20 where the reads
-// take 14 us each; the three in one take 25 us, a whole call 121 against
+// take 14 us each; the three in one take 25 us, a whole call 111 against
 // 400 us.)
 
 // Count, mean and sum of squared deviations of a set of samples; merged
@@ -1939,8 +1939,10 @@ __device__ __forceinline__ float from_f32<float>(float v) { return v; }
 // element alignment); grid.y = row, strided where there are more than 65535.
 template <typename Out>
 __global__ void __launch_bounds__(256)
-    norm_apply_kernel(const float* __restrict__ x, int T, int N, long stride, double loc, float sd,
-                      float clamp, Out* __restrict__ out) {
+    norm_apply_kernel(const float* __restrict__ x, int T, int N, long stride,
+                      const double* __restrict__ moments, float clamp, Out* __restrict__ out) {
+  const double loc = moments[2];
+  const float sd = (float)(moments[1] > 0.0 ? moments[1] : 1.0);
   typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
   struct __attribute__((packed, aligned(sizeof(Out)))) Out4 {
     Out v[4];
@@ -2504,16 +2506,14 @@ hipError_t launch_path_sums(const void* x, int dtype, long stride, int T, int N,
 }
 
 namespace {
-// Scratch of launch_norm_moments: moments out, partial moments, column sums,
-// statistics state (unused by the median alone), histograms.
+// Scratch of launch_norm_moments: partial moments, column sums, histograms.
 constexpr size_t norm_align(size_t n) { return (n + 255) / 256 * 256; }
 struct NormScratch {
   int parts;
-  size_t moments, part, colsum, hist, total;
+  size_t part, colsum, hist, total;
   explicit NormScratch(int N) {
     parts = (int)(((long)N + 255) / 256);
-    moments = 0;
-    part = norm_align(3 * sizeof(double));
+    part = 0;
     colsum = part + norm_align(sizeof(Moments) * (size_t)parts);
     hist = colsum + norm_align(sizeof(float) * (size_t)N);
     total = hist + norm_align(device_stats_hist_bytes());
@@ -2524,7 +2524,7 @@ struct NormScratch {
 size_t norm_scratch_bytes(int N) { return NormScratch(N).total; }
 
 hipError_t launch_norm_moments(const float* x, int T, int N, long stride, void* scratch,
-                               hipStream_t stream) {
+                               double* moments, hipStream_t stream) {
   const NormScratch L(N);
   char* base = (char*)scratch;
   // Location: the median of the raw column sums over T, so the normalised
@@ -2541,30 +2541,40 @@ hipError_t launch_norm_moments(const float* x, int T, int N, long stride, void* 
   hipLaunchKernelGGL(stats_pass2_kernel, grid, block, 0, stream, colsum, N, hist);
   hipLaunchKernelGGL(stats_pass3_kernel, grid, block, 0, stream, colsum, N, hist);
   hipLaunchKernelGGL(norm_final_kernel, dim3(1), dim3(1024), 0, stream, part, L.parts, T, hist,
-                     (double*)(base + L.moments));
+                     moments);
   return hipGetLastError();
 }
 
-hipError_t launch_norm_apply(const float* x, int T, int N, long stride, int out_dtype, double loc,
-                             double std_dev, float clamp, void* out, hipStream_t stream) {
-  const float sd = (float)(std_dev > 0.0 ? std_dev : 1.0);
+hipError_t launch_norm_apply(const float* x, int T, int N, long stride, int out_dtype,
+                             const double* moments, float clamp, void* out, hipStream_t stream) {
   const dim3 grid((unsigned)(((long)N + 1023) / 1024), std::min(T, 65535)), block(256);
   switch (out_dtype) {
     case 0:
-      hipLaunchKernelGGL(norm_apply_kernel<float>, grid, block, 0, stream, x, T, N, stride, loc,
-                         sd, clamp, (float*)out);
+      hipLaunchKernelGGL(norm_apply_kernel<float>, grid, block, 0, stream, x, T, N, stride,
+                         moments, clamp, (float*)out);
       break;
     case 1:
-      hipLaunchKernelGGL(norm_apply_kernel<__half>, grid, block, 0, stream, x, T, N, stride, loc,
-                         sd, clamp, (__half*)out);
+      hipLaunchKernelGGL(norm_apply_kernel<__half>, grid, block, 0, stream, x, T, N, stride,
+                         moments, clamp, (__half*)out);
       break;
     case 2:
-      hipLaunchKernelGGL(norm_apply_kernel<__hip_bfloat16>, grid, block, 0, stream, x, T, N,
-                         stride, loc, sd, clamp, (__hip_bfloat16*)out);
+      hipLaunchKernelGGL(norm_apply_kernel<__hip_bfloat16>, grid, block, 0, stream, x, T, N, stride,
+                         moments, clamp, (__hip_bfloat16*)out);
       break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
+}
+
+namespace {
+__device__ double norm_slots[kNormSlots][4];
+}
+
+hipError_t norm_slot_address(int slot, double** out) {
+  void* p = nullptr;
+  const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(norm_slots));
+  *out = (double*)p + 4 * slot;
+  return e;
 }
 
 hipError_t launch_condition(float* data, int T, int T_r, int N, long stride, int dc_spike,

@@ -144,3 +144,23 @@ def test_normalize_against_float64(gpu, T, N, stride, dtype):
         z, loc2, sd2 = sc.normalize(d, code, out=d)  # in place
         assert (loc2, sd2) == (loc, sd)
         np.testing.assert_array_equal(z.cpu().numpy(), y.cpu().numpy())
+
+
+def test_normalize_from_several_threads(gpu):
+    import torch
+    from concurrent.futures import ThreadPoolExecutor
+    x = [torch.from_numpy(np.random.default_rng(i).exponential(size=(16, 20001)).astype(np.float32) * (i + 1)).cuda()
+         for i in range(8)]
+    want = [sc.normalize(v, sc.SC_BF16) for v in x]
+    torch.cuda.synchronize()
+
+    def many(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            return [sc.normalize(x[i], sc.SC_BF16) for _ in range(5)]
+
+    print("normalize, 8 threads", flush=True)
+    with ThreadPoolExecutor(8) as pool:
+        for i, got in enumerate(pool.map(many, range(8))):
+            for y, loc, sd in got:
+                assert (loc, sd) == want[i][1:]
+                assert torch.equal(y, want[i][0])
