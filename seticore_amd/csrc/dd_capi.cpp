@@ -1397,16 +1397,8 @@ sc_status enqueue_front_set(sc_batch* b, size_t a, size_t e, hipStream_t stream)
   return SC_OK;
 }
 
-// The runs [a, e) of a gated batch: consecutive instances of one shape
-// (set_run), the first run of at most four. Nothing hides the first run's
-// front, so it is shorter: 16 x (16 x 2^18) at 60 % flagged take 1.68 ms in
-// runs of 8 and 8, 1.64 in 4, 8 and 4, 1.67 in 2, 4, 8 and 2 (whose second
-// front outlasts the first tree).
 std::vector<std::pair<size_t, size_t>> gated_runs(const sc_batch* b) {
-  std::vector<std::pair<size_t, size_t>> runs;
-  for (size_t a = 0, most = 4; a < b->inst.size(); a = runs.back().second, most *= 2)
-    runs.push_back({a, a + std::min(set_run(b, a), std::min<size_t>(most, sc::kMaxFusedSet))});
-  return runs;
+  return sc::gated_runs(b->inst.size(), [&](size_t i) { return set_run(b, i); });
 }
 
 // Gated batch run, as direct launches on three streams joined by events

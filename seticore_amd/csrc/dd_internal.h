@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include "../../include/seticore_amd.h"
+#include "batch_runs.h"
 
 namespace sc {
 
@@ -63,7 +64,6 @@ hipError_t launch_fused_tree_top(const void* x, int dtype, long stride, int T, i
 int fused_tile_width(int T, int C);
 // Up to kMaxFusedSet coarse channels of one shape (same T, N, row stride,
 // sample type and drift range) searched by one launch of the T_r = 16 kernel.
-constexpr int kMaxFusedSet = 8;
 struct FusedSet {
   const void* x[kMaxFusedSet];
   top_key_t* key[kMaxFusedSet];

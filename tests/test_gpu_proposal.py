@@ -318,3 +318,46 @@ def test_gated_batch_runs_share_a_tree_launch(gpu, dtype):
     for i in range(n_cc):
         assert none.flagged(i) == (0, 0)
         assert none.hits(i) == []
+
+
+# Twelve channels are runs of four and eight (every slot of a run's launches used); 70 instances whose
+# neighbours differ in width are 70 runs, more than twice the handles of either width.
+@pytest.mark.parametrize("widths,n_cc", [([1 << 15], 12), ([1 << 12, 1 << 13], 70)])
+def test_gated_batch_of_many_runs(gpu, widths, n_cc):
+    import torch
+    from seticore_amd import batch as B
+    net = sc.ProposalNet(max_batch=max(widths) // 4096, seed=11)
+    dds = {N: sc.Dedopplerer(T, N, FOFF, TSAMP) for N in widths}
+    metas = {N: sc.FilterbankMetadata(coarse_channel_size=N, foff=FOFF) for N in widths}
+    for dd in dds.values():
+        dd.set_stats_mode(sc.SC_STATS_DEVICE)
+    logits, data = [], []
+    for i in range(n_cc):
+        N = widths[i % len(widths)]
+        x = sc.normalize(_coarse_channel(torch, N, 300 + i), sc.SC_BF16)[0]
+        dds[N].search(sc.FilterbankBuffer(T, N, data=x, dtype=sc.SC_BF16), metas[N], -1, 0, 10.0, 0.0,
+                      8.0, [])
+        st = dds[N].state()
+        stats = torch.tensor([st["median"], st["std"]], dtype=torch.float32, device="cuda")
+        logits.append(net.forward(net.pool(x, stats)).cpu())
+        data.append(x)
+    thr = float(torch.cat(logits).median())
+    per_call, inst = [], []
+    for i, x in enumerate(data):
+        N, out = x.shape[1], []
+        flagged = dds[N].search_proposed(sc.FilterbankBuffer(T, N, data=x, dtype=sc.SC_BF16), net,
+                                         metas[N], -1, i, 10.0, 0.0, 8.0, thr, out)
+        per_call.append((flagged, out))
+        inst.append(B.instance(x, T, FOFF, TSAMP, 10.0, 0.0, 8.0, coarse_channel=i,
+                               dtype=sc.SC_BF16, metadata=metas[N]))
+    total, blocks = sum(f for f, _ in per_call), sum(x.shape[1] // 4096 for x in data)
+    print("%d instances, %d of %d blocks flagged, %d hits" %
+          (n_cc, total, blocks, sum(len(o) for _, o in per_call)), flush=True)
+    assert 0 < total < blocks
+    assert any(out for _, out in per_call)
+    gb = B.Batch(inst, proposal=net, logit_threshold=thr)
+    for _ in range(2):
+        gb.run()
+        for i, (flagged, out) in enumerate(per_call):
+            assert gb.flagged(i)[1] == flagged, i
+            assert _fields(gb.hits(i)) == _fields(out), i
