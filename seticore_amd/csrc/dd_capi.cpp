@@ -94,6 +94,12 @@ void default_tuning(int T, int N, bool half_width, int* lanes, int* group, int* 
   if (T == 256) *group = N < (1 << 15) ? 4 : N < (half_width ? 3 << 18 : 1 << 17) ? 16 : 256;
 }
 
+KernelShape search_shape(int T, int N, int dtype, bool tuned, const KernelShape& set) {
+  KernelShape s = set;
+  if (!tuned) default_tuning(T, N, dtype != SC_F32, &s.lanes, &s.group, &s.prefetch);
+  return s;
+}
+
 }  // namespace sc
 
 struct sc_dd {
@@ -154,7 +160,7 @@ struct sc_dd {
     long stride;
     int bmin, nblocks, window;
     double snr;
-    int lanes, group, prefetch;
+    sc::KernelShape shape;
     int pass_group, pass_blocks;
     bool use_two_pass;
     hipGraphExec_t exec;
@@ -589,6 +595,11 @@ bool block_key_search(const sc_dd* dd) {
          (!dd->use_two_pass && sc::staged_shape(dd->rounded, dd->lanes, dd->group, dd->prefetch));
 }
 
+sc::KernelShape search_shape(const sc_dd* dd, int dtype) {
+  return sc::search_shape(dd->rounded, dd->num_channels, dtype, dd->tuned,
+                          {dd->lanes, dd->group, dd->prefetch});
+}
+
 sc_status enqueue_path_sums(sc_dd* dd, const void* data, int dtype, long row_stride,
                             const DriftRange& r, hipStream_t stream,
                             bool overlap_stats = false, bool device_tail = false,
@@ -600,9 +611,7 @@ sc_status enqueue_path_sums(sc_dd* dd, const void* data, int dtype, long row_str
   SC_HIP(sc::launch_reset(dd->top_key, N, dd->stats_hist, stream), "reset");
   const bool one_pass = (T <= 16 || !dd->use_two_pass) &&
                         sc::fused_supported(T, dd->lanes, dd->group, dd->prefetch);
-  // The default shape follows the sample type too.
-  int lanes = dd->lanes, group = dd->group, prefetch = dd->prefetch;
-  if (!dd->tuned) sc::default_tuning(T, N, dtype != SC_F32, &lanes, &group, &prefetch);
+  const sc::KernelShape shape = search_shape(dd, dtype);
   // The fork point is right after the reset, but the side stream's launches
   // are issued after the path sums': a captured graph submits its nodes in
   // the order they were captured, and with the statistics first the tree
@@ -611,8 +620,8 @@ sc_status enqueue_path_sums(sc_dd* dd, const void* data, int dtype, long row_str
   if (overlap_stats) SC_HIP(hipEventRecord(dd->ev_fork, stream), "fork");
   if (dd->timing) SC_HIP(hipEventRecord(dd->ev_start, stream), "timing event");
   if (one_pass) {
-    SC_HIP(sc::launch_fused_tree_top(data, dtype, row_stride, T, N, r.bmin, nblocks, lanes,
-                                     group, prefetch, dd->top_key,
+    SC_HIP(sc::launch_fused_tree_top(data, dtype, row_stride, T, N, r.bmin, nblocks,
+                                     shape.lanes, shape.group, shape.prefetch, dd->top_key,
                                      overlap_stats ? nullptr : dd->colsum, stream, nullptr,
                                      nullptr, device_tail && block_key_search(dd)),
            "fused tree");
@@ -703,11 +712,11 @@ sc_status enqueue_device_tail(sc_dd* dd, const DriftRange& r, double snr_thresho
 sc_status search_graph(sc_dd* dd, const void* data, int dtype, long row_stride,
                        const DriftRange& r, double snr_threshold, hipGraphExec_t* out) {
   const int nblocks = r.bmax - r.bmin + 1;
+  const sc::KernelShape shape = search_shape(dd, dtype);
   for (auto& g : dd->graph_cache) {
     if (g.data == data && g.dtype == dtype && g.stride == row_stride && g.bmin == r.bmin &&
         g.nblocks == nblocks && g.window == r.window && g.snr == snr_threshold &&
-        g.lanes == dd->lanes && g.group == dd->group && g.prefetch == dd->prefetch &&
-        g.pass_group == dd->pass_group && g.pass_blocks == pass_blocks(dd) &&
+        g.shape == shape && g.pass_group == dd->pass_group && g.pass_blocks == pass_blocks(dd) &&
         g.use_two_pass == dd->use_two_pass) {
       *out = g.exec;
       return SC_OK;
@@ -738,8 +747,7 @@ sc_status search_graph(sc_dd* dd, const void* data, int dtype, long row_stride,
     dd->graph_cache.erase(dd->graph_cache.begin());
   }
   dd->graph_cache.push_back({data, dtype, row_stride, r.bmin, nblocks, r.window, snr_threshold,
-                             dd->lanes, dd->group, dd->prefetch, dd->pass_group,
-                             pass_blocks(dd), dd->use_two_pass, exec});
+                             shape, dd->pass_group, pass_blocks(dd), dd->use_two_pass, exec});
   *out = exec;
   return SC_OK;
 }
@@ -911,11 +919,12 @@ sc_status sc_dd_search(sc_dd* dd, const void* data, int dtype, int rounded_times
   } else {
     bool use_graph = dd->graphs && !dd->timing;
     if (use_graph) {
+      const sc::KernelShape shape = search_shape(dd, dtype);
       size_t h = std::hash<const void*>()(data);
       for (size_t v : {(size_t)dtype, (size_t)row_stride, (size_t)(long)r.bmin,
                        (size_t)(long)r.bmax, (size_t)r.window,
-                       std::hash<double>()(snr_threshold), (size_t)dd->lanes,
-                       (size_t)dd->group, (size_t)dd->prefetch, (size_t)dd->pass_group,
+                       std::hash<double>()(snr_threshold), (size_t)shape.lanes,
+                       (size_t)shape.group, (size_t)shape.prefetch, (size_t)dd->pass_group,
                        (size_t)pass_blocks(dd), (size_t)dd->use_two_pass})
         h = h * 1000003u ^ v;
       bool cached = false;

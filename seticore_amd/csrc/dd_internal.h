@@ -39,6 +39,17 @@ sc_hit make_hit(const sc_meta* meta, int index, int drift_steps, double drift_ra
 // mode / kernel selector), as measured best.
 void default_tuning(int T, int N, bool half_width, int* lanes, int* group, int* prefetch);
 
+struct KernelShape {
+  int lanes, group, prefetch;
+  bool operator==(const KernelShape& o) const {
+    return lanes == o.lanes && group == o.group && prefetch == o.prefetch;
+  }
+};
+// The shape a search of samples of `dtype` launches: `set`, the handle's, where
+// the caller chose it, else the default for that sample type (the handle holds
+// the one for float32). A captured search is looked up by it.
+KernelShape search_shape(int T, int N, int dtype, bool tuned, const KernelShape& set);
+
 // Per-channel search state: the bits of an FP64 key whose value orders
 // (top path sum, -code) lexicographically - the float sum widened to double
 // with 0x1FFFFFFF - code in the 29 low mantissa bits, where

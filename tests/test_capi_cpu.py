@@ -218,3 +218,16 @@ def test_batch_instance_checks_its_tensor():
         B.instance(torch.zeros((16, 8192)), 16, *args)      # host memory
     with pytest.raises(ValueError, match="2-D"):
         B.instance(torch.zeros((2, 16, 8192)), 16, *args)
+
+
+def test_captured_searches_are_kept_by_the_launched_shape(tmp_path):
+    import subprocess
+    from seticore_amd import build as b
+    exe = str(tmp_path / "search_shape")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-I", os.path.join(b.ROCM, "include"),
+                    "-D__HIP_PLATFORM_AMD__", os.path.join(b.CPP_TESTS, "search_shape.cpp"),
+                    "-L", b.HERE, "-lseticore_amd", "-L", os.path.join(b.ROCM, "lib"), "-lamdhip64",
+                    "-Wl,-rpath," + b.HERE, "-Wl,-rpath," + os.path.join(b.ROCM, "lib"), "-o", exe],
+                   check=True)
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0, out.stdout
