@@ -1225,9 +1225,14 @@ constexpr int kStatsBlocks = 256;
 // Workgroups of a counting pass over one channel where it runs beside a tree or
 // over several channels at once: its cost is the flush of every workgroup's
 // non-zero bins and the slots taken from the tree. 16 x 2^20, 54 drift blocks:
-// 276 us a call with 256, 272 with 64, 267 with 32, 272 with 16. (Alone, in
-// normalize, 256 are as fast.)
+// 276 us a call with 256, 272 with 64, 267 with 32, 272 with 16. Above 2^20
+// channels the reading counts for more, so each workgroup keeps to 32768 of
+// them: a 16 x 2^22 search in BF16 over 4 drift blocks takes 363 us (32
+// workgroups: 490), 16 x 2^24 1050 us (1818).
 constexpr int kCountBlocks = 32;
+int count_blocks(int N) {
+  return (int)std::min<long>(kStatsBlocks, std::max<long>(kCountBlocks, ((long)N + 32767) / 32768));
+}
 constexpr int kStatsThreads = 256;
 constexpr int kL1Bits = 13, kL2Bits = 10, kL3Bits = 9;
 constexpr int kL1 = 1 << kL1Bits, kL2 = 1 << kL2Bits, kL3 = 1 << kL3Bits;
@@ -1356,7 +1361,8 @@ __device__ __forceinline__ void for_each_value(const float* __restrict__ v, int 
 // LDS word (16 KB at level 1, 6 KB at level 2), so the workgroup fits
 // beside the tree kernels' 20 KB windows when one of them retires; a round
 // adds at most 256 * 16 to a counter, so the counts are flushed every 15
-// rounds, which only happens above 15.7 M values.
+// rounds, which only happens above 15.7 M values (256 workgroups of 4096
+// values a round; count_blocks).
 template <int NBINS, int RANKS, typename Match, typename Digit>
 __device__ void block_histogram(const float* __restrict__ v, int N, unsigned* lds,
                                 unsigned* __restrict__ out, Match match, Digit digit) {
@@ -2433,7 +2439,7 @@ size_t device_stats_hist_bytes() { return sizeof(unsigned) * stats_hist_words();
 hipError_t launch_device_stats(const float* colsum, int N, void* scratch, unsigned* hist,
                                float* stats_out, hipStream_t stream) {
   StatsState* st = (StatsState*)scratch;
-  const dim3 grid(kCountBlocks), block(kStatsThreads);
+  const dim3 grid(count_blocks(N)), block(kStatsThreads);
   hipLaunchKernelGGL(stats_pass1_kernel, grid, block, 0, stream, colsum, N, hist);
   hipLaunchKernelGGL(stats_pass2_kernel, grid, block, 0, stream, colsum, N, hist);
   hipLaunchKernelGGL(stats_pass3_kernel, grid, block, 0, stream, colsum, N, hist);
@@ -2474,7 +2480,7 @@ hipError_t launch_front_set_stats(const FrontSet& fs, int n, int dtype, long str
 hipError_t launch_device_stats_set(const FrontSet& fs, int n, int N, hipStream_t stream) {
   if (n < 1 || n > kMaxFusedSet) return hipErrorInvalidValue;
   const dim3 block(kStatsThreads);
-  const dim3 grid(kCountBlocks, n);
+  const dim3 grid(count_blocks(N), n);
   hipLaunchKernelGGL(stats_pass1_set_kernel, grid, block, 0, stream, fs, N);
   hipLaunchKernelGGL(stats_pass2_set_kernel, grid, block, 0, stream, fs, N);
   hipLaunchKernelGGL(stats_pass3_set_kernel, grid, block, 0, stream, fs, N);

@@ -641,3 +641,32 @@ def test_block_key_offsets_match_full_keys(gpu, oracle, T, ties):
     for i in dev:
         assert st["top_offsets"][i] == ref.top_offsets[i], i
         assert st["top_blocks"][i] == ref.top_blocks[i], i
+
+
+# Device statistics of wide coarse channels: more than 32 counting workgroups from 2^20 on, 256 and the
+# 16-bit counters emptied midway above 15.7 M. With ties nearly every value lands in one counter.
+@pytest.mark.parametrize("ties", [False, True])
+@pytest.mark.parametrize("N", [(1 << 20) + 1, (1 << 21) + 3, (1 << 24) + 5])
+def test_device_stats_of_wide_channels(gpu, N, ties):
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(N)
+    x = torch.empty((2, N), device="cuda")
+    if ties:
+        x[0] = 1.0 + (torch.rand(N, generator=g, device="cuda") < 0.2)
+        x[1] = 1.0
+    else:
+        x.exponential_(generator=g)
+    dd = sc.Dedopplerer(2, N, -2.79e-6, 18.25)
+    dd.set_stats_mode(sc.SC_STATS_DEVICE)
+    print("wide", N, ties, flush=True)
+    dd.search(sc.FilterbankBuffer(2, N, data=x), sc.FilterbankMetadata(coarse_channel_size=N),
+              sc.NO_BEAM, 0, 2.0, 0.0, 1e6, [])
+    st = dd.state()
+    v = (x[0] + x[1]).cpu().numpy()
+    np.testing.assert_array_equal(st["column_sums"], v)
+    first, last = int(np.ceil(0.05 * N)), int(np.floor(0.95 * N))
+    v = np.sort(v).astype(np.float64)
+    assert st["median"] == v[N // 2]
+    kept = v[first:last + 1]
+    assert abs(st["std"] - kept.std()) <= 1e-6 * kept.std()  # the tolerance of test_device_stats_mode
