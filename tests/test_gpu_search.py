@@ -670,3 +670,31 @@ def test_device_stats_of_wide_channels(gpu, N, ties):
     assert st["median"] == v[N // 2]
     kept = v[first:last + 1]
     assert abs(st["std"] - kept.std()) <= 1e-6 * kept.std()  # the tolerance of test_device_stats_mode
+
+
+# The window merge runs one wave (or a thread per path offset) where windows are at most 128 channels
+# wide, 256 threads above: either side of that and of a wave, and the narrowest window there is.
+@pytest.mark.parametrize("T", [2, 16, 64, 128, 256])
+@pytest.mark.parametrize("window", [2, 64, 66, 128, 130])
+def test_merge_of_narrow_windows(gpu, oracle, T, window):
+    from parity_helpers import device_hits_match_oracle
+    import torch
+    N, foff, tsamp = 8209, -2.79e-6, 18.25
+    max_drift = (window / 2 - 0.5) * abs(1e6 * foff / ((T - 1) * tsamp))
+    host = np.random.default_rng(T + window).exponential(size=(T, N)).astype(np.float32)
+    x = torch.from_numpy(host).cuda()
+    buf = sc.FilterbankBuffer(T, N, data=x)
+    meta = sc.FilterbankMetadata(coarse_channel_size=N, foff=foff)
+    dd = sc.Dedopplerer(T, N, foff, tsamp)
+    dd.set_stats_mode(sc.SC_STATS_DEVICE)
+    hits = []
+    print("merge", T, window, flush=True)
+    dd.search(buf, meta, sc.NO_BEAM, 0, max_drift, 0.0, 1.0, hits)
+    ref = oracle.search(host, T, foff, tsamp, max_drift, 0.0, 1.0)
+    got = device_hits_match_oracle(hits, ref, host, 1.0, T - 1)
+    assert got["same"] > 10
+    for _ in range(2):  # the captured search
+        again = []
+        dd.search(buf, meta, sc.NO_BEAM, 0, max_drift, 0.0, 1.0, again)
+        assert [(h.index, h.drift_steps, h.snr) for h in again] == \
+            [(h.index, h.drift_steps, h.snr) for h in hits]
