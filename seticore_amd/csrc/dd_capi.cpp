@@ -126,6 +126,7 @@ struct sc_dd {
   void* stats_scratch = nullptr;
   unsigned* stats_hist = nullptr;  // level-1 and level-2 histograms
   float* stats_out = nullptr;  // {median, std, mean, count}
+  int4* cand = nullptr;        // per-window candidates of a search of many windows
   float* tree_a = nullptr;     // T_r*N scratch for the staged path and tree API
   float* tree_b = nullptr;
   // Two-pass search (T_r = 32..256): scratch of pass_blocks * T_r * pass_pitch
@@ -220,6 +221,7 @@ void release(sc_dd* dd) {
   (void)hipFree(dd->stats_scratch);
   (void)hipFree(dd->stats_hist);
   (void)hipFree(dd->stats_out);
+  (void)hipFree(dd->cand);
   (void)hipFree(dd->tree_a);
   (void)hipFree(dd->tree_b);
   (void)hipFree(dd->pass_scratch);
@@ -255,6 +257,29 @@ sc_status ensure_tree_scratch(sc_dd* dd) {
   sc_status s = dev_alloc(dd, (void**)&dd->tree_a, bytes, "tree scratch");
   if (s != SC_OK) return s;
   return dev_alloc(dd, (void**)&dd->tree_b, bytes, "tree scratch");
+}
+
+// At most one candidate per window and window >= 2 (max_drift > 0).
+size_t cand_capacity(const sc_dd* dd) { return ((size_t)dd->num_channels + 1) / 2 + 1; }
+
+// Whether a search's candidates are collected in device memory and copied to
+// the host at once instead of written there by the merge. A copy costs a
+// launch; written, 16 bytes per window cross the bus one by one, also beside
+// the next instance of a batch. Written / copied: a search of 16 x 2^20 197 /
+// 198 us at 16384 windows, 213 / 201 at 32768, 915 / 665 at 2^19; a batch of
+// eight 2 x 2^20 at 65536 windows each 1875 / 1550.
+constexpr int kManyWindows = 16384;
+int num_windows(const sc_dd* dd, const DriftRange& r) {
+  return (int)(((long)dd->num_channels + r.window - 1) / r.window);
+}
+bool many_windows(const sc_dd* dd, const DriftRange& r) {
+  return num_windows(dd, r) > kManyWindows;
+}
+
+// The device candidates of such a search, allocated on first use.
+sc_status ensure_cand(sc_dd* dd, const DriftRange& r) {
+  if (dd->cand || !many_windows(dd, r)) return SC_OK;
+  return dev_alloc(dd, (void**)&dd->cand, cand_capacity(dd) * sizeof(int4), "candidates");
 }
 
 // Drift blocks per launch pair of the two-pass search: as set, or as many as
@@ -479,14 +504,12 @@ sc_status sc_dd_create(int num_timesteps, int num_channels, double foff_mhz, dou
   if (s == SC_OK)
     s = dev_alloc(dd, (void**)&dd->stats_hist, sc::device_stats_hist_bytes(), "stats hist");
   if (s == SC_OK) s = dev_alloc(dd, (void**)&dd->stats_out, 4 * sizeof(float), "stats");
-  // At most one candidate per window and window >= 2 (max_drift > 0).
-  const size_t cand_capacity = (N + 1) / 2 + 1;
   if (s == SC_OK) s = host_alloc((void**)&dd->h_colsum, N * sizeof(float), "column sums");
   if (s == SC_OK) s = host_alloc((void**)&dd->h_top_sum, N * sizeof(float), "top sums");
   if (s == SC_OK) s = host_alloc((void**)&dd->h_top_blk, N * sizeof(int), "top blocks");
   if (s == SC_OK) s = host_alloc((void**)&dd->h_top_off, N * sizeof(int), "top offsets");
   if (s == SC_OK)
-    s = host_alloc((void**)&dd->h_cand, cand_capacity * sizeof(int4), "candidates");
+    s = host_alloc((void**)&dd->h_cand, cand_capacity(dd) * sizeof(int4), "candidates");
   if (s == SC_OK) s = host_alloc((void**)&dd->h_stats, 4 * sizeof(float), "stats");
   if (sc::two_pass_supported(rounded, dd->pass_group)) {
     // The one-pass kernels (default up to 256 time steps) need no scratch;
@@ -671,8 +694,8 @@ sc_status enqueue_path_sums(sc_dd* dd, const void* data, int dtype, long row_str
   return SC_OK;
 }
 
-// One channel's part of a tail launch on handle dd: candidates and statistics
-// go straight to host memory.
+// One channel's part of a tail launch on handle dd: the statistics and, up to
+// kManyWindows, the candidates go straight to host memory.
 void tail_entry(sc::TailSet* ts, int i, const sc_dd* dd, const void* data, const DriftRange& r,
                 double snr_threshold, int4* h_cand, float* h_stats) {
   ts->x[i] = data;
@@ -681,10 +704,19 @@ void tail_entry(sc::TailSet* ts, int i, const sc_dd* dd, const void* data, const
   ts->top_sum[i] = dd->top_sum;
   ts->top_blk[i] = dd->top_blk;
   ts->top_off[i] = dd->top_off;
-  ts->cand[i] = h_cand;
+  ts->cand[i] = many_windows(dd, r) ? dd->cand : h_cand;
   ts->stats_copy[i] = h_stats;
   ts->window[i] = r.window;
   ts->snr[i] = snr_threshold;
+}
+
+// After the tail launch: the candidates to the host, unless they are there.
+sc_status copy_candidates(const sc_dd* dd, const DriftRange& r, int4* h_cand, hipStream_t stream) {
+  if (many_windows(dd, r))
+    SC_HIP(hipMemcpyAsync(h_cand, dd->cand, num_windows(dd, r) * sizeof(int4),
+                          hipMemcpyDeviceToHost, stream),
+           "copy candidates");
+  return SC_OK;
 }
 
 // Device statistics, then the window merge with the candidates' offsets after
@@ -705,7 +737,7 @@ sc_status enqueue_device_tail(sc_dd* dd, const DriftRange& r, double snr_thresho
   SC_HIP(sc::launch_window_merge_set(ts, 1, dtype, row_stride, N, T, r.bmin, block_key_search(dd),
                                      stream, gated),
          "window merge");
-  return SC_OK;
+  return copy_candidates(dd, r, h_cand, stream);
 }
 
 // The cached graph for this search, capturing it on first use.
@@ -763,8 +795,7 @@ sc_status device_hits(sc_dd* dd, const DriftRange& r, const sc_meta* meta, int b
   if (!h_stats) h_stats = dd->h_stats;
   if (!out) out = &dd->hits;
   if (num_timesteps <= 0) num_timesteps = dd->num_timesteps;
-  const int N = dd->num_channels;
-  const int nwin = (int)(((long)N + r.window - 1) / r.window);
+  const int nwin = num_windows(dd, r);
   if (h_stats[3] != 0.0f)
     return fail(SC_ERR_INVALID_ARGUMENT,
                 "input has NaN or infinite samples (" + std::to_string((long)h_stats[3]) +
@@ -917,6 +948,8 @@ sc_status sc_dd_search(sc_dd* dd, const void* data, int dtype, int rounded_times
     dd->last_std = std_dev;
     host_merge(dd, r, meta, beam, coarse_channel, min_drift, snr_threshold, median, std_dev);
   } else {
+    s = ensure_cand(dd, r);
+    if (s != SC_OK) return s;
     bool use_graph = dd->graphs && !dd->timing;
     if (use_graph) {
       const sc::KernelShape shape = search_shape(dd, dtype);
@@ -994,6 +1027,8 @@ sc_status sc_dd_search_proposed(sc_dd* dd, sc_pn* pn, const void* data, int dtyp
   if (r.window <= 0) return fail(SC_ERR_INVALID_ARGUMENT, "window size is 0");
   if ((long)(r.bmax - r.bmin + 1) * T > 0x1FFFFFFFL)
     return fail(SC_ERR_UNSUPPORTED, "drift range too large");
+  s = ensure_cand(dd, r);
+  if (s != SC_OK) return s;
   dd->hits.clear();
   dd->state_valid = false;
 
@@ -1497,7 +1532,11 @@ sc_status enqueue_gated(sc_batch* b, hipStream_t stream) {
     SC_HIP(sc::launch_window_merge_set(ts, (int)(e - a), b0.in.dtype, b0.in.row_stride,
                                        d0->num_channels, 16, b0.r.bmin, true, Q, true),
            "window merges");
-    for (size_t i = a; i < e; ++i) SC_HIP(hipEventRecord(tail_ev(i), Q), "tail done");
+    for (size_t i = a; i < e && s == SC_OK; ++i) {
+      const sc_batch::Instance& bi = b->inst[i];
+      s = copy_candidates(b->shapes[bi.shape], bi.r, b->h_cand + bi.cand_offset, Q);
+      if (s == SC_OK) SC_HIP(hipEventRecord(tail_ev(i), Q), "tail done");
+    }
   }
   if (s != SC_OK) return s;
   // Each run's tails follow its tree, and its front precedes it: the tails'
@@ -1563,6 +1602,8 @@ sc_status enqueue_plain(sc_batch* b, hipStream_t M, hipStream_t Q, NewEvent&& ne
         s = enqueue_device_tail(b->shapes[bj.shape], bj.r, bj.in.snr_threshold, bj.in.data,
                                 bj.in.dtype, bj.in.row_stride, Q, b->h_cand + bj.cand_offset,
                                 b->h_stats + 4 * j);
+      else
+        s = copy_candidates(b->shapes[bj.shape], bj.r, b->h_cand + bj.cand_offset, Q);
       if (s != SC_OK) break;
       hipEvent_t tail = nullptr;
       e = new_event(&tail);
@@ -1770,8 +1811,10 @@ sc_status batch_create(const sc_instance* instances, int count, const sc_tuning*
         break;
       }
     }
+    s = ensure_cand(b->shapes[shape], bi.r);
+    if (s != SC_OK) break;
     bi.cand_offset = total_windows;
-    total_windows += ((size_t)in.num_channels + bi.r.window - 1) / bi.r.window;
+    total_windows += (size_t)num_windows(b->shapes[shape], bi.r);
     b->inst.push_back(bi);
   }
   if (s == SC_OK) s = host_alloc((void**)&b->h_cand, total_windows * sizeof(int4), "candidates");

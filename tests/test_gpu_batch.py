@@ -222,3 +222,36 @@ def test_half_width_runs_share_a_launch(gpu, dtype):
     assert b.kernel_time()[1:] == (1, 5)  # one launch over the five channels
     assert _batch_hits(b) == want
     assert sum(len(w) for w in want) > 0
+
+
+# Candidates go to the host one by one up to 16384 merge windows and in one copy above: single searches
+# (direct, then captured, with other inputs between) and batches on both sides against the
+# allocation-free search, which copies them in pieces.
+@pytest.mark.parametrize("T,N,window", [(16, 65536, 4), (16, 65540, 4), (2, 40000, 2)])
+def test_candidates_of_many_windows(gpu, T, N, window):
+    import torch
+    max_drift = (window / 2 - 0.5) * abs(1e6 * FOFF / ((T - 1) * TSAMP))
+    meta = sc.FilterbankMetadata(coarse_channel_size=N, foff=FOFF)
+    xs = [torch.from_numpy(np.random.default_rng(i).exponential(size=(T, N)).astype(np.float32)).cuda()
+          for i in range(3)]
+
+    def fields(hits):
+        return [(h.index, h.drift_steps, h.snr, h.power) for h in hits]
+
+    want = [fields(sc.search_static(sc.FilterbankBuffer(T, N, data=x), T, FOFF, TSAMP, meta,
+                                    sc.NO_BEAM, 0, max_drift, 0.0, 1.5)) for x in xs]
+    assert all(len(w) > 100 for w in want)
+    dd = sc.Dedopplerer(T, N, FOFF, TSAMP)
+    dd.set_stats_mode(sc.SC_STATS_DEVICE)
+    buf = xs[0].clone()
+    for k in range(6):  # one buffer, changing contents
+        buf.copy_(xs[k % 3])
+        hits = []
+        dd.search(sc.FilterbankBuffer(T, N, data=buf), meta, sc.NO_BEAM, 0, max_drift, 0.0, 1.5, hits)
+        assert fields(hits) == want[k % 3], k
+    b = B.Batch([B.instance(xs[i % 3], T, FOFF, TSAMP, max_drift, 0.0, 1.5, metadata=meta)
+                 for i in range(11)])
+    for _ in range(2):
+        b.run()
+        for i in range(11):
+            assert fields(b.hits(i)) == want[i % 3], i
