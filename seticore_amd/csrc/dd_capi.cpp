@@ -433,6 +433,18 @@ void host_merge(sc_dd* dd, const DriftRange& r, const sc_meta* meta, int beam,
   }
 }
 
+// Whether p lies in the current device's own memory: not host memory (where a
+// kernel's reads cross the bus and its atomics depend on it) and not a peer's.
+bool on_current_device(const void* p) {
+  hipPointerAttribute_t a = {};
+  int device = -1;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess || hipGetDevice(&device) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice && a.device == device;
+}
+
 sc_status validate_input(const sc_dd* dd, const void* data, int dtype, int rounded, int N,
                          long stride) {
   if (!dd) return fail(SC_ERR_INVALID_ARGUMENT, "null handle");
@@ -1214,10 +1226,11 @@ sc_status sc_normalize(const float* data, int rounded_timesteps, int num_channel
   hipStream_t stream = (hipStream_t)stream_ptr;
   // The intermediates (column sums, partial moments, histograms) are done with
   // before the first normalised sample is written, so they live in the output
-  // where it is large enough and lies apart from the input, the moments, which
-  // the last pass reads, in a slot of their own (16 x 2^20 to BF16: 111 us a call,
-  // 119 with a wait for the host between the passes); else in memory allocated
-  // for the call.
+  // where it is large enough, lies apart from the input and is this device's
+  // memory, the moments, which the last pass reads, in a slot of their own
+  // (16 x 2^20 to BF16: 111 us a call, 119 with a wait for the host between the
+  // passes); else in memory allocated for the call. (In a pinned host output
+  // the passes' reads and atomics cross the bus: 16 x 2^18 took 3.4 ms.)
   const int T = rounded_timesteps, N = num_channels;
   const size_t need = sc::norm_scratch_bytes(N);
   const uintptr_t o0 = (uintptr_t)out, d0 = (uintptr_t)data;
@@ -1229,7 +1242,7 @@ sc_status sc_normalize(const float* data, int rounded_timesteps, int num_channel
   char* own = nullptr;
   void* scratch = (void*)base;
   double* moments = nullptr;
-  if (!apart || base + need > o0 + out_bytes || slot.index < 0) {
+  if (!apart || base + need > o0 + out_bytes || slot.index < 0 || !on_current_device(out)) {
     SC_HIP(hipMalloc((void**)&own, 256 + need), "normalize scratch");
     scratch = own + 256;
     moments = (double*)own;

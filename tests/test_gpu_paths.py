@@ -164,3 +164,18 @@ def test_normalize_from_several_threads(gpu):
             for y, loc, sd in got:
                 assert (loc, sd) == want[i][1:]
                 assert torch.equal(y, want[i][0])
+
+
+# An output in pinned host memory takes no intermediates (they are read back and added to atomically).
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_normalize_into_host_memory(gpu, dtype):
+    import torch
+    T, N = 16, 70001
+    code, kind = {"f32": (sc.SC_F32, torch.float32), "bf16": (sc.SC_BF16, torch.bfloat16)}[dtype]
+    _, x, _ = _data(T, N, "f32", 8)
+    want, loc, sd = sc.normalize(x, code)
+    out = torch.empty((T, N), dtype=kind, pin_memory=True)
+    print("normalize to the host", dtype, flush=True)
+    got = sc.normalize(x, code, out=out)
+    assert got[1:] == (loc, sd)
+    assert torch.equal(out, want.cpu())
