@@ -150,8 +150,12 @@ struct sc_dd {
   int* h_top_off = nullptr;
   int4* h_cand = nullptr;
   float* h_stats = nullptr;
-  int4* h_paths = nullptr;  // addIncoherentPower's path queries and results
+  // addIncoherentPower: the path queries, then as many sums; the same on the
+  // device for many hits.
+  int4* h_paths = nullptr;
   size_t paths_capacity = 0;
+  int4* d_paths = nullptr;
+  size_t d_paths_capacity = 0;
 
   // Graph replay of the device-statistics search (keyed by input and
   // parameters), captured on a private stream and launched on the caller's.
@@ -229,6 +233,7 @@ void release(sc_dd* dd) {
   (void)hipFree(dd->gate_count);
   (void)hipHostFree(dd->h_gate);
   (void)hipHostFree(dd->h_paths);
+  (void)hipFree(dd->d_paths);
   (void)hipHostFree(dd->h_colsum);
   (void)hipHostFree(dd->h_top_sum);
   (void)hipHostFree(dd->h_top_blk);
@@ -335,6 +340,15 @@ sc_status run_tree(sc_dd* dd, const void* data, int dtype, long stride, int drif
 // thread and run while the tree does; below, a thread or a further stream costs
 // more than it saves (a 13 x 5003 search takes 57 us in all).
 constexpr int kParallelStats = 65536;
+
+// With more hits than this over up to kManyPathsRows rows, addIncoherentPower
+// copies its queries to the device and the sums back; below, the kernel reads
+// and writes them in host memory, which costs less than the copies until the
+// accesses over the bus take longer than the sums. In host memory / copied:
+// 16 x 2^20 116 / 112 us at 8000 hits, 914 / 760 at 64000; 256 x 2^18 at 64000
+// 890 / 940.
+constexpr size_t kManyPaths = 8192;
+constexpr int kManyPathsRows = 64;
 
 // dedoppler.cu:241-262, same calls on a copy of the column sums.
 void host_exact_stats(const float* colsums, int n, float* median_out, float* std_out) {
@@ -1159,13 +1173,24 @@ sc_status sc_dd_add_incoherent_power(sc_dd* dd, const void* data, int dtype,
   std::sort(hits, hits + num_hits, [](const sc_hit& a, const sc_hit& b) {
     return a.drift_steps < b.drift_steps;
   });
+  const size_t query_bytes = sizeof(int4) + sizeof(float);
   if (num_hits > dd->paths_capacity) {
     (void)hipHostFree(dd->h_paths);
     dd->h_paths = nullptr;
     dd->paths_capacity = 0;
-    s = host_alloc((void**)&dd->h_paths, num_hits * sizeof(int4), "path queries");
+    s = host_alloc((void**)&dd->h_paths, num_hits * query_bytes, "path queries");
     if (s != SC_OK) return s;
     dd->paths_capacity = num_hits;
+  }
+  const bool many = num_hits > kManyPaths && dd->rounded <= kManyPathsRows;
+  if (many && num_hits > dd->d_paths_capacity) {
+    (void)hipFree(dd->d_paths);
+    dd->d_paths = nullptr;
+    dd->device_bytes -= dd->d_paths_capacity * query_bytes;
+    dd->d_paths_capacity = 0;
+    s = dev_alloc(dd, (void**)&dd->d_paths, num_hits * query_bytes, "path queries");
+    if (s != SC_OK) return s;
+    dd->d_paths_capacity = num_hits;
   }
   // Every hit's own path is summed in the tree's order, all hits in one launch
   // (the reference runs the whole tree of each drift block that has a hit and
@@ -1181,12 +1206,21 @@ sc_status sc_dd_add_incoherent_power(sc_dd* dd, const void* data, int dtype,
       return fail(SC_ERR_INVALID_ARGUMENT, "hit outside the searched range");
     dd->h_paths[i] = make_int4(hits[i].index, block, offset, 0);
   }
-  SC_HIP(sc::launch_path_sums(data, dtype, row_stride, dd->rounded, dd->num_channels, dd->h_paths,
-                              (int)num_hits, stream),
+  float* sums = (float*)(dd->h_paths + num_hits);
+  int4* queries = many ? dd->d_paths : dd->h_paths;
+  float* out = many ? (float*)(dd->d_paths + num_hits) : sums;
+  if (many)
+    SC_HIP(hipMemcpyAsync(queries, dd->h_paths, num_hits * sizeof(int4), hipMemcpyHostToDevice,
+                          stream),
+           "copy path queries");
+  SC_HIP(sc::launch_path_sums(data, dtype, row_stride, dd->rounded, dd->num_channels, queries,
+                              (int)num_hits, out, stream),
          "path sums");
+  if (many)
+    SC_HIP(hipMemcpyAsync(sums, out, num_hits * sizeof(float), hipMemcpyDeviceToHost, stream),
+           "copy path sums");
   SC_HIP(hipStreamSynchronize(stream), "incoherent power");
-  for (size_t i = 0; i < num_hits; ++i)
-    std::memcpy(&hits[i].incoherent_power, &dd->h_paths[i].w, sizeof(float));
+  for (size_t i = 0; i < num_hits; ++i) hits[i].incoherent_power = sums[i];
   return SC_OK;
 }
 

@@ -205,11 +205,11 @@ size_t device_stats_hist_bytes();
 hipError_t launch_device_stats(const float* colsum, int N, void* scratch, unsigned* hist,
                                float* stats_out, hipStream_t stream);
 
-// queries[i] = {channel, drift block, path offset, -}: the path sum's float bits
-// into .w (host-visible memory; T up to 4096 rows, samples outside the coarse
-// channel count as 0).
-hipError_t launch_path_sums(const void* x, int dtype, long stride, int T, int N, int4* queries,
-                            int n, hipStream_t stream);
+// sums[i] = the path sum of queries[i] = {channel, drift block, path offset, -}
+// (both may be host-visible memory; T up to 4096 rows, samples outside the
+// coarse channel count as 0).
+hipError_t launch_path_sums(const void* x, int dtype, long stride, int T, int N,
+                            const int4* queries, int n, float* sums, hipStream_t stream);
 
 // ---- normalisation and synthetic data -------------------------------------
 // {mean, standard deviation, location} of the samples as three doubles in device

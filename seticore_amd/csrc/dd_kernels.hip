@@ -969,12 +969,13 @@ __global__ void __launch_bounds__(kWave * Staged<M>::kWaves, Staged<M>::kMinWave
 // L whose upper half holds t, (offset of that level + 1)/2 channels on. T up
 // to 4096 rows: lane i owns rows i*T/64 .. of a shared array, then the lanes
 // combine by butterflies (float addition commutes, so both sides hold the
-// same sum). q[i] = {index, block, offset, result}; the array is in host
-// memory. Latency bound: T loads per hit in flight at once.
+// same sum). q[i] = {index, block, offset, -}. Latency bound: T loads per hit
+// in flight at once.
 constexpr int kMaxPathRows = 4096;
 template <typename In>
 __global__ void __launch_bounds__(kWave)
-    path_sums_kernel(const In* __restrict__ x, long stride, int T, int N, int4* __restrict__ q) {
+    path_sums_kernel(const In* __restrict__ x, long stride, int T, int N, const int4* __restrict__ q,
+                     float* __restrict__ sums) {
   __shared__ float leaf[kMaxPathRows];
   const int lane = threadIdx.x;
   const int4 h = q[blockIdx.x];
@@ -994,7 +995,7 @@ __global__ void __launch_bounds__(kWave)
     for (int i = 0; i < per; i += 2 * w) own[i] += own[i + w];
   float s = lane < T ? own[0] : 0.0f;
   for (int o = 1; o < min(T, kWave); o *= 2) s += __shfl_xor(s, o);
-  if (lane == 0) q[blockIdx.x].w = __float_as_int(s);
+  if (lane == 0) sums[blockIdx.x] = s;
 }
 
 // taylor.cu:97-109 + taylor.h:30-86: one stage in global memory, level L from
@@ -2493,22 +2494,22 @@ hipError_t launch_device_stats_set(const FrontSet& fs, int n, int N, hipStream_t
   return hipGetLastError();
 }
 
-hipError_t launch_path_sums(const void* x, int dtype, long stride, int T, int N, int4* queries,
-                            int n, hipStream_t stream) {
+hipError_t launch_path_sums(const void* x, int dtype, long stride, int T, int N,
+                            const int4* queries, int n, float* sums, hipStream_t stream) {
   if (n <= 0) return hipSuccess;
   if (T > kMaxPathRows) return hipErrorInvalidValue;
   switch (dtype) {
     case 0:
       hipLaunchKernelGGL(path_sums_kernel<float>, dim3(n), dim3(kWave), 0, stream,
-                         (const float*)x, stride, T, N, queries);
+                         (const float*)x, stride, T, N, queries, sums);
       break;
     case 1:
       hipLaunchKernelGGL(path_sums_kernel<__half>, dim3(n), dim3(kWave), 0, stream,
-                         (const __half*)x, stride, T, N, queries);
+                         (const __half*)x, stride, T, N, queries, sums);
       break;
     case 2:
       hipLaunchKernelGGL(path_sums_kernel<__hip_bfloat16>, dim3(n), dim3(kWave), 0, stream,
-                         (const __hip_bfloat16*)x, stride, T, N, queries);
+                         (const __hip_bfloat16*)x, stride, T, N, queries, sums);
       break;
     default: return hipErrorInvalidValue;
   }

@@ -179,3 +179,29 @@ def test_normalize_into_host_memory(gpu, dtype):
     got = sc.normalize(x, code, out=out)
     assert got[1:] == (loc, sd)
     assert torch.equal(out, want.cpu())
+
+
+# Up to 8192 hits are read and written in host memory, more at up to 64 rows copied; one handle, its
+# buffers growing and then larger than needed.
+@pytest.mark.parametrize("T,dtype", [(2, "f16"), (64, "f32"), (128, "f32")])
+def test_incoherent_power_of_many_hits(gpu, oracle, T, dtype):
+    N = 3001
+    host, x, code = _data(T, N, dtype, T)
+    dd = sc.Dedopplerer(T, N, 1.0, 1.0)
+    trees = {b: oracle.basic_taylor_tree(host, b) for b in (-1, 0, 1)}
+    rng = np.random.default_rng(T)
+    for n in (8192, 8193, 20000, 9000):
+        d = rng.integers(-(T - 1), 2 * (T - 1), size=n)
+        c = rng.integers(np.maximum(0, -d), N - np.maximum(0, d))
+        hits = [sc.DedopplerHit(index=int(i), drift_steps=int(s)) for i, s in zip(c, d)]
+        print("many hits", T, dtype, n, flush=True)
+        dd.addIncoherentPower(sc.FilterbankBuffer(T, N, data=x, dtype=code), hits)
+        steps = np.array([h.drift_steps for h in hits])
+        index = np.array([h.index for h in hits])
+        got = np.array([h.incoherent_power for h in hits], np.float32)
+        block, offset = np.divmod(steps, T - 1)
+        want = np.empty(n, np.float32)
+        for b in trees:
+            m = block == b
+            want[m] = trees[b][offset[m], index[m]]
+        np.testing.assert_array_equal(got, want)
