@@ -205,3 +205,20 @@ def test_incoherent_power_of_many_hits(gpu, oracle, T, dtype):
             m = block == b
             want[m] = trees[b][offset[m], index[m]]
         np.testing.assert_array_equal(got, want)
+
+
+# Path sums into pinned host memory: written there up to 512 rows, copied above.
+@pytest.mark.parametrize("T", [16, 64, 512, 1024])
+def test_tree_into_host_memory(gpu, T):
+    import ctypes
+    import torch
+    N = 2003
+    _, x, code = _data(T, N, "f32", T)
+    dd = sc.Dedopplerer(T, N, 1.0, 1.0)
+    want = dd.taylor_tree(sc.FilterbankBuffer(T, N, data=x, dtype=code), 1).cpu().numpy()
+    out = torch.zeros((T, N), pin_memory=True)
+    print("tree to the host", T, flush=True)
+    sc.check(sc.lib().sc_dd_taylor_tree(dd._h, ctypes.c_void_p(x.data_ptr()), code, T, N, N, 1,
+                                        ctypes.c_void_p(out.data_ptr()), None))
+    ok = _valid(T, N, 1)
+    np.testing.assert_array_equal(out.numpy()[ok], want[ok])
