@@ -2462,7 +2462,8 @@ hipError_t launch_reset_set(const FrontSet& fs, int n, int N, hipStream_t stream
 
 hipError_t launch_front_set_stats(const FrontSet& fs, int n, int dtype, long stride, int T,
                                   int N, hipStream_t stream) {
-  if (launch_reset_set(fs, n, N, stream) != hipSuccess) return hipErrorInvalidValue;
+  const hipError_t reset = launch_reset_set(fs, n, N, stream);
+  if (reset != hipSuccess) return reset;
   const dim3 cgrid((N + 1023) / 1024, n);
   switch (dtype) {
     case 0:
