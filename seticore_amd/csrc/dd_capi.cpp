@@ -369,7 +369,9 @@ void host_exact_stats(const float* colsums, int n, float* median_out, float* std
     } catch (const std::system_error&) {
     }
   }
-  std::nth_element(sums, sums + first, sums + mid - 1);
+  // (One channel has no lower range: it would end before it begins, and the
+  // reference's call runs through memory.)
+  if (mid > 0) std::nth_element(sums, sums + first, sums + mid - 1);
   if (upper.joinable())
     upper.join();
   else

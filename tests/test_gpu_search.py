@@ -698,3 +698,27 @@ def test_merge_of_narrow_windows(gpu, oracle, T, window):
         dd.search(buf, meta, sc.NO_BEAM, 0, max_drift, 0.0, 1.0, again)
         assert [(h.index, h.drift_steps, h.snr) for h in again] == \
             [(h.index, h.drift_steps, h.snr) for h in hits]
+
+
+# A few channels: the ranges of the trimmed statistics are empty or hold one value; one channel has no
+# deviation, so no threshold and no hits.
+@pytest.mark.parametrize("T", [2, 16, 300])
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 8])
+def test_search_of_a_few_channels(gpu, oracle, T, N):
+    T_r = sc.round_up_to_power_of_two(T)
+    data = np.zeros((T_r, N), np.float32)
+    data[:T] = np.random.default_rng(10 * T + N).exponential(size=(T, N))
+    import torch
+    dd = sc.Dedopplerer(T, N, -2.79e-6, 18.25)
+    hits = []
+    print("few", T, N, flush=True)
+    dd.search(sc.FilterbankBuffer(T_r, N, data=torch.from_numpy(data).cuda()),
+              sc.FilterbankMetadata(coarse_channel_size=N, foff=-2.79e-6), sc.NO_BEAM, 0, 0.1, 0.0, 0.5, hits)
+    st = dd.state()
+    if N == 1:
+        assert not hits and st["median"] == st["column_sums"][0] and np.isnan(st["std"])
+        return
+    ref = oracle.search(data, T, -2.79e-6, 18.25, 0.1, 0.0, 0.5)
+    np.testing.assert_array_equal(st["top_sums"], ref.top_sums)
+    assert (st["median"], st["std"]) == (ref.median, ref.std)
+    assert [_hit_fields(h) for h in hits] == [_hit_fields(h) for h in ref.hits]
