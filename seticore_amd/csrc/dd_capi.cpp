@@ -124,7 +124,7 @@ struct sc_dd {
   int* top_blk = nullptr;
   int* top_off = nullptr;
   void* stats_scratch = nullptr;
-  unsigned* stats_hist = nullptr;  // level-1 and level-2 histograms
+  unsigned* stats_hist = nullptr;  // the radix levels' histograms and selections
   float* stats_out = nullptr;  // {median, std, mean, count}
   int4* cand = nullptr;        // per-window candidates of a search of many windows
   float* tree_a = nullptr;     // T_r*N scratch for the staged path and tree API
@@ -1368,11 +1368,11 @@ extern "C" sc_status sc_condition_coarse_channel(float* data, int num_timesteps,
 //
 // The reference searches one coarse channel per call (run_dedoppler.cpp:35-51,
 // beamforming_pipeline.cpp:145-253). Here every instance's launch sequence
-// (reset, path sums, device statistics, window merge, candidate copy) is
-// captured once into a single hipGraph and the whole batch runs as one graph
-// launch. The path sums of successive instances form one chain; each
-// instance's statistics/merge/copy tail hangs off its path sums on a second
-// chain, so it can overlap the next instance's path sums. Instances of one
+// (reset, path sums, device statistics, window merge) is captured once into a
+// single hipGraph and the whole batch runs as one graph launch. The path sums of
+// successive instances form one chain; each instance's statistics and merge hang
+// off its path sums on a second chain, so they can overlap the next instance's
+// path sums. Instances of one
 // shape (rounded time steps, channels, foff, tsamp) share search handles:
 // two, used alternately (measured +10 % at 16 x 2^20 and +1.6 % on the uneven
 // 16..256 batch), 2 x kMaxFusedSet at 16 time steps (runs of consecutive
@@ -1508,7 +1508,7 @@ std::vector<std::pair<size_t, size_t>> gated_runs(const sc_batch* b) {
 // Gated batch run, as direct launches on three streams joined by events
 // (device-side waits): the trees on one in instance order, the fronts (reset,
 // column sums, statistics, pooling, network, tile lists) on the second, the
-// tails (merge, offsets, copies) on the third. Runs of consecutive instances
+// tails (the window merges) on the third. Runs of consecutive instances
 // of one shape (set_run) share one launch per step of the front and one tree
 // launch over their tile lists. The next run's front is enqueued right after
 // the current run's tree, so it runs beside it, once the tails of the
@@ -1612,7 +1612,7 @@ struct BatchTimer {
 };
 
 // The plain batch's launch sequence, into streams M (path sums) and Q
-// (statistics, merge, copies), captured or launched directly: every
+// (statistics, merge), captured or launched directly: every
 // instance's tail hangs off its path sums on Q; an instance's path sums wait
 // for the tail of the previous instance on the same handle. Runs of
 // consecutive instances of one 16-step shape share one launch of the fused
@@ -1628,9 +1628,8 @@ sc_status enqueue_plain(sc_batch* b, hipStream_t M, hipStream_t Q, NewEvent&& ne
   hipEvent_t tail_done = nullptr;
   // last_tail[h]: the tail event of the previous instance on handle h.
   std::vector<hipEvent_t> last_tail(b->shapes.size(), nullptr);
-  // The tails of run [i, i + n), after its path sums; a set run's statistics
-  // (one launch per pass), window merges and candidate offsets in one launch
-  // each for all its channels.
+  // The tails of run [i, i + n), after its path sums; for a set run one launch
+  // per statistics pass and one for the window merges of all its channels.
   auto enqueue_tails = [&](size_t i, size_t n, hipEvent_t sums) {
     e = hipStreamWaitEvent(Q, sums, 0);
     if (e == hipSuccess && n > 1) {

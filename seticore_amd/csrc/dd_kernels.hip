@@ -1229,7 +1229,8 @@ constexpr int kStatsBlocks = 256;
 // 276 us a call with 256, 272 with 64, 267 with 32, 272 with 16. Above 2^20
 // channels the reading counts for more, so each workgroup keeps to 32768 of
 // them: a 16 x 2^22 search in BF16 over 4 drift blocks takes 363 us (32
-// workgroups: 490), 16 x 2^24 1050 us (1818).
+// workgroups: 490), 16 x 2^24 1050 us (1818). Where nothing runs beside them
+// (the allocation-free and the single gated search) more would be quicker.
 constexpr int kCountBlocks = 32;
 int count_blocks(int N) {
   return (int)std::min<long>(kStatsBlocks, std::max<long>(kCountBlocks, ((long)N + 32767) / 32768));

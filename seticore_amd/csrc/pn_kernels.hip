@@ -138,7 +138,7 @@ __global__ void __launch_bounds__(256)
 //
 // A workgroup takes kTile3 = 16 columns of h3 of one block: 35 columns of h2
 // and 80 of h1 (73 needed, in whole groups of 16 so that a group lies in one
-// row), halo included, 72 KB of LDS, two workgroups (16 waves) per CU. Columns
+// row), halo included, 63.5 KB of LDS, two workgroups (16 waves) per CU. Columns
 // outside the maps and the row above them are zero in LDS, so the products
 // need no bounds tests. A stride-2 convolution reads every second column, so
 // columns are stored split by parity, and each group of four channels (a
